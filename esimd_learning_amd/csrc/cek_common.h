@@ -135,6 +135,15 @@ __device__ inline void decode16(u4 w, u4& lo, u4& hi) {
           __builtin_bit_cast(uint32_t, p[6]), __builtin_bit_cast(uint32_t, p[7])};
 }
 
+// Decode 8 fp8 bytes (lo, then hi) into one MFMA operand of 8 values.
+template <typename T, int FMT>
+__device__ inline u4 decode8(uint32_t lo, uint32_t hi) {
+  return u4{__builtin_bit_cast(uint32_t, fp8x2_to_pair<T, FMT, false>(lo)),
+            __builtin_bit_cast(uint32_t, fp8x2_to_pair<T, FMT, true>(lo)),
+            __builtin_bit_cast(uint32_t, fp8x2_to_pair<T, FMT, false>(hi)),
+            __builtin_bit_cast(uint32_t, fp8x2_to_pair<T, FMT, true>(hi))};
+}
+
 // Exact decode of one fp8 byte to fp32 (used by the generic paths).
 template <int FMT>
 __device__ inline float fp8_to_f32(uint32_t byte) {

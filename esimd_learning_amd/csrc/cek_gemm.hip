@@ -19,7 +19,7 @@
 #include <atomic>
 #include <mutex>
 
-#include "cek_common.h"
+#include "cek_segs.h"
 
 namespace cek {
 
@@ -29,8 +29,6 @@ int launch_gemv_generic(const void* x, const void* w, const void* scale, int ski
                         int64_t M, int64_t N, int64_t K, int io_dtype, int fp8_fmt, hipStream_t st);
 int launch_gemv_a8w8(const uint8_t* x, const float* xs, const uint8_t* w, const float* ws, void* y,
                      int64_t M, int64_t N, int64_t K, int out_dtype, hipStream_t st);
-int launch_gemv_wide(const void* x, const void* w, const void* scale, int skind, void* y,
-                     int64_t M, int64_t N, int64_t K, int io_dtype, int fp8_fmt, hipStream_t st);
 
 // ---------------------------------------------------------------------------
 // a8w8, direct-from-global v0: workgroup = 4 waves = 64 x 64 C tile, each wave
@@ -1277,11 +1275,12 @@ namespace cek {
 // and the row layout of gemm_a8w8_lds_kernel's launches
 constexpr int kW8a16Loaders = 4;
 constexpr int kA8w8LdsLayout = 1;
+constexpr int64_t kStreamM = 64;
 
 // w8a16 product for any M with a weight scale of kind skind (ScaleKind):
 // M <= 16 the GEMV kernels, N <= 16 the activation-streaming kernel,
-// 16 < M <= 32 the LDS-staged GEMV where it has an instantiation, else the
-// tiled MFMA GEMM (or the generic kernels for unaligned shapes).
+// 16 < M <= 64 the weight-streaming kernel (cek_stream.hip), else the tiled
+// MFMA GEMM (or the generic kernels for unaligned shapes).
 // Tiled w8a16 configurations of the round model (M, N >= 128, matrices
 // below 4 GB): the 8-wave register-pipelined kernel (2 x 4 waves, four
 // loader waves) with its ring slots, and t0 / step of the round model (us
@@ -1366,8 +1365,19 @@ int launch_w8a16(const void* x, const void* w, const void* scale, int skind, voi
 #undef CEK_TINYN
     return check_launch();
   }
-  if (M <= 32 && aligned(x, 16) && aligned(w, 16)) {
-    const int rc = launch_gemv_wide(x, w, scale, skind, y, M, N, K, io_dtype, fp8_fmt, st);
+  // M <= 64: the weight-streaming kernel, but for very wide matrices of short
+  // K, whose many workgroups each read the activations again (M = 64, K =
+  // 1024, N = 49152: tiles 20.6 us, streaming 23.1; K = 2048 34.3 / 35.2).  M =
+  // 48, K = 4096, N = 6144 47.7 -> 12.5 us; M = 64, K = 14336, N = 4096 157 -> 34;
+  // M = 32, K = 4096, N = 14336 (staged GEMV before) 36.7 -> 15.2.
+  if (M <= kStreamM && (N <= 32768 || K >= 4096) && aligned(x, 16) && aligned(w, 16) && N * K <= ((int64_t)1 << 40)) {
+    GemvSegs sg{};
+    sg.count = 1;
+    sg.w[0] = static_cast<const uint8_t*>(w);
+    sg.s[0] = scale;
+    sg.y[0] = static_cast<uint16_t*>(y);
+    sg.n[0] = (int)N;
+    const int rc = launch_stream(x, sg, skind, M, K, io_dtype, fp8_fmt, st);
     if (rc != CEK_ERR_UNSUPPORTED) return rc;
   }
   if (K % 64 != 0 || !aligned(x, 16) || !aligned(w, 16) || M > 65535 * 64)

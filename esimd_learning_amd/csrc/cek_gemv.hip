@@ -1,5 +1,4 @@
-// cek_gemv.hip -- fp8-weight GEMV for decode (M <= 16 activation rows; up
-// to 64 for the skinny GEMMs that reuse these kernels), gfx950.
+// cek_gemv.hip -- fp8-weight GEMV for decode (M <= 16 activation rows), gfx950.
 //
 // y[m, n] = Out((sum_k x[m, k] * dq(W[n, k])) * scale[n])   (scale after the
 // reduction, as reference fp8_GEMV_v2.h:77 / :355 apply it).
@@ -23,19 +22,16 @@
 //    pairs and accumulated with v_dot2_f32_{f16,bf16} (fp32 accumulation).
 //    The activation slice a thread needs is re-read from L1/L2 (x is tiny).
 //    DPP wave sums and an LDS combine end a row.
-//  * gemv_lds_kernel (3 <= M <= 64, K in {2, 3, 4, 5, 14, 24} x 1024): MFMA
+//  * gemv_lds_kernel (3 <= M <= 16, K in {2, 3, 4, 5, 14, 24} x 1024): MFMA
 //    on weights staged through LDS so that every load instruction still
 //    reads 1 KB of one row (see the comment at the kernel).  Also the a8w8
-//    path (e4m3 activations) for 3 <= M <= 64.
-//  * gemv_mfma_kernel (4 < M <= 16, other K % 64 == 0): the 16 x 16 x 32
-//    f16/bf16 MFMA does the M x 16-row dot products; lane l streams row
-//    (l & 15) of a 16-row tile at k-offset 16 * (l >> 4) of each 64-byte
-//    step.  The four waves of a workgroup interleave over the K steps of the
-//    same tile and reduce through LDS.
-//  * gemv_xres_kernel (9 <= M <= 16, 512 < N / 16 <= 2048, K <= 4096) and
-//    gemv_xres8_kernel (e4m3 activations, 17 <= M <= 32): the activations
-//    stay in LDS for the whole launch and the weights stream straight into
-//    MFMA operand registers (see the comments at the kernels).
+//    path (e4m3 activations).
+//  * the weight-streaming kernel of cek_stream.hip: 3 <= M <= 16 at other K,
+//    and where it is faster at these (stream_matrix); the a8w8 GEMV of up to
+//    64 rows.
+//  * gemv_xres8_kernel (e4m3 activations, 17 <= M <= 32, N > 16384): the
+//    activations stay in LDS for the whole launch and the weights stream
+//    straight into MFMA operand registers (see the comment at the kernel).
 //  * gemv_generic_kernel: any K / alignment; byte loads.  Correctness path
 //    for shapes the vector kernels do not take.
 //
@@ -48,26 +44,12 @@
 #include <type_traits>
 
 #include "cek_rowops.h"
+#include "cek_segs.h"
 
 namespace cek {
 
-constexpr int kCUs = 256;  // MI355X compute units, for the launch-balance rules
-
 int launch_w8a16(const void* x, const void* w, const void* scale, int skind, void* y, int64_t M, int64_t N, int64_t K,
                  int io_dtype, int fp8_fmt, float* ws, int64_t ws_bytes, hipStream_t st);  // cek_gemm.hip
-
-constexpr int MAX_SEGS = 8;
-
-// Weight matrices sharing one x; gstart[i] = first workgroup of segment i.
-struct GemvSegs {
-  const uint8_t* w[MAX_SEGS];
-  const void* s[MAX_SEGS];
-  uint16_t* y[MAX_SEGS];
-  int n[MAX_SEGS];
-  int gstart[MAX_SEGS + 1];
-  int count;
-  const float* xs;  // per-row activation scales [M] when x holds e4m3 codes
-};
 
 // Inputs and side outputs of the add+RMSNorm (+ e4m3 quant) that
 // gemv_lds_kernel's NORM form computes in its prologue (unused otherwise).
@@ -120,21 +102,6 @@ struct NormArgs {
 // (nss <= 256 and a multiple of 4, M <= 4), inv = rsqrt(sum / K + eps), and
 // scales its outputs by inv[m].
 enum EpiKind { EPI_NONE = 0, EPI_ADDNORM = 1, EPI_ROWSCALE = 2, EPI_ADDNORM12 = 3 };
-
-struct SegRef {
-  const uint8_t* w;
-  const void* s;
-  uint16_t* y;
-  int n, group;
-};
-
-__device__ inline SegRef find_seg(const GemvSegs& sg, int b) {
-  int i = 0;
-#pragma unroll
-  for (int j = 1; j < MAX_SEGS; ++j)
-    if (j < sg.count && b >= sg.gstart[j]) i = j;
-  return SegRef{sg.w[i], sg.s[i], sg.y[i], sg.n[i], b - sg.gstart[i]};
-}
 
 // ---------------------------------------------------------------------------
 // M <= MT (MT in {1, 2, 4}): v_dot2 path.  A 256-thread workgroup owns R
@@ -276,102 +243,7 @@ __global__ __launch_bounds__(256) void gemv_dot_kernel(const uint16_t* __restric
 }
 
 // ---------------------------------------------------------------------------
-// 4 < M <= 16: MFMA 16x16x32 path.  Workgroup = 4 waves = one 16*NT-row
-// tile of one segment; wave w takes the 64-byte K steps s with s % 4 == w.
-// ---------------------------------------------------------------------------
-template <typename T, typename TO, int FMT, bool XF8, int NT, int UNROLL>
-__global__ __launch_bounds__(256) void gemv_mfma_kernel(const uint16_t* __restrict__ x, GemvSegs sg, int skind,
-                                                        int M, int K) {
-  typedef typename T::pair P;
-  __shared__ f4 red[3][NT][64];
-  const SegRef sr = find_seg(sg, blockIdx.x);
-  const int N = sr.n;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int n0 = sr.group * 16 * NT;
-  const int r16 = lane & 15;
-  const int g = lane >> 4;
-  const int steps = K >> 6;  // 64-byte K steps (K % 64 == 0 on this path)
-
-  const uint8_t* wrow[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    int row = n0 + t * 16 + r16;
-    row = row < N ? row : N - 1;  // clamped rows are never stored
-    wrow[t] = sr.w + (size_t)row * K + g * 16;
-  }
-  const bool xrow_ok = r16 < M;
-  const uint16_t* xrow = x + (size_t)(xrow_ok ? r16 : 0) * K + g * 16;
-  const uint8_t* xrow8 = reinterpret_cast<const uint8_t*>(x) + (size_t)(xrow_ok ? r16 : 0) * K + g * 16;
-  // wave 0's output scales, loaded up front (their latency then overlaps the
-  // weight loads')
-  uint32_t sc_n[NT];
-  float sc_m[4];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) sc_n[t] = wave == 0 ? load_scale_bits(sr.s, skind, min(n0 + t * 16 + r16, N - 1)) : 0u;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) sc_m[v] = (XF8 && wave == 0) ? sg.xs[min(g * 4 + v, M - 1)] : 1.f;
-
-  f4 acc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-
-  for (int s0 = wave; s0 < steps; s0 += 4 * UNROLL) {
-    u4 wv[UNROLL][NT];
-    u4 xa[UNROLL], xb[UNROLL];
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      const int s = s0 + 4 * u;
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        wv[u][t] = s < steps ? load_u4_stream(wrow[t] + (size_t)s * 64) : u4{0, 0, 0, 0};
-      if (s < steps && xrow_ok && XF8) {
-        decode16<T, CEK_E4M3>(load_u4(xrow8 + (size_t)s * 64), xa[u], xb[u]);
-      } else if (s < steps && xrow_ok) {
-        const u4* xp = reinterpret_cast<const u4*>(xrow + (size_t)s * 64);
-        xa[u] = xp[0];
-        xb[u] = xp[1];
-      } else {
-        xa[u] = u4{0, 0, 0, 0};
-        xb[u] = u4{0, 0, 0, 0};
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);  // all loads of the round before any arithmetic
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        u4 lo, hi;  // decoded weights for k-slots [0,8) and [8,16) of this lane
-        decode16<T, FMT>(wv[u][t], lo, hi);
-        // A = activations (row r16 = m), B = weights (column r16 = n).
-        acc[t] = mfma16x16x32<T>(xa[u], lo, acc[t]);
-        acc[t] = mfma16x16x32<T>(xb[u], hi, acc[t]);
-      }
-    }
-  }
-
-  if (wave > 0) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t) red[wave - 1][t][lane] = acc[t];
-  }
-  __syncthreads();
-  if (wave != 0) return;
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    f4 c = acc[t] + red[0][t][lane] + red[1][t][lane] + red[2][t][lane];
-    const int n = n0 + t * 16 + r16;  // D column = lane & 15
-    if (n >= N) continue;
-    const float sc = scale_value(sc_n[t], skind);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int m = g * 4 + v;  // D row = 4 * (lane >> 4) + v
-      if (m < M) sr.y[(size_t)m * N + n] = TO::from_f32(c[v] * (XF8 ? sc * sc_m[v] : sc));
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// 4 < M <= 64, K % 1024 == 0: LDS-staged MFMA path.
+// 3 <= M <= 16, K % 1024 == 0: LDS-staged MFMA path.
 //
 // HBM streams best when every load instruction of a wave reads 1 KB of ONE
 // row (measured on MI355X: 6.4 TB/s, against 4.0-5.3 TB/s when an instruction
@@ -507,12 +379,6 @@ __device__ inline void lds_reduce_addnorm(const f4& acc, uint8_t* smem, int wave
   for (int v = 0; v < 4; ++v)
     if (n16 == 0 && g * 4 + v < M) na.ss_out[(size_t)(g * 4 + v) * (N / ROWS) + n0 / ROWS] = s2[v];
 }
-
-// LDS writes of this wave done, then a workgroup barrier -- without the
-// vmcnt(0) a fenced __syncthreads adds, which would drain the loads of the
-// stages in flight.  The "memory" clobber keeps LDS accesses (and the
-// activation loads, which are therefore not __restrict__) on their side.
-__device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // The cross-wave sum of one tile of a multi-tile workgroup, in a reduction
 // area of its own (red, 3 x NT x MB x 64 f4), with LDS-only barriers so that
@@ -1187,191 +1053,49 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs 
 }
 
 // ---------------------------------------------------------------------------
-// 9 <= M <= 16 with wide N: the activations resident in LDS.
-//
-// gemv_lds_kernel reads, for every 16-row tile, the 16 activation rows of
-// each K stage from L2 straight into MFMA operand layout: lane l takes row
-// l & 15, so every such load touches 16 cache lines, and at M = 16 the
-// texture-address unit stalls on them (its waves wait on outstanding loads
-// most of their cycles).  Here a workgroup loads the whole activation matrix
-// (16 rows x K values, rows >= M repeating row M - 1: 64-128 KB) into LDS
-// once, by direct-to-LDS loads, and streams its weight rows from global
-// memory straight into operand registers (no weight staging, no barrier per
-// stage).  A workgroup runs TPB tiles of 16 weight rows at a time, each tile
-// split over two waves: the wave of half h takes K values [h K / 2,
-// (h + 1) K / 2) of the tile's rows, as 64-byte chunks (lane group g = lane
-// >> 4 takes bytes 16 g .. 16 g + 15 of a chunk, two 8-value MFMA operands),
-// PD chunks in flight; the second half's sum is then added to the first's
-// through LDS, scaled and rounded as in gemv_lds_kernel.  The sum order
-// differs from gemv_lds_kernel's, so the outputs may differ from it in the
-// last bit: the dispatcher picks the kernel per weight matrix (by its own
-// row count), so a multi-matrix launch still gives each matrix what it gets
-// alone.  Slots of TPB tiles run grid-stride over the tiles of all segments.
-//
-// LDS: activation chunk lc (16 bytes) of row r sits at (lc & ~15) | ((lc ^ r)
-// & 15): the 16 rows that one 16-lane group of a ds_read_b128 reads at the
-// same K land in 16 different 16-byte bank groups.  The direct-to-LDS loads
-// fill LDS in order, so lane i of load j fetches the logical chunk that
-// belongs at physical chunk 64 j + i (the map is its own inverse).
-//
-// Measured on MI355X against gemv_lds_kernel (weights from HBM, M = 16 unless
-// given): K = 4096, N = 14336 17.37 -> 15.25 us, N = 28672 29.99 -> 26.49,
-// M = 12, N = 14336 16.44 -> 15.01, M = 9, N = 28672 27.15 -> 26.31;
-// K = 3072, N = 12288 12.65 -> 12.29.  Not faster at 512 tiles or fewer
-// (N = 6144: 10.34 us against 9.99 for gemv_lds_kernel; N = 8192 equal) nor
-// above 2048 (N = 49152: 44.7 against 44.2).  Splitting each tile's K by residues mod 4 over the
-// waves instead (which sums in gemv_lds_kernel's order, bit for bit) was
-// 0-8% slower than this form where it gained, and 8% slower than
-// gemv_lds_kernel at M = 9, N = 28672.
-template <typename T, typename TO, int FMT, int K, int TPB, int PD>
-__global__ __launch_bounds__(128 * TPB) void gemv_xres_kernel(const uint16_t* __restrict__ x, GemvSegs sg, int skind,
-                                                             int M, int tiles) {
-  constexpr int NCW = K / 128;  // 64-byte chunks per wave and tile (half of the K values)
-  constexpr int XBYTES = 16 * K * 2, CPR = K / 8;
-  static_assert(NCW % PD == 0, "whole prefetch groups");
-  static_assert(XBYTES % 1024 == 0, "1 KB direct-to-LDS loads");
-  __shared__ __attribute__((aligned(1024))) uint8_t sx[XBYTES];
-  __shared__ f4 red[TPB * 64];  // the second halves' sums
-  static_assert(sizeof(sx) + sizeof(red) <= 160 * 1024, "LDS");
-  // wave-uniform indices (so that the segment table is read by scalar loads,
-  // which do not count against the weight loads' vmcnt)
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int tw = wave >> 1, kh = wave & 1;
-  const int r16 = lane & 15, g = lane >> 4;
-  const int nslot = (tiles + TPB - 1) / TPB;
-  // this wave's tile of slot s (clamped: a wave past the last tile repeats
-  // it and stores nothing) and the first weight byte it reads: its row
-  // (clamped into its matrix; rows past it are never stored), K half, lane group
-  auto wsrc = [&](int s) {
-    const SegRef r = find_seg(sg, min(s * TPB + tw, tiles - 1));
-    return r.w + (size_t)min(16 * r.group + r16, r.n - 1) * K + (K / 2) * kh + 16 * g;
-  };
-  // half 0: the weight scale of this lane's output column of slot s's tile
-  auto scale_bits = [&](int s) {
-    const SegRef r = find_seg(sg, min(s * TPB + tw, tiles - 1));
-    return kh == 0 ? load_scale_bits(r.s, skind, min(16 * r.group + r16, r.n - 1)) : 0u;
-  };
-  int s = blockIdx.x;
-  uint32_t scb = s < nslot ? scale_bits(s) : 0u;
-  {
-    const __amdgpu_buffer_rsrc_t rx =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, M * K * 2, 0x00020000);
-    for (int j = wave; j < XBYTES / 1024; j += 2 * TPB) {
-      const int pc = 64 * j + lane, r = pc / CPR, p = pc % CPR;
-      const int lc = (p & ~15) | ((p ^ r) & 15);
-#if defined(__HIP_DEVICE_COMPILE__)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr_t)(sx + 1024 * j), 16,
-                                               (uint32_t)((min(r, M - 1) * K + 8 * lc) * 2), 0, 0, 0);
-#endif
-    }
-  }
-  u4 wb[PD];
-  const uint8_t* wr = wsrc(s);
-  if (s < nslot) {
-#pragma unroll
-    for (int i = 0; i < PD; ++i) wb[i] = load_u4(wr + 64 * i);
-    wait_vmcnt<PD>();  // this wave's activation loads (older) are in LDS
-  } else {
-    wait_vmcnt<0>();
-  }
-  bare_barrier();
-  const uint8_t* xr = sx + r16 * (K * 2);
-  const int c0 = NCW * kh;  // this wave's first chunk
-  for (; s < nslot; s += gridDim.x) {
-    const int sn = s + gridDim.x;
-    const uint8_t* wn = wsrc(sn);
-    f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int j0 = 0; j0 < NCW; j0 += PD) {
-      // the next PD chunks of this tile, or the first of the next slot's
-      // (after the last slot: the PD chunks just read again, still in the
-      // caches and never used -- the loads stay unconditional, so every wait
-      // count is static)
-      const uint8_t* src = j0 + PD < NCW ? wr + 64 * (j0 + PD) : (sn < nslot ? wn : wr + 64 * (NCW - PD));
-#pragma unroll
-      for (int i = 0; i < PD; ++i) {
-        const u4 w = wb[i];
-        wb[i] = load_u4(src + 64 * i);
-        u4 lo, hi;
-        decode16<T, FMT>(w, lo, hi);
-        const int lc = 8 * (c0 + j0 + i) + 2 * g;  // chunk c: 16-byte activation pieces 8 c + 2 g, + 1
-        const u4 x0 = *reinterpret_cast<const u4*>(xr + 16 * ((lc & ~15) | ((lc ^ r16) & 15)));
-        const u4 x1 = *reinterpret_cast<const u4*>(xr + 16 * (((lc + 1) & ~15) | (((lc + 1) ^ r16) & 15)));
-        acc = mfma16x16x32<T>(x0, lo, acc);
-        acc = mfma16x16x32<T>(x1, hi, acc);
-      }
-    }
-    if (kh == 1) red[tw * 64 + lane] = acc;
-    lds_barrier();
-    const int tile = s * TPB + tw;
-    if (kh == 0 && tile < tiles) {
-      const SegRef r = find_seg(sg, tile);
-      const f4 c = acc + red[tw * 64 + lane];
-      const int n = 16 * r.group + r16;
-      const float sc = scale_value(scb, skind);
-      if (n < r.n) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int m = 4 * g + v;
-          if (m < M) r.y[(size_t)m * r.n + n] = TO::from_f32(f32_round(c[v] * sc));
-        }
-      }
-    }
-    if (sn < nslot) scb = scale_bits(sn);
-    lds_barrier();  // half 0 has read red before the next slot writes it
-    wr = wn;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// The same for e4m3 activations (the a8w8 GEMV, per-row activation scales
-// sg.xs, fp32 per-channel weight scales), 17 <= M <= 32: the activation codes
-// of MB = 2 blocks of 16 rows (rows >= M repeating row M - 1; 32 K bytes: up
-// to 128 KB) resident in LDS, the weights straight into the operands of
-// v_mfma_f32_16x16x128_f8f6f4.  A lane's operand for the 128-byte K chunk c
-// is bytes 128 c + 16 g .. + 15 and 128 c + 64 + 16 g .. + 15 of its row (two
-// 16-byte loads, each of 16 rows x 64 contiguous bytes), the activation
-// operand the same bytes of its activation row.  Each tile's K is split in
-// KS contiguous parts over KS waves, added in order through LDS; outputs
-// Out(sum * (sb[n] * sa[m])) as in gemv_lds_kernel.  Measured on MI355X
-// against gemv_lds_kernel (weights from HBM, K = 4096, M = 32 unless given):
-// N = 6144 (32 tokens into a 4096-wide QKV) 12.53 -> 10.32 us, N = 14336
-// 23.71 -> 16.1, N = 28672 33.97 -> 27.28, M = 24, N = 6144 11.09 -> 10.21,
-// M = 17, N = 14336 18.3 -> 15.83; at 256 tiles (N = 4096) no faster
-// (8.69-9.74 us against 8.68 for gemv_lds_kernel).  Of 1 x 4, 2 x 2, 2 x 4 and 4 x 2 (tiles per slot x K parts),
-// 2 x 4 was the fastest or within 1% of it wherever the kernel gained.
-// ONE (the launch runs one slot per workgroup): the later K parts' sums go
-// through the activation area, once every wave is done reading it, so that
-// 32 rows of K = 5120 (160 KB, all of LDS) fit.
-// RT = 12: tiles of 12 weight rows (the segment table counts 12-row groups);
-// operand lanes 12-15 load row 11 again (the same cache lines as lane 11's,
-// in the same instruction) and are not stored.  A tile's K parts and their
-// order do not depend on RT, so neither do the outputs.
-template <typename TO, int K, int TPB, int KS, int PD, bool ONE = false, int RT = 16>
+// a8w8 GEMV (e4m3 activations, per-row activation scales sg.xs, fp32
+// per-channel weight scales) of 17 <= M <= 32 rows with more than 16384
+// weight rows of K = 2, 3 or 4 KiB: the activation codes of MB = 2 blocks of
+// 16 rows (rows >= M repeating row M - 1; 32 K bytes: up to 128 KB) stay in
+// LDS for the whole launch, loaded once by direct-to-LDS loads, and the
+// weights go straight into the operands of v_mfma_f32_16x16x128_f8f6f4.  A
+// lane's operand for the 128-byte K chunk c is bytes 128 c + 16 g .. + 15 and
+// 128 c + 64 + 16 g .. + 15 of its row (two 16-byte loads, each of 16 rows x 64
+// contiguous bytes; g = lane >> 4), the activation operand the same bytes of
+// its activation row.  A workgroup runs slots of TPB tiles of 16 weight rows,
+// grid-stride, each tile's K split in KS contiguous parts over KS waves,
+// added in order through LDS; outputs Out(sum * (sb[n] * sa[m])) as in
+// gemv_lds_kernel.  LDS: activation chunk lc (16 bytes) of row r sits at
+// (lc & ~15) | ((lc ^ r) & 15): the 16 rows that a 16-lane group of a
+// ds_read_b128 reads at the same K land in 16 different bank groups.
+// Where the activations are loaded once for many weight rows this beats the
+// weight-streaming kernel, which reads them again for every workgroup
+// (MI355X, weights from HBM, M = 32, us, this kernel / streaming: K = 2048, N =
+// 24576 14.2 / 15.7, N = 49152 23.6 / 26.5; K = 3072, N = 49152 33.5 / 36.0;
+// K = 4096, N = 28672 28.5 / 28.6; at N = 16384 11.0 / 9.7 and 15.1 / 13.0).
+template <typename TO, int K, int TPB, int KS, int PD>
 __global__ __launch_bounds__(64 * TPB * KS) void gemv_xres8_kernel(const uint8_t* __restrict__ x, GemvSegs sg, int M,
                                                                   int tiles) {
-  static_assert(RT == 16 || RT == 12, "tile rows");
   constexpr int MB = 2;
   constexpr int NCW = K / 128 / KS;  // 128-byte K chunks per wave and tile
   constexpr int XBYTES = 16 * MB * K, CPR = K / 16;
   constexpr int REDB = TPB * (KS - 1) * MB * 64 * 16;  // bytes of the later parts' sums
   static_assert(NCW % PD == 0, "whole prefetch groups");
   static_assert(XBYTES % 1024 == 0, "1 KB direct-to-LDS loads");
-  static_assert(!ONE || REDB <= XBYTES, "the sums fit the activation area");
-  __shared__ __attribute__((aligned(1024))) uint8_t sx[XBYTES + (ONE ? 0 : REDB)];
+  __shared__ __attribute__((aligned(1024))) uint8_t sx[XBYTES + REDB];
   static_assert(sizeof(sx) <= 160 * 1024, "LDS");
-  f4* red = reinterpret_cast<f4*>(ONE ? sx : sx + XBYTES);
+  f4* red = reinterpret_cast<f4*>(sx + XBYTES);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int tw = wave / KS, kh = wave % KS;
   const int r16 = lane & 15, g = lane >> 4;
   const int nslot = (tiles + TPB - 1) / TPB;
   auto wsrc = [&](int s) {
     const SegRef r = find_seg(sg, min(s * TPB + tw, tiles - 1));
-    return r.w + (size_t)min(RT * r.group + min(r16, RT - 1), r.n - 1) * K + (K / KS) * kh + 16 * g;
+    return r.w + (size_t)min(16 * r.group + r16, r.n - 1) * K + (K / KS) * kh + 16 * g;
   };
   auto scale_bits = [&](int s) {
     const SegRef r = find_seg(sg, min(s * TPB + tw, tiles - 1));
-    return kh == 0 ? load_scale_bits(r.s, SK_F32, min(RT * r.group + min(r16, RT - 1), r.n - 1)) : 0u;
+    return kh == 0 ? load_scale_bits(r.s, SK_F32, min(16 * r.group + r16, r.n - 1)) : 0u;
   };
   float scm[MB][4];  // the activation rows' scales (D row 16 b + 4 g + v)
 #pragma unroll
@@ -1433,7 +1157,6 @@ __global__ __launch_bounds__(64 * TPB * KS) void gemv_xres8_kernel(const uint8_t
         }
       }
     }
-    if constexpr (ONE) lds_barrier();  // every wave is done reading the activations
     if (kh > 0) {
 #pragma unroll
       for (int b = 0; b < MB; ++b) red[((tw * (KS - 1) + kh - 1) * MB + b) * 64 + lane] = acc[b];
@@ -1442,9 +1165,9 @@ __global__ __launch_bounds__(64 * TPB * KS) void gemv_xres8_kernel(const uint8_t
     const int tile = s * TPB + tw;
     if (kh == 0 && tile < tiles) {
       const SegRef r = find_seg(sg, tile);
-      const int n = RT * r.group + r16;
+      const int n = 16 * r.group + r16;
       const float sc = scale_value(scb, SK_F32);
-      if (n < r.n && r16 < RT) {
+      if (n < r.n) {
 #pragma unroll
         for (int b = 0; b < MB; ++b) {
           f4 c = acc[b];
@@ -1490,17 +1213,6 @@ __global__ __launch_bounds__(256) void gemv_generic_kernel(const uint16_t* __res
 // ---------------------------------------------------------------------------
 // Host dispatch
 // ---------------------------------------------------------------------------
-// Fill gstart for `rows_per_wg` output rows per workgroup; returns the grid.
-static int seg_grid(GemvSegs& sg, int rows_per_wg) {
-  int g = 0;
-  for (int i = 0; i < sg.count; ++i) {
-    sg.gstart[i] = g;
-    g += (sg.n[i] + rows_per_wg - 1) / rows_per_wg;
-  }
-  for (int i = sg.count; i <= MAX_SEGS; ++i) sg.gstart[i] = g;
-  return g;
-}
-
 // LDS-staged path: configuration per (rows M, total weight rows N, K stages),
 // from sweeps on MI355X over the decode shapes.  Returns false when no
 // instantiation covers the shape (K not one of 2, 3, 4, 5, 14 or 24 KiB
@@ -1656,23 +1368,18 @@ static bool launch_lds_steps(const void* x, GemvSegs& sg, int skind, int M, int 
     }
     return true;
   }
-  if (M <= 32 && N <= 16384) {  // wider N is served as well by the tiled GEMM
-    if constexpr (XF8) CEK_LDS(1, 2, 2);
-    else CEK_LDS(1, 2, 1);
-    return true;
-  }
-  if constexpr (XF8) {
-    if (M <= 64 && N <= 8192) {
-      CEK_LDS(1, 4, 1);
-      return true;
-    }
-  }
   return false;
 #undef CEK_LDS
 #undef CEK_LDS_T
 #undef CEK_LDS_T12
 #undef CEK_LDS_24
 #undef CEK_LDS_TPW
+}
+
+// K with an instantiation of gemv_lds_kernel
+static bool lds_k(int64_t K) {
+  const int64_t s = K >> 10;
+  return K % 1024 == 0 && ((s >= 2 && s <= 5) || s == 14 || s == 24);
 }
 
 template <typename T, typename TO, int FMT, bool XF8>
@@ -1687,47 +1394,6 @@ static bool launch_lds(const void* x, GemvSegs& sg, int skind, int M, int K, int
     case 24: return launch_lds_steps<T, TO, FMT, XF8, 24>(x, sg, skind, M, N, st);
     default: return false;
   }
-}
-
-// gemv_xres_kernel takes a weight matrix of 512 < tiles <= 2048 16-row tiles
-// (8208 <= N <= 32768) when 9 <= M <= 16, the activations are fp16 / bf16 and
-// K is 2, 3 or 4 KiB values (the range where it measured faster).
-static bool xres_matrix(int M, int K, int n) {
-  const int tiles = (n + 15) / 16;
-  return M >= 9 && M <= 16 && (K == 2048 || K == 3072 || K == 4096) && tiles > 512 && tiles <= 2048;
-}
-
-// gemv_xres_kernel over every segment of sg (all of them xres_matrix): one
-// slot per workgroup (one workgroup per CU) as far as the CUs go, TPB =
-// ceil(tiles / CUs) tiles per slot (3 to 8), so that the slots spread evenly
-// over the CUs (each tile's sum does not depend on TPB).  Measured on MI355X
-// at M = 16 against 4 tiles per slot up to 1024 tiles and 8 above (weights
-// from HBM): K = 4096, N = 9000 13.74 -> 12.36 us, N = 16400 23.24 -> 18.55,
-// N = 20480 23.86 -> 20.51, N = 24576 25.09 -> 22.50, N = 28672 26.72 ->
-// 25.78; K = 3072, N = 12288 12.17 -> 11.83; N = 14336 equal.
-template <typename T, typename TO, int FMT>
-static void launch_xres(const void* x, GemvSegs& sg, int skind, int M, int K, hipStream_t st) {
-  const int tiles = seg_grid(sg, 16);  // gstart: first tile of each segment
-  int tpb = (tiles + kCUs - 1) / kCUs;
-  tpb = tpb < 3 ? 3 : (tpb > 8 ? 8 : tpb);
-  const int nslot = (tiles + tpb - 1) / tpb;
-  const dim3 grid((unsigned)(nslot < kCUs ? nslot : kCUs));
-  const uint16_t* xp = static_cast<const uint16_t*>(x);
-#define CEK_XRES(KK, TT) gemv_xres_kernel<T, TO, FMT, KK, TT, 8><<<grid, 128 * (TT), 0, st>>>(xp, sg, skind, M, tiles)
-#define CEK_XRES_K(KK)            \
-  do {                            \
-    if (tpb == 3) CEK_XRES(KK, 3);      \
-    else if (tpb == 4) CEK_XRES(KK, 4); \
-    else if (tpb == 5) CEK_XRES(KK, 5); \
-    else if (tpb == 6) CEK_XRES(KK, 6); \
-    else if (tpb == 7) CEK_XRES(KK, 7); \
-    else CEK_XRES(KK, 8);               \
-  } while (0)
-  if (K == 2048) CEK_XRES_K(2048);
-  else if (K == 3072) CEK_XRES_K(3072);
-  else CEK_XRES_K(4096);
-#undef CEK_XRES_K
-#undef CEK_XRES
 }
 
 // Gate/up GEMV with gelu_and_mul fused (gemv_lds_kernel's GLU form): one
@@ -1880,6 +1546,30 @@ int launch_norm_gemv(const NormArgs& na, const void* w, const void* scale, int s
   return check_launch();
 }
 
+// Whether a matrix of n rows goes to the weight-streaming kernel (cek_stream.hip)
+// rather than to the kernels here, by measured time (MI355X, weights from HBM,
+// us, this file's kernel -> the streaming one).
+// K that gemv_lds_kernel has no instantiation for, from three rows on: M = 4,
+// K = 10240, N = 2560 11.1 -> 8.4; M = 8, K = 2560, N = 20480 23.2 -> 12.5; M =
+// 16, K = 8192, N = 8192 33.0 -> 14.8 -- but for up to four rows of a short and
+// long-K matrix, whose few workgroups each pay the stages' barriers (N = 1000,
+// K = 6144 5.3 against 5.9; N = 2048 6.6 -> 6.2; e4m3 activations N = 2048, K =
+// 8192 6.6 against 7.0).
+// K that it has (16-bit activations): 9 .. 16 rows of a wide matrix (M = 16,
+// K = 4096, N = 8208 12.3 -> 9.6, N = 14336 15.5 -> 13.2, N = 28672 26.5 -> 25.2;
+// K = 14336, N = 16384 66.7 -> 43.4; M = 9, N = 9000 12.0 -> 9.6, but K = 3072, N =
+// 49152 28.2 against 30.2), K = 2048 above 4096 rows (M = 16, N = 6144 7.4 ->
+// 5.7; N = 4096 4.9 against 5.1) and K = 24576 from 12 rows on (M = 16, N = 3072
+// 29.4 -> 23.9).  The wide bound is above every merged gate/up width at which
+// the fused gate/up launch is held to the plain one bit for bit.
+static bool stream_matrix(bool xf8, int64_t M, int64_t K, int64_t n) {
+  if (M < 3 || M > 16 || K % 64 != 0 || K > kStreamMaxK) return false;
+  if (!lds_k(K)) return !(M <= 4 && n <= (xf8 ? 2048 : 1024) && K > 4096);
+  if (xf8 || M < 9) return false;
+  if (n >= 8192) return M >= 12 || n <= 24576 || (n <= 32768 && K <= 4096);
+  return (K == 2048 && n > 4096) || (K == 24576 && M >= 12 && n >= 2048);
+}
+
 template <typename T, typename TO, int FMT, bool XF8>
 static int launch_gemv_t(const void* x, GemvSegs sg, int skind, int M, int K, bool vec16, hipStream_t st) {
   const uint16_t* xp = static_cast<const uint16_t*>(x);
@@ -1893,33 +1583,30 @@ static int launch_gemv_t(const void* x, GemvSegs sg, int skind, int M, int K, bo
   // each matrix alone would (the LDS forms it may pick between agree bit for
   // bit).
   const int m_lds = K >= 14336 ? 1 : 3;
-  if constexpr (!XF8) {
-    // matrices that gemv_xres_kernel serves go to one launch of it, the rest
-    // on through the kernels below (its sum order differs from theirs, so the
-    // choice is per matrix: a multi-matrix launch gives each matrix what it
-    // gets alone)
-    if (vec16) {
-      GemvSegs sx{}, so{};
-      sx.xs = so.xs = sg.xs;
-      for (int i = 0; i < sg.count; ++i) {
-        GemvSegs& d = xres_matrix(M, K, sg.n[i]) ? sx : so;
-        d.w[d.count] = sg.w[i];
-        d.s[d.count] = sg.s[i];
-        d.y[d.count] = sg.y[i];
-        d.n[d.count] = sg.n[i];
-        ++d.count;
-      }
-      if (sx.count > 0) {
-        launch_xres<T, TO, FMT>(x, sx, skind, M, K, st);
-        if (so.count == 0) return check_launch();
-        sg = so;
-        N = 0;
-        for (int i = 0; i < sg.count; ++i) N += sg.n[i];
-      }
+  // Matrices that the weight-streaming kernel serves go to it, the rest on
+  // through the kernels below (its sum order differs from theirs, so the
+  // choice is per matrix: a multi-matrix launch gives each matrix what it
+  // gets alone).
+  if (vec16) {
+    GemvSegs ss{}, so{};
+    ss.xs = so.xs = sg.xs;
+    for (int i = 0; i < sg.count; ++i) {
+      GemvSegs& d = stream_matrix(XF8, M, K, sg.n[i]) ? ss : so;
+      d.w[d.count] = sg.w[i];
+      d.s[d.count] = sg.s[i];
+      d.y[d.count] = sg.y[i];
+      d.n[d.count] = sg.n[i];
+      ++d.count;
+    }
+    if (ss.count > 0) {
+      const int rc = launch_stream(x, ss, skind, M, K, TO::code, FMT, st);
+      if (rc != CEK_OK || so.count == 0) return rc;
+      sg = so;
+      N = 0;
+      for (int i = 0; i < sg.count; ++i) N += sg.n[i];
     }
   }
   if (vec16 && M >= m_lds && launch_lds<T, TO, FMT, XF8>(x, sg, skind, M, K, N, st)) return check_launch();
-  if (M > 16) return CEK_ERR_UNSUPPORTED;
   if (vec16 && M <= 4) {
     // Rows per workgroup (measured on MI355X, one pass over > 2 GB of
     // rotating weights): 2 for M = 1 up to K = 4096, else 4, which amortises
@@ -1950,16 +1637,6 @@ static int launch_gemv_t(const void* x, GemvSegs sg, int skind, int M, int K, bo
     } else if (M == 2) CEK_DOT(2, 4, 1);
     else CEK_DOT(4, 4, 1);
 #undef CEK_DOT
-  } else if (vec16 && K % 64 == 0 && M <= 16) {
-    // 16-row tiles per wave (NT) and 64-byte K steps in flight per wave
-    // (UNROLL), measured per shape class: wide N amortises the activation
-    // reads over more tiles; narrow N needs more workgroups and deeper K.
-#define CEK_MF(NT, UN) gemv_mfma_kernel<T, TO, FMT, XF8, NT, UN><<<dim3(seg_grid(sg, 16 * NT)), 256, 0, st>>>(xp, sg, skind, M, K)
-    if (N >= 16384) CEK_MF(4, 4);
-    else if (N >= 8192) { if (M > 8) CEK_MF(4, 2); else if (K <= 3072) CEK_MF(1, 8); else CEK_MF(2, 8); }
-    else if (K <= 4096) { if (N >= 6144) CEK_MF(2, 16); else CEK_MF(1, 16); }
-    else CEK_MF(1, 4);
-#undef CEK_MF
   } else if (!XF8) {
     gemv_generic_kernel<T, FMT><<<dim3(seg_grid(sg, 4)), 256, 0, st>>>(xp, sg, skind, M, K);
   } else {
@@ -1969,12 +1646,9 @@ static int launch_gemv_t(const void* x, GemvSegs sg, int skind, int M, int K, bo
 }
 
 // Validates and launches one GEMV over count (<= MAX_SEGS) weight matrices.
-// M <= 16 for the GEMV entry points; the GEMM entry point also sends
-// 16 < M <= 32 here (max_m = 32), which only the LDS path takes
-// (CEK_ERR_UNSUPPORTED otherwise).
 int launch_gemv_segs(const void* x, int count, const void* const* w, const void* const* scale,
                      void* const* y, const int64_t* Ns, int64_t M, int64_t K, int skind, int io_dtype,
-                     int fp8_fmt, hipStream_t st, int max_m = 16) {
+                     int fp8_fmt, hipStream_t st) {
   if (count < 1 || count > MAX_SEGS || !w || !scale || !y || !Ns) return CEK_ERR_INVALID;
   if (M < 0 || K <= 0 || K > INT32_MAX) return CEK_ERR_INVALID;
   if (io_dtype != CEK_F16 && io_dtype != CEK_BF16) return CEK_ERR_INVALID;
@@ -1996,7 +1670,7 @@ int launch_gemv_segs(const void* x, int count, const void* const* w, const void*
   }
   if (total > INT32_MAX) return CEK_ERR_INVALID;
   if (M == 0 || sg.count == 0) return CEK_OK;
-  if (M > max_m) return CEK_ERR_INVALID;
+  if (M > 16) return CEK_ERR_INVALID;
   if (!x) return CEK_ERR_INVALID;
   if (io_dtype == CEK_F16 && fp8_fmt == CEK_E4M3) return launch_gemv_t<F16, F16, CEK_E4M3, false>(x, sg, skind, M, K, vec16, st);
   if (io_dtype == CEK_F16 && fp8_fmt == CEK_E5M2) return launch_gemv_t<F16, F16, CEK_E5M2, false>(x, sg, skind, M, K, vec16, st);
@@ -2018,75 +1692,33 @@ int launch_gemv_a8w8(const uint8_t* x, const float* xs, const uint8_t* w, const 
   sg.y[0] = static_cast<uint16_t*>(y);
   sg.n[0] = (int)N;
   sg.xs = xs;
-  // 17 <= M <= 32 with K of 2, 3 or 4 KiB values and at least 384 16-row
-  // tiles: gemv_xres8_kernel, 2 tiles x 4 K parts per workgroup, one slot per
-  // workgroup as far as 256 workgroups go; K = 5120 (160 KB of activations)
-  // only where one round of slots covers the tiles (384 to 512 tiles).  Where
-  // a workgroup has one slot (up to 512 tiles) only from 24 rows on: its
-  // activation load is not amortised, and below that the other kernel's
-  // repeated rows cost little (K = 5120, N = 8000: M = 17 12.04 -> 13.23 us,
-  // M = 24, N = 6144 13.37 -> 12.28, M = 32 15.12 -> 12.38).
-  const int tiles16 = (int)((N + 15) / 16);
-  const int m_min = tiles16 <= 512 ? 24 : 17;
-  // 12-row tiles (RT = 12) where they cut the busiest CU's rows by a fifth
-  // or more (N ~ 6144: 256 slots of 2 x 12 rows against 192 of 2 x 16; the
-  // outputs do not change).  Measured on MI355X, weights from HBM: M = 32,
-  // N = 6144, K = 4096 10.29 -> 9.89 us, K = 5120 12.36 -> 11.87 us; M = 24
-  // 10.17 -> 9.78 and 12.20 -> 11.69 us.
-  auto busiest_rows = [&](int rt) {
-    const int ns = ((int)((N + rt - 1) / rt) + 1) / 2;
-    return 2 * rt * ((ns + kCUs - 1) / kCUs);
-  };
-  const bool x12 = 5 * busiest_rows(12) <= 4 * busiest_rows(16);
-  // With 12-row tiles the kernel also takes N from 384 12-row tiles (4608)
-  // up: M = 32, K = 4096, N = 4608 / 5120 / 6100 12.13 / 12.25 / 12.53 ->
-  // 8.92 / 9.20 / 9.91 us against the LDS kernel; K = 5120 14.81 / 14.87 /
-  // 15.05 -> 10.56 / 10.85 / 11.80 us; M = 24, N = 5120 10.77 -> 9.21 us.
-  const int tiles12 = (int)((N + 11) / 12);
-  const bool wide = tiles16 >= 384 || (x12 && tiles12 >= 384);
-  if (M >= m_min && M <= 32 && K == 5120 && wide && (tiles16 <= 512 || (x12 && tiles12 <= 512))) {
-    // (RT = 12 only where one round of slots still covers its tiles)
-    const bool r12 = x12 && (((int)((N + 11) / 12) + 1) / 2 <= kCUs);
-    const int tiles = seg_grid(sg, r12 ? 12 : 16);
-    const int nslot = (tiles + 1) / 2;
-    const int m = (int)M;
-#define CEK_X8ONE(TY, RTT) gemv_xres8_kernel<TY, 5120, 2, 4, 5, true, RTT><<<nslot, 512, 0, st>>>(x, sg, m, tiles)
-    if (out_dtype == CEK_F16) {
-      if (r12) CEK_X8ONE(F16, 12);
-      else CEK_X8ONE(F16, 16);
-    } else {
-      if (r12) CEK_X8ONE(BF16, 12);
-      else CEK_X8ONE(BF16, 16);
-    }
-#undef CEK_X8ONE
-    return check_launch();
-  }
-  if (M >= m_min && M <= 32 && (K == 2048 || K == 3072 || K == 4096) && wide) {
-    const int tiles = seg_grid(sg, x12 ? 12 : 16);
+  // 17 <= M <= 32 of a wide matrix: 2 tiles x 4 K parts per workgroup
+  if (M > 16 && M <= 32 && N > 16384 && (K == 2048 || K == 3072 || K == 4096)) {
+    const int tiles = seg_grid(sg, 16);
     const int nslot = (tiles + 1) / 2;
     const dim3 grid((unsigned)(nslot < kCUs ? nslot : kCUs));
     const int m = (int)M;
-#define CEK_X8R(KK, PP, RTT)                                                                                         \
-  do {                                                                                                               \
-    if (out_dtype == CEK_F16) gemv_xres8_kernel<F16, KK, 2, 4, PP, false, RTT><<<grid, 512, 0, st>>>(x, sg, m, tiles); \
-    else gemv_xres8_kernel<BF16, KK, 2, 4, PP, false, RTT><<<grid, 512, 0, st>>>(x, sg, m, tiles);                     \
-  } while (0)
-#define CEK_X8(KK, PP)               \
-  do {                               \
-    if (x12) CEK_X8R(KK, PP, 12);    \
-    else CEK_X8R(KK, PP, 16);        \
+#define CEK_X8(KK, PP)                                                                                    \
+  do {                                                                                                    \
+    if (out_dtype == CEK_F16) gemv_xres8_kernel<F16, KK, 2, 4, PP><<<grid, 512, 0, st>>>(x, sg, m, tiles); \
+    else gemv_xres8_kernel<BF16, KK, 2, 4, PP><<<grid, 512, 0, st>>>(x, sg, m, tiles);                     \
   } while (0)
     if (K == 2048) CEK_X8(2048, 4);
     else if (K == 3072) CEK_X8(3072, 6);
     else CEK_X8(4096, 4);
 #undef CEK_X8
-#undef CEK_X8R
     return check_launch();
   }
-  if (M > 16) {  // only the LDS path takes these
-    const bool ok = out_dtype == CEK_F16 ? launch_lds<F16, F16, CEK_E4M3, true>(x, sg, SK_F32, (int)M, (int)K, (int)N, st)
-                                         : launch_lds<F16, BF16, CEK_E4M3, true>(x, sg, SK_F32, (int)M, (int)K, (int)N, st);
-    return ok ? check_launch() : CEK_ERR_UNSUPPORTED;
+  if (M > 16) {
+    // The weight-streaming kernel reads the activations once per workgroup
+    // of up to 64 weight rows: with several of those per CU and short K the
+    // tiled GEMM is faster (MI355X, weights from HBM, us, tiles / streaming:
+    // M = 64, K = 2048, N = 16384 16.3 / 12.4, N = 24576 17.6 / 19.6; K = 4096, N
+    // = 24576 33.9 / 31.4, N = 32768 37.0 / 37.7; M = 48, K = 2048, N = 24576 18.5
+    // / 16.5, N = 32768 19.6 / 20.2; K = 1024, N = 20480 10.9 / 11.4).
+    const bool wide = M <= 48 ? K >= 2048 && (N <= 24576 || K >= 4096) : K >= 4096 && N <= 24576;
+    if (N > 16384 && M > 32 && !wide) return CEK_ERR_UNSUPPORTED;
+    return launch_stream(x, sg, SK_F32, M, K, out_dtype, CEK_E4M3, st);
   }
   if (out_dtype == CEK_F16) return launch_gemv_t<F16, F16, CEK_E4M3, true>(x, sg, SK_F32, (int)M, (int)K, true, st);
   return launch_gemv_t<F16, BF16, CEK_E4M3, true>(x, sg, SK_F32, (int)M, (int)K, true, st);
@@ -2098,13 +1730,6 @@ int launch_gemv(const void* x, const void* w, const void* scale, int skind, void
   if (M < 0 || M > 16) return CEK_ERR_INVALID;
   if (M == 0 || N == 0) return K > 0 ? CEK_OK : CEK_ERR_INVALID;
   return launch_gemv_segs(x, 1, &w, &scale, &y, &N, M, K, skind, io_dtype, fp8_fmt, st);
-}
-
-// 16 < M <= 32 (GEMM entry point): the LDS path when it covers the shape.
-int launch_gemv_wide(const void* x, const void* w, const void* scale, int skind, void* y,
-                     int64_t M, int64_t N, int64_t K, int io_dtype, int fp8_fmt, hipStream_t st) {
-  if (M <= 16 || M > 32 || N <= 0) return CEK_ERR_UNSUPPORTED;
-  return launch_gemv_segs(x, 1, &w, &scale, &y, &N, M, K, skind, io_dtype, fp8_fmt, st, 32);
 }
 
 // Generic path for any M (used by the GEMM entry point for odd shapes).
