@@ -1142,6 +1142,194 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_w8a16_pipe_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// w8a16, 128 x 128 tile, two K teams.  In the 8-wave pipelined kernel above a
+// 128 x 128 tile is bound by LDS: its 64 x 32 wave tiles read 80 KB of
+// fragments per 64-deep K step beside the 24 KB that the loads write, about
+// 830 cycles at 128 bytes per cycle against 512 of MFMA.  Here a stage is 128
+// deep and the eight waves are two teams of 2 x 2 waves with 64 x 64 tiles:
+// team t takes K values 64 t .. 64 t + 63 of every stage, 48 KB of fragments
+// per 64 values, and half the barriers.  The teams' sums meet in LDS at the
+// end: each wave gives the other team's wave of its quadrant half of its
+// blocks, so that a wave ends with a 32 x 64 tile.
+// Stage: A as 128 rows of 256 bytes (chunk c of row r at c ^ (r & 15)), B as 128
+// rows of 128 bytes (chunk c at c ^ swzA(r)); whole cache lines of both.
+// Order of work, loader waves (0 .. 3), ring and buffer loads as in
+// gemm_w8a16_pipe_kernel; the K % 128 = 64 values left by an odd count of
+// 64-deep steps are team 0's alone.  M and N below the tile are taken (the
+// loads clamp rows).
+// ---------------------------------------------------------------------------
+template <typename T, int FMT, int RING>
+struct W8Team {
+  static constexpr int BM = 128, BN = 128, BK = 128, LW = 4, FM = 4, FN = 4;
+  static constexpr int ASZ = BM * 256, STAGE = ASZ + BN * 128;
+  static constexpr int ACH = ASZ / 1024 / LW, BCH = BN * 128 / 1024 / LW;  // 1 KB loads per loader wave and stage
+
+  __device__ static __forceinline__ void issue(uint8_t* smem, int slot, int kb, int wave, __amdgpu_buffer_rsrc_t rX,
+                                               __amdgpu_buffer_rsrc_t rW, const uint32_t (&oa)[ACH],
+                                               const uint32_t (&ob)[BCH]) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    uint8_t* sA = smem + slot * STAGE;
+    uint8_t* sB = sA + ASZ;
+#pragma unroll
+    for (int i = 0; i < ACH; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rX, (lds_ptr_t)(sA + (wave + LW * i) * 1024), 16,
+                                               oa[i] + 2u * (uint32_t)kb, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < BCH; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, (lds_ptr_t)(sB + (wave + LW * i) * 1024), 16, ob[i] + (uint32_t)kb,
+                                               0, 0, 0);
+#endif
+  }
+  __device__ static inline void read_a(const uint8_t* row, int pa0, int pa1, u4 (&a)[2]) {
+    a[0] = *reinterpret_cast<const u4*>(row + pa0 * 16);
+    a[1] = *reinterpret_cast<const u4*>(row + pa1 * 16);
+  }
+  __device__ static inline void read_b(const uint8_t* sB, int pb, u4 (&b)[FN][2]) {
+#pragma unroll
+    for (int j = 0; j < FN; ++j) decode16<T, FMT>(*reinterpret_cast<const u4*>(sB + j * 16 * 128 + pb * 16), b[j][0], b[j][1]);
+  }
+
+  // stage kt from ring slot c (the next stage's slot cn); mine: this team has
+  // K values in the stage
+  __device__ static __forceinline__ void step(int kt, int KT, int c, int cn, bool mine, uint8_t* smem, bool loader,
+                                              int wave, int oa_row, int ob_row, int pa0, int pa1, int pb,
+                                              __amdgpu_buffer_rsrc_t rX, __amdgpu_buffer_rsrc_t rW,
+                                              const uint32_t (&ga)[ACH], const uint32_t (&gb)[BCH], f4 (&acc)[FM][FN],
+                                              u4 (&a)[2][2], const u4 (&bc)[FN][2], u4 (&bn)[FN][2]) {
+    const uint8_t* sA = smem + c * STAGE + oa_row;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      if (i + 1 < FM) {
+        read_a(sA + (i + 1) * 16 * 256, pa0, pa1, a[(i + 1) & 1]);
+      } else if (kt + 1 < KT) {
+        // stage kt + 1 has landed (later stages' loads may fly); slot c is free
+        barrier_upto<RING - 2, ACH + BCH>(KT - 2 - kt);
+        if (loader && kt + RING < KT) issue(smem, c, (kt + RING) * BK, wave, rX, rW, ga, gb);
+        const uint8_t* nxt = smem + cn * STAGE;
+        read_b(nxt + ASZ + ob_row, pb, bn);
+        read_a(nxt + oa_row, pa0, pa1, a[0]);
+      }
+      if (mine) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          acc[i][j] = mfma16x16x32<T>(a[i & 1][0], bc[j][0], acc[i][j]);
+          acc[i][j] = mfma16x16x32<T>(a[i & 1][1], bc[j][1], acc[i][j]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+};
+
+template <typename T, int FMT, int SPLIT, int RING>
+__global__ __launch_bounds__(512, 1) void gemm_w8a16_team_kernel(
+    const uint16_t* __restrict__ X, const uint8_t* __restrict__ W, const void* __restrict__ scale, int skind,
+    uint16_t* __restrict__ Y, float* __restrict__ Pw, int M, int N, int K, int tiles_m, int tiles_n) {
+  using P = W8Team<T, FMT, RING>;
+  constexpr int BK = P::BK, FM = P::FM, FN = P::FN, ACH = P::ACH, BCH = P::BCH;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[RING * P::STAGE];
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int team = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+  const bool loader = wave < P::LW;
+  const int part = SPLIT > 1 ? (int)blockIdx.x % SPLIT : 0;
+  const int Kp = K / SPLIT;  // K values of this part
+  const uint32_t kpart = (uint32_t)(part * Kp);
+  int tm, tn;
+  tile_of<P::BM, P::BN, 8>(SPLIT > 1 ? blockIdx.x / SPLIT : blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * P::BM, n0 = tn * P::BN;
+  const __amdgpu_buffer_rsrc_t rX = buf_rsrc(X, (uint32_t)((size_t)M * K * 2));
+  const __amdgpu_buffer_rsrc_t rW = buf_rsrc(W, (uint32_t)((size_t)N * K));
+
+  // A load j = wave + LW i: lane l -> row 4 j + (l >> 4), position l & 15
+  // B load j = wave + LW i: lane l -> row 8 j + (l >> 3), position l & 7
+  uint32_t ga[ACH], gb[BCH];
+#pragma unroll
+  for (int i = 0; i < ACH; ++i) {
+    const int row = (wave + P::LW * i) * 4 + (lane >> 4);
+    ga[i] = (uint32_t)min(m0 + row, M - 1) * (uint32_t)K * 2u + 2u * kpart + (uint32_t)(((lane & 15) ^ (row & 15)) * 16);
+  }
+#pragma unroll
+  for (int i = 0; i < BCH; ++i) {
+    const int row = (wave + P::LW * i) * 8 + (lane >> 3);
+    gb[i] = (uint32_t)min(n0 + row, N - 1) * (uint32_t)K + kpart + (uint32_t)(((lane & 7) ^ swzA(row)) * 16);
+  }
+  const int r16 = lane & 15, g = lane >> 4;
+  const int pa0 = (8 * team + 2 * g) ^ r16, pa1 = (8 * team + 2 * g + 1) ^ r16, pb = (4 * team + g) ^ swzA(r16);
+  const int oa_row = (wm * 64 + r16) * 256, ob_row = (wn * 64 + r16) * 128;
+
+  f4 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+
+  const int KT = (Kp + BK - 1) / BK;
+  if (loader) {
+#pragma unroll
+    for (int s = 0; s < RING; ++s)
+      if (s < KT) P::issue(smem, s, s * BK, wave, rX, rW, ga, gb);
+  }
+  barrier_upto<RING - 1, ACH + BCH>(KT - 1);
+  u4 a[2][2], b0[FN][2], b1[FN][2];
+  P::read_b(smem + P::ASZ + ob_row, pb, b0);
+  P::read_a(smem + oa_row, pa0, pa1, a[0]);
+  auto nxt = [](int v) { return v + 1 == RING ? 0 : v + 1; };
+  auto mine = [&](int kt) { return kt * BK + 64 * team < Kp; };
+  int kt = 0, c = 0;
+  for (; kt + 1 < KT; kt += 2) {
+    const int c1 = nxt(c), c2 = nxt(c1);
+    P::step(kt, KT, c, c1, true, smem, loader, wave, oa_row, ob_row, pa0, pa1, pb, rX, rW, ga, gb, acc, a, b0, b1);
+    P::step(kt + 1, KT, c1, c2, mine(kt + 1), smem, loader, wave, oa_row, ob_row, pa0, pa1, pb, rX, rW, ga, gb, acc, a,
+            b1, b0);
+    c = c2;
+  }
+  if (kt < KT)
+    P::step(kt, KT, c, nxt(c), mine(kt), smem, loader, wave, oa_row, ob_row, pa0, pa1, pb, rX, rW, ga, gb, acc, a, b0,
+            b1);
+
+  // the other team's wave of this quadrant (wave ^ 4) takes the two block rows
+  // this one does not keep: team t keeps block rows 2 t and 2 t + 1
+  static_assert(8 * 8 * 1024 <= RING * P::STAGE, "the teams' sums fit the stages");
+  f4* const red = reinterpret_cast<f4*>(smem);  // [8 waves][2][FN][64]
+  f4 sum[2][FN];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      red[((wave * 2 + i) * FN + j) * 64 + lane] = team == 0 ? acc[2 + i][j] : acc[i][j];
+      sum[i][j] = team == 0 ? acc[i][j] : acc[2 + i][j];
+    }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) sum[i][j] += red[(((wave ^ 4) * 2 + i) * FN + j) * 64 + lane];
+  const int wm4 = 2 * wm + team;  // this wave's 32 x 64 tile in a 4 x 2 grid
+
+  static_assert(sizeof(smem) >= out_tile_bytes(P::BM, P::BN), "output tile must fit the stages");
+  if constexpr (SPLIT > 1) {
+    // fp32 partial sums in D layout, as in gemm_w8a16_pipe_kernel
+    float* Pp = Pw + (size_t)part * M * N;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        const int n = n0 + wn * 64 + j * 16 + r16;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int m = m0 + wm4 * 32 + i * 16 + g * 4 + v;
+          if (m < M && n < N) Pp[(size_t)m * N + n] = sum[i][j][v];
+        }
+      }
+  } else {
+    store_tile<T, P::BM, P::BN, 4, 2, 512>(sum, smem, wm4, wn, lane, m0, n0, M, N, nullptr, nullptr, 1.f, Y, 0, 0, scale,
+                                           skind);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // w8a16 with N <= 16 and M > 16 (the reference's tiny-N M-parallel path,
 // fp8_GEMM_pert.h:3913-3994 via the dispatcher at :4030-4046): here the
 // activations are the large operand, so the roles flip.  A workgroup owns 16
@@ -1281,7 +1469,7 @@ constexpr int64_t kStreamM = 64;
 // M <= 16 the GEMV kernels, N <= 16 the activation-streaming kernel,
 // 16 < M <= 64 the weight-streaming kernel (cek_stream.hip), else the tiled
 // MFMA GEMM (or the generic kernels for unaligned shapes).
-// Tiled w8a16 configurations of the round model (M, N >= 128, matrices
+// Tiled w8a16 configurations of the round model (M > 64, N >= 128, matrices
 // below 4 GB): the 8-wave register-pipelined kernel (2 x 4 waves, four
 // loader waves) with its ring slots, and t0 / step of the round model (us
 // per round: t0 + step per 64-deep K step of one workgroup), fitted to the
@@ -1289,16 +1477,30 @@ constexpr int64_t kStreamM = 64;
 //  0  256 x 128, 3 slots;   1  256 x 192, 3 slots;   2  256 x 256, 2 slots;
 //  3  128 x 256, 3 slots;   4  128 x 128, 3 slots (split K only);
 //  5  128 x 96 (4 x 2 waves, two loader waves), 3 slots, unsplit, only as one
-//     round of 192 .. 256 tiles with K <= 8192 (fitted at M = 512, N = 6144).
-// Unsplit: 0-3 and 5; split in 2, 4 or 8 parts (K values per part >= 1024): 0
-// and 3, and 4 in 4 or 8 parts.  On the nine config-4 shapes (HBM and
+//     round of 192 .. 256 tiles with K <= 8192 (fitted at M = 512, N = 6144);
+//  6  128 x 128 in two K teams (gemm_w8a16_team_kernel), 3 slots, unsplit or
+//     split, only as one round of at most 256 workgroups, where it is 4-10%
+//     faster than 4 (two rounds are slower: a workgroup's fill is longer).
+//     Also for 64 < M < 128.  In that round a workgroup takes t0 + step per
+//     64-deep step, 0.9 of it with few others and 1.1 with all CUs busy.  (An
+//     unsplit launch of the others that does not fill its first round pays a
+//     whole t0, at least 4.3: 128 x 256, M = 256, K = 1024, N = 5120 16.4 us in
+//     40 workgroups, against 11.7 in 80 of 6.)
+//     Measured (us, weights from HBM, before -> now): M = 333, K = 2560, N =
+//     10752 32.0 (256 split parts of 128 x 256) -> 23.5; M = 512, K = 4096, N =
+//     6144 32.0 -> 30.2; M = 256, K = 14336, N = 4096 in 4 parts 37.7 -> 36.2;
+//     M = 100, K = 4096, N = 6144 47.9 (128 x 128, two per CU) -> 29.5, in 4
+//     parts of 4 18.5.
+// Unsplit: 0-3, 5 and 6; split in 2, 4 or 8 parts (K values per part >= 1024):
+// 0, 3 and 6, and 4 in 4 or 8 parts.  On the nine config-4 shapes (HBM and
 // cache-resident) and ten others (M = 128 .. 3000) the plan's pick measured
 // within 7% of the fastest of sixteen forms (M = 512, K = 14336: 171 -> 68 us
 // split in 4; M = 512, K = 4096, N = 6144: 52 -> 36 us).
 struct W8Opt { int bm, bn; double t0, step; };
-constexpr int kW8Cfgs = 6;
+constexpr int kW8Cfgs = 7;
 constexpr W8Opt kW8Opts[kW8Cfgs] = {{256, 128, 0.49, 0.972}, {256, 192, 6.84, 1.166}, {256, 256, 0.0, 1.595},
-                                    {128, 256, 2.05, 0.904}, {128, 128, 0.0, 0.491},  {128, 96, 4.30, 0.447}};
+                                    {128, 256, 2.05, 0.904}, {128, 128, 0.0, 0.491},  {128, 96, 4.30, 0.447},
+                                    {128, 128, 5.0, 0.400}};
 struct W8Plan { int cfg, split; };
 
 static bool w8_off32(int64_t M, int64_t N, int64_t K) {
@@ -1309,23 +1511,29 @@ static bool w8_off32(int64_t M, int64_t N, int64_t K) {
 // launch_w8a16 applies)
 static W8Plan plan_w8a16(int64_t M, int64_t N, int64_t K, bool allow_split) {
   W8Plan best{-1, 1};
-  if (M < 128 || N < 128 || K % 64 != 0 || !w8_off32(M, N, K)) return best;
+  if (M <= kStreamM || N < 128 || K % 64 != 0 || !w8_off32(M, N, K)) return best;
   double tbest = -1.0;
   for (int c = 0; c < kW8Cfgs; ++c) {
     const W8Opt& o = kW8Opts[c];
-    if (M < o.bm || N < o.bn) continue;
+    // (128 rows at 64 < M < 128 for 4 and 6: every tiled kernel's loads clamp rows)
+    if ((M < o.bm && c != 4 && c != 6) || N < o.bn) continue;
     for (int sp : {1, 2, 4, 8}) {
-      const bool ok = sp == 1 ? c != 4 : (allow_split && (c == 0 || c == 3 || (c == 4 && sp >= 4)));
+      const bool ok = sp == 1 ? c != 4 : (allow_split && (c == 0 || c == 3 || c == 6 || (c == 4 && sp >= 4)));
       if (!ok || (K / 64) % sp || (sp > 1 && K / sp < 1024)) continue;
       const int64_t units = ((M + o.bm - 1) / o.bm) * ((N + o.bn - 1) / o.bn) * sp;
       // 128 x 96 only as one nearly full round of at most 8192 K values, where
       // it was measured (M = 384 / 512, N = 6144, K = 1024 .. 8192; with a
       // quarter or more of the CUs idle, or two rounds, it lost)
       if (c == 5 && (units > 256 || units < 192 || K > 8192)) continue;
+      if (c == 6 && units > 256) continue;
       const int64_t full = units / 256;
       const double f = (double)(units - full * 256) / 256.0;
-      const double rounds = (double)full + (f > 0.0 ? 0.6 + 0.4 * f : 0.0);
-      double t = rounds * (o.t0 + (double)(K / 64 / sp) * o.step);
+      const double steps = (double)(K / 64 / sp) * o.step;
+      const double part = 0.6 + 0.4 * f;
+      double t;
+      if (c == 6) t = (0.9 + 0.2 * (double)units / 256.0) * (o.t0 + steps);
+      else if (full == 0 && sp == 1) t = std::max(o.t0, 4.3) + steps * part;
+      else t = ((double)full + (f > 0.0 ? part : 0.0)) * (o.t0 + steps);
       if (sp > 1) t += ((double)sp * M * N * 4.0 + (double)M * N * 2.0) / 5.0e6 + 1.5;
       if (tbest < 0 || t < tbest) {
         tbest = t;
@@ -1338,7 +1546,7 @@ static W8Plan plan_w8a16(int64_t M, int64_t N, int64_t K, bool allow_split) {
 
 // Bytes of fp32 partials the w8a16 split-K plan needs for (M, N, K) (0: unsplit).
 static int64_t w8a16_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  if (M <= 32 || N <= 16 || M > 65535 * 64 || N > INT32_MAX || K > INT32_MAX || K <= 0) return 0;
+  if (M <= kStreamM || N <= 16 || M > 65535 * 64 || N > INT32_MAX || K > INT32_MAX || K <= 0) return 0;
   const W8Plan p = plan_w8a16(M, N, K, true);
   return p.split > 1 ? (int64_t)p.split * M * N * 4 : 0;
 }
@@ -1406,6 +1614,16 @@ int launch_w8a16(const void* x, const void* w, const void* scale, int skind, voi
     gemm_w8a16_pipe_kernel<TY, F, 128, 96, 1, 4, 2, 2, 1, 3>                                                    \
         <<<dim3((unsigned)(tm * tn)), 512, 0, st>>>(xp, wp, scale, skind, yp, ws, M, N, K, tm, tn);             \
   } while (0)
+// 128 x 128 in two K teams
+#define CEK_W8T(TY, F, SP)                                                                                       \
+  do {                                                                                                          \
+    const int tm = (int)((M + 127) / 128), tn = (int)((N + 127) / 128);                                          \
+    gemm_w8a16_team_kernel<TY, F, SP, 3>                                                                         \
+        <<<dim3((unsigned)(tm * tn * SP)), 512, 0, st>>>(xp, wp, scale, skind, yp, ws, M, N, K, tm, tn);         \
+    if (SP > 1)                                                                                                 \
+      gemm_splitk_finalize_w<TY, SP><<<dim3((unsigned)((N + 2047) / 2048), (unsigned)(M < 65535 ? M : 65535)),  \
+                                        256, 0, st>>>(ws, scale, skind, yp, (int)M, (int)N);                     \
+  } while (0)
 #define CEK_W8P_SPLITS(TY, F, BM, BN)                        \
   do {                                                       \
     if (plan.split == 2) CEK_W8P(TY, F, BM, BN, 2, 3);       \
@@ -1414,7 +1632,12 @@ int launch_w8a16(const void* x, const void* w, const void* scale, int skind, voi
   } while (0)
 #define CEK_W8P_ALL(TY, F)                                                 \
   do {                                                                     \
-    if (plan.split > 1) {                                                  \
+    if (plan.cfg == 6) {                                                   \
+      if (plan.split == 1) CEK_W8T(TY, F, 1);                              \
+      else if (plan.split == 2) CEK_W8T(TY, F, 2);                         \
+      else if (plan.split == 4) CEK_W8T(TY, F, 4);                         \
+      else CEK_W8T(TY, F, 8);                                              \
+    } else if (plan.split > 1) {                                           \
       if (plan.cfg == 0) CEK_W8P_SPLITS(TY, F, 256, 128);                  \
       else if (plan.cfg == 3) CEK_W8P_SPLITS(TY, F, 128, 256);             \
       else if (plan.split == 4) CEK_W8P(TY, F, 128, 128, 4, 3);            \
@@ -1437,6 +1660,7 @@ int launch_w8a16(const void* x, const void* w, const void* scale, int skind, voi
       else CEK_W8P_ALL(BF16, CEK_E5M2);
 #undef CEK_W8P_ALL
 #undef CEK_W8P96
+#undef CEK_W8T
 #undef CEK_W8P_SPLITS
 #undef CEK_W8P
       return check_launch();
