@@ -53,15 +53,19 @@ __device__ inline float f32_round(float v) {
 }
 
 // gelu with the tanh approximation, fp32 math:
-// gelu_tanh(u) = 0.5 u (1 + tanh(sqrt(2/pi) (u + 0.044715 u^3))).  One
-// definition for gelu_and_mul and the GEMV epilogue that fuses it, each
-// operation rounded to fp32 (no contraction into fma), so every call site
-// computes the same value.
+// gelu_tanh(u) = 0.5 u (1 + tanh(z)) = u / (1 + exp(-2 z)),
+// z = sqrt(2/pi) (u + 0.044715 u^3), with the hardware exp2 and reciprocal
+// (1 ulp each): about ten VALU operations where tanhf takes several times as
+// many, and no 1 + tanh cancellation for negative u.  Infinities and overflow
+// of u^3 end as with tanh: exp2 gives 0 or inf, the reciprocal 1 or 0.  One
+// definition for gelu_and_mul and the kernels that fuse it, each operation
+// rounded to fp32 (no contraction into fma), so every call site computes the
+// same value.
 __device__ inline float gelu_tanh(float u) {
 #pragma clang fp contract(off)
-  const float k0 = 0.7978845608028654f;  // sqrt(2/pi)
+  const float k0 = -2.3022081985f;  // -2 sqrt(2/pi) log2(e)
   const float k1 = 0.044715f;
-  return 0.5f * u * (1.0f + tanhf(k0 * (u + k1 * u * u * u)));
+  return u * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(k0 * (u + k1 * u * u * u)));
 }
 
 // Decode the two fp8 bytes in the low (HI=false) or high (HI=true) half of
@@ -172,8 +176,23 @@ __device__ inline uint32_t f32x4_to_e4m3x4(float a, float b, float c, float d) {
 constexpr float E4M3_MAX = 448.0f;
 constexpr float MIN_SCALE = 1.0f / (448.0f * 512.0f);
 __device__ inline float quant_scale(float amax) { return fmaxf(amax / E4M3_MAX, MIN_SCALE); }
-__device__ inline float quant_clamp(float v, float s) {
-  return fminf(fmaxf(v / s, -E4M3_MAX), E4M3_MAX);  // IEEE divide (no fast math)
+// The IEEE quotient v / s of every element by its row's one scale, without a
+// divide per element: r = 1 / s rounded once per row, q0 = v r, and the
+// correction q0 + r (v - q0 s) in two fma, which is the correctly rounded
+// quotient when r is the correctly rounded reciprocal (Markstein, "Computation
+// of elementary functions on the IBM RISC System/6000 processor", 1990) -- four
+// VALU operations where the compiler's divide takes about twelve.  The sign
+// of a zero quotient is v's.  s = inf (a row that holds one): s = 1, r = 0 give
+// the quotients v / inf = 0 and inf / inf = NaN.
+struct QuantDiv { float s, r; };
+__device__ inline QuantDiv quant_div(float s) {
+  const bool inf = __builtin_isinf(s);
+  return QuantDiv{inf ? 1.0f : s, inf ? 0.0f : 1.0f / s};
+}
+__device__ inline float quant_clamp(float v, QuantDiv d) {
+  const float q0 = v * d.r;
+  const float q = fmaf(fmaf(-q0, d.s, v), d.r, q0);
+  return fminf(fmaxf(__builtin_copysignf(q, v), -E4M3_MAX), E4M3_MAX);
 }
 
 // Butterfly sum over the 64 lanes of a wave; every lane gets the total.

@@ -933,6 +933,7 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs 
         const float* mx = nsh + (MX + m) * 4;
         const float sq = quant_scale(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])));
         rsc[m] = sq;
+        const QuantDiv qd = quant_div(sq);
         if (side && m < M && t == 0) na.s_out[m] = sq;
 #pragma unroll
         for (int j = 0; j < NU; ++j) {
@@ -942,8 +943,8 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs 
 #pragma unroll
           for (int e = 0; e < 2; ++e) {
             const uint32_t a = nv[m][j][2 * e], b = nv[m][j][2 * e + 1];
-            c[e] = f32x4_to_e4m3x4(quant_clamp(TN::to_f32(a & 0xFFFF), sq), quant_clamp(TN::to_f32(a >> 16), sq),
-                                   quant_clamp(TN::to_f32(b & 0xFFFF), sq), quant_clamp(TN::to_f32(b >> 16), sq));
+            c[e] = f32x4_to_e4m3x4(quant_clamp(TN::to_f32(a & 0xFFFF), qd), quant_clamp(TN::to_f32(a >> 16), qd),
+                                   quant_clamp(TN::to_f32(b & 0xFFFF), qd), quant_clamp(TN::to_f32(b >> 16), qd));
           }
           // unit u = half u & 1 of 16-code chunk (u % 128) / 2 of stage u / 128
           *reinterpret_cast<uint2*>(xall + (u >> 7) * XSTAGE + m * XROW + 16 * (((u & 127) >> 1) ^ (m & 7)) +

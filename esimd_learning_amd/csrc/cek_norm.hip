@@ -34,7 +34,7 @@ __device__ inline float block_max(float v, float* sh) {
 
 
 // Vector path: H % 8 == 0, 16-byte aligned rows, H <= 8 * NORM_THREADS * UPT.
-template <typename T, int UPT, bool QUANT>
+template <typename T, int UPT, bool QUANT, bool EARLY>
 __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_kernel(
     uint16_t* __restrict__ hidden, uint16_t* __restrict__ residual,
     const uint16_t* __restrict__ weight, int H, float eps,
@@ -45,13 +45,28 @@ __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_kernel(
   uint16_t* hr = hidden + (size_t)row * H;
   uint16_t* rr = residual + (size_t)row * H;
 
-  u4 rv[UPT];
+  // EARLY (up to 1024 rows, where the chain of latencies is what a launch
+  // takes, and always when quantising): the norm weight's loads go out with the
+  // row's, not after the reduction (64 rows of 5120 3.9 -> 3.5 us, quantising
+  // 5.0 -> 4.3; 2048 rows of 4096 quantising 14.8 -> 13.5, but 2% slower
+  // without, which HBM bounds)
+  u4 hv[UPT], rv[UPT], wv[UPT];
+#pragma unroll
+  for (int j = 0; j < UPT; ++j) {
+    const int u = min((int)threadIdx.x + j * NORM_THREADS, units - 1);
+    hv[j] = load_u4(hr + u * 8);
+    rv[j] = load_u4(rr + u * 8);
+  }
+  if constexpr (EARLY) {
+#pragma unroll
+    for (int j = 0; j < UPT; ++j) wv[j] = load_u4(weight + min((int)threadIdx.x + j * NORM_THREADS, units - 1) * 8);
+  }
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < UPT; ++j) {
     const int u = threadIdx.x + j * NORM_THREADS;
     if (u < units) {
-      const u4 o = addnorm_pass1<T>(load_u4(hr + u * 8), load_u4(rr + u * 8), ss);
+      const u4 o = addnorm_pass1<T>(hv[j], rv[j], ss);
       rv[j] = o;
       *reinterpret_cast<u4*>(rr + u * 8) = o;
     }
@@ -65,7 +80,8 @@ __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_kernel(
   for (int j = 0; j < UPT; ++j) {
     const int u = threadIdx.x + j * NORM_THREADS;
     if (u < units) {
-      const u4 o = addnorm_pass2<T>(rv[j], load_u4(weight + u * 8), inv);
+      if constexpr (!EARLY) wv[j] = load_u4(weight + u * 8);
+      const u4 o = addnorm_pass2<T>(rv[j], wv[j], inv);
       if (QUANT) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -80,6 +96,7 @@ __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_kernel(
 
   amax = block_max(amax, sh);
   const float s = quant_scale(amax);
+  const QuantDiv qd = quant_div(s);
   if (threadIdx.x == 0) qscale[row] = s;
   uint8_t* qr = q + (size_t)row * H;
 #pragma unroll
@@ -90,8 +107,8 @@ __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_kernel(
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         const uint32_t a = nv[j][2 * e], b = nv[j][2 * e + 1];
-        c[e] = f32x4_to_e4m3x4(quant_clamp(T::to_f32(a & 0xFFFF), s), quant_clamp(T::to_f32(a >> 16), s),
-                               quant_clamp(T::to_f32(b & 0xFFFF), s), quant_clamp(T::to_f32(b >> 16), s));
+        c[e] = f32x4_to_e4m3x4(quant_clamp(T::to_f32(a & 0xFFFF), qd), quant_clamp(T::to_f32(a >> 16), qd),
+                               quant_clamp(T::to_f32(b & 0xFFFF), qd), quant_clamp(T::to_f32(b >> 16), qd));
       }
       *reinterpret_cast<uint2*>(qr + u * 8) = make_uint2(c[0], c[1]);
     }
@@ -125,14 +142,16 @@ __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_generic_kernel(
   if (!QUANT) return;
   amax = block_max(amax, sh);
   const float s = quant_scale(amax);
+  const QuantDiv qd = quant_div(s);
   if (threadIdx.x == 0) qscale[row] = s;
   for (int i = threadIdx.x; i < H; i += NORM_THREADS) {
     uint16_t b = T::from_f32(f32_round(T::to_f32(rr[i]) * inv * T::to_f32(weight[i])));
-    q[(size_t)row * H + i] = (uint8_t)f32_to_e4m3(quant_clamp(T::to_f32(b), s));
+    q[(size_t)row * H + i] = (uint8_t)f32_to_e4m3(quant_clamp(T::to_f32(b), qd));
   }
 }
 
-// Per-token quantisation of a [rows, H] activation matrix.
+// Per-token quantisation of a [rows, H] activation matrix: rows that the
+// register form below does not take (unaligned, or longer than 32768).
 template <typename T>
 __global__ __launch_bounds__(NORM_THREADS) void per_token_quant_kernel(
     const uint16_t* __restrict__ x, int H, uint8_t* __restrict__ q, float* __restrict__ qscale, int vec) {
@@ -153,6 +172,7 @@ __global__ __launch_bounds__(NORM_THREADS) void per_token_quant_kernel(
   }
   amax = block_max(amax, sh);
   const float s = quant_scale(amax);
+  const QuantDiv qd = quant_div(s);
   if (threadIdx.x == 0) qscale[row] = s;
   if (vec) {
     for (int u = threadIdx.x; u < (H >> 3); u += NORM_THREADS) {
@@ -161,15 +181,79 @@ __global__ __launch_bounds__(NORM_THREADS) void per_token_quant_kernel(
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         const uint32_t a = v[2 * e], b = v[2 * e + 1];
-        c[e] = f32x4_to_e4m3x4(quant_clamp(T::to_f32(a & 0xFFFF), s), quant_clamp(T::to_f32(a >> 16), s),
-                               quant_clamp(T::to_f32(b & 0xFFFF), s), quant_clamp(T::to_f32(b >> 16), s));
+        c[e] = f32x4_to_e4m3x4(quant_clamp(T::to_f32(a & 0xFFFF), qd), quant_clamp(T::to_f32(a >> 16), qd),
+                               quant_clamp(T::to_f32(b & 0xFFFF), qd), quant_clamp(T::to_f32(b >> 16), qd));
       }
       *reinterpret_cast<uint2*>(qr + u * 8) = make_uint2(c[0], c[1]);
     }
   } else {
     for (int i = threadIdx.x; i < H; i += NORM_THREADS)
-      qr[i] = (uint8_t)f32_to_e4m3(quant_clamp(T::to_f32(xr[i]), s));
+      qr[i] = (uint8_t)f32_to_e4m3(quant_clamp(T::to_f32(xr[i]), qd));
   }
+}
+
+// The same with the row held in registers between the maximum and the codes
+// (read once): H % 8 == 0, 16-byte aligned rows, H <= 8 NT UPT.  The maximum does
+// not depend on the thread layout, so neither do scale and codes.  What bounds
+// it: HBM for many rows (2048 rows of 14336: 28.6 us reading twice with a
+// divide per element -> 20.4; 23.4 with 1024 threads a row), the chain load,
+// reduction, store for few, so a long row takes up to 1024 threads (64 rows of
+// 14336 7.1 -> 3.9 us, 4 of 24576 8.7 -> 4.3).
+template <typename T, int NT, int UPT>
+__global__ __launch_bounds__(NT) void per_token_quant_row_kernel(const uint16_t* __restrict__ x, int H,
+                                                                 uint8_t* __restrict__ q, float* __restrict__ qscale) {
+  __shared__ float sh[NT / 64];
+  const int row = blockIdx.x, units = H >> 3;
+  const uint16_t* xr = x + (size_t)row * H;
+  uint8_t* qr = q + (size_t)row * H;
+  u4 v[UPT];
+#pragma unroll
+  for (int j = 0; j < UPT; ++j) v[j] = load_u4(xr + min((int)threadIdx.x + j * NT, units - 1) * 8);
+  float amax = 0.f;  // (units past the row repeat its last one)
+#pragma unroll
+  for (int j = 0; j < UPT; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      amax = fmaxf(amax, fmaxf(fabsf(T::to_f32(v[j][e] & 0xFFFF)), fabsf(T::to_f32(v[j][e] >> 16))));
+  amax = wave_max(amax);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = amax;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) amax = fmaxf(amax, sh[w]);
+  const float s = quant_scale(amax);
+  const QuantDiv qd = quant_div(s);
+  if (threadIdx.x == 0) qscale[row] = s;
+#pragma unroll
+  for (int j = 0; j < UPT; ++j) {
+    const int u = threadIdx.x + j * NT;
+    if (u < units) {
+      uint32_t c[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const uint32_t a = v[j][2 * e], b = v[j][2 * e + 1];
+        c[e] = f32x4_to_e4m3x4(quant_clamp(T::to_f32(a & 0xFFFF), qd), quant_clamp(T::to_f32(a >> 16), qd),
+                               quant_clamp(T::to_f32(b & 0xFFFF), qd), quant_clamp(T::to_f32(b >> 16), qd));
+      }
+      *reinterpret_cast<uint2*>(qr + u * 8) = make_uint2(c[0], c[1]);
+    }
+  }
+}
+
+template <typename T>
+static void launch_quant_t(const uint16_t* x, int64_t rows, int H, uint8_t* q, float* s, bool vec, hipStream_t st) {
+  const dim3 grid((unsigned)rows);
+  const int units = H / 8;
+  // many rows: few threads per row, so that a CU holds many rows in flight;
+  // few rows: many threads, for the latency of a long row
+  const bool many = rows >= 512;
+#define CEK_Q(NT, UPT) per_token_quant_row_kernel<T, NT, UPT><<<grid, NT, 0, st>>>(x, H, q, s)
+  if (vec && units <= 256) CEK_Q(256, 1);
+  else if (vec && units <= 512) CEK_Q(256, 2);
+  else if (vec && units <= 1024) { if (many) CEK_Q(256, 4); else CEK_Q(512, 2); }
+  else if (vec && units <= 2048) { if (many) CEK_Q(256, 8); else CEK_Q(1024, 2); }
+  else if (vec && units <= 4096) { if (many) CEK_Q(512, 8); else CEK_Q(1024, 4); }
+  else per_token_quant_kernel<T><<<grid, NORM_THREADS, 0, st>>>(x, H, q, s, vec);
+#undef CEK_Q
 }
 
 template <typename T, bool QUANT>
@@ -183,11 +267,17 @@ static int launch_norm_t(void* hidden, void* residual, const void* weight, int r
                    (!QUANT || aligned(q, 8));
   const int upt = (units + NORM_THREADS - 1) / NORM_THREADS;
   dim3 grid(rows);
-  if (vec && upt <= 1) add_rmsnorm_kernel<T, 1, QUANT><<<grid, NORM_THREADS, 0, st>>>(h, r, w, H, eps, q, qs);
-  else if (vec && upt <= 2) add_rmsnorm_kernel<T, 2, QUANT><<<grid, NORM_THREADS, 0, st>>>(h, r, w, H, eps, q, qs);
-  else if (vec && upt <= 3) add_rmsnorm_kernel<T, 3, QUANT><<<grid, NORM_THREADS, 0, st>>>(h, r, w, H, eps, q, qs);
-  else if (vec && upt <= 4) add_rmsnorm_kernel<T, 4, QUANT><<<grid, NORM_THREADS, 0, st>>>(h, r, w, H, eps, q, qs);
-  else if (vec && upt <= 8) add_rmsnorm_kernel<T, 8, QUANT><<<grid, NORM_THREADS, 0, st>>>(h, r, w, H, eps, q, qs);
+#define CEK_NORM(UPT)                                                                                          \
+  do {                                                                                                         \
+    if (QUANT || rows <= 1024) add_rmsnorm_kernel<T, UPT, QUANT, true><<<grid, NORM_THREADS, 0, st>>>(h, r, w, H, eps, q, qs); \
+    else add_rmsnorm_kernel<T, UPT, QUANT, false><<<grid, NORM_THREADS, 0, st>>>(h, r, w, H, eps, q, qs);      \
+  } while (0)
+  if (vec && upt <= 1) CEK_NORM(1);
+  else if (vec && upt <= 2) CEK_NORM(2);
+  else if (vec && upt <= 3) CEK_NORM(3);
+  else if (vec && upt <= 4) CEK_NORM(4);
+  else if (vec && upt <= 8) CEK_NORM(8);
+#undef CEK_NORM
   else add_rmsnorm_generic_kernel<T, QUANT><<<grid, NORM_THREADS, 0, st>>>(h, r, w, H, eps, q, qs);
   return check_launch();
 }
@@ -234,10 +324,10 @@ extern "C" int cek_per_token_quant_fp8(const void* x, int64_t rows, int64_t H, i
   if (rows == 0) return CEK_OK;
   if (!x || !q || !scale) return CEK_ERR_INVALID;
   hipStream_t st = (hipStream_t)stream;
-  const int vec = H % 8 == 0 && aligned(x, 16) && aligned(q, 8);
+  const bool vec = H % 8 == 0 && aligned(x, 16) && aligned(q, 8);
   const uint16_t* xp = static_cast<const uint16_t*>(x);
-  if (io_dtype == CEK_F16) per_token_quant_kernel<F16><<<dim3(rows), NORM_THREADS, 0, st>>>(xp, H, q, scale, vec);
-  else if (io_dtype == CEK_BF16) per_token_quant_kernel<BF16><<<dim3(rows), NORM_THREADS, 0, st>>>(xp, H, q, scale, vec);
+  if (io_dtype == CEK_F16) launch_quant_t<F16>(xp, rows, (int)H, q, scale, vec, st);
+  else if (io_dtype == CEK_BF16) launch_quant_t<BF16>(xp, rows, (int)H, q, scale, vec, st);
   else return CEK_ERR_INVALID;
   return check_launch();
 }
