@@ -2102,13 +2102,22 @@ extern "C" int cek_gemv_fp8_gelu_and_mul(const void* x, const float* x_scale, co
 
 // More than 16 rows: the w8a16 GEMM dispatch (cek_gemm.hip), which streams
 // the weights once for all rows instead of once per 16-row slab.
+extern "C" int cek_gemv_fp8_pern_ws(const void* x, const void* w, const void* scale, void* y,
+                                    int64_t M, int64_t N, int64_t K, int io_dtype, int fp8_fmt, int scale_dtype,
+                                    void* workspace, int64_t workspace_bytes, void* stream) {
+  const int skind = cek::scale_kind(scale_dtype);
+  if (skind < 0) return CEK_ERR_INVALID;
+  if (workspace_bytes < 0 || (workspace_bytes > 0 && (!workspace || !cek::aligned(workspace, 4)))) return CEK_ERR_INVALID;
+  if (M > 16)
+    return cek::launch_w8a16(x, w, scale, skind, y, M, N, K, io_dtype, fp8_fmt, static_cast<float*>(workspace),
+                             workspace_bytes, (hipStream_t)stream);
+  return cek::launch_gemv(x, w, scale, skind, y, M, N, K, io_dtype, fp8_fmt, (hipStream_t)stream);
+}
+
 extern "C" int cek_gemv_fp8_pern(const void* x, const void* w, const void* scale, void* y,
                                  int64_t M, int64_t N, int64_t K,
                                  int io_dtype, int fp8_fmt, int scale_dtype, void* stream) {
-  const int skind = cek::scale_kind(scale_dtype);
-  if (skind < 0) return CEK_ERR_INVALID;
-  if (M > 16) return cek::launch_w8a16(x, w, scale, skind, y, M, N, K, io_dtype, fp8_fmt, nullptr, 0, (hipStream_t)stream);
-  return cek::launch_gemv(x, w, scale, skind, y, M, N, K, io_dtype, fp8_fmt, (hipStream_t)stream);
+  return cek_gemv_fp8_pern_ws(x, w, scale, y, M, N, K, io_dtype, fp8_fmt, scale_dtype, nullptr, 0, stream);
 }
 
 extern "C" int cek_gemv_fp8_pert(const void* x, const void* w, const float* scale, void* y,

@@ -36,14 +36,15 @@ __device__ inline float block_max(float v, float* sh) {
 // Vector path: H % 8 == 0, 16-byte aligned rows, H <= 8 * NORM_THREADS * UPT.
 template <typename T, int UPT, bool QUANT, bool EARLY>
 __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_kernel(
-    uint16_t* __restrict__ hidden, uint16_t* __restrict__ residual,
-    const uint16_t* __restrict__ weight, int H, float eps,
-    uint8_t* __restrict__ q, float* __restrict__ qscale) {
+    const uint16_t* hidden, const uint16_t* residual, uint16_t* hidden_out, uint16_t* residual_out,
+    const uint16_t* __restrict__ weight, int H, float eps, uint8_t* __restrict__ q, float* __restrict__ qscale) {
   __shared__ float sh[4];
   const int row = blockIdx.x;
   const int units = H >> 3;
-  uint16_t* hr = hidden + (size_t)row * H;
-  uint16_t* rr = residual + (size_t)row * H;
+  const uint16_t* hr = hidden + (size_t)row * H;
+  const uint16_t* rr = residual + (size_t)row * H;
+  uint16_t* ho = hidden_out + (size_t)row * H;
+  uint16_t* ro = residual_out + (size_t)row * H;
 
   // EARLY (up to 1024 rows, where the chain of latencies is what a launch
   // takes, and always when quantising): the norm weight's loads go out with the
@@ -68,7 +69,7 @@ __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_kernel(
     if (u < units) {
       const u4 o = addnorm_pass1<T>(hv[j], rv[j], ss);
       rv[j] = o;
-      *reinterpret_cast<u4*>(rr + u * 8) = o;
+      *reinterpret_cast<u4*>(ro + u * 8) = o;
     }
   }
   ss = block_sum(ss, sh);
@@ -88,7 +89,7 @@ __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_kernel(
           amax = fmaxf(amax, fmaxf(fabsf(T::to_f32(o[e] & 0xFFFF)), fabsf(T::to_f32(o[e] >> 16))));
         nv[j] = o;
       } else {
-        *reinterpret_cast<u4*>(hr + u * 8) = o;
+        *reinterpret_cast<u4*>(ho + u * 8) = o;
       }
     }
   }
@@ -118,26 +119,27 @@ __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_kernel(
 // Scalar path for any H / alignment: three passes over global memory.
 template <typename T, bool QUANT>
 __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_generic_kernel(
-    uint16_t* __restrict__ hidden, uint16_t* __restrict__ residual,
-    const uint16_t* __restrict__ weight, int H, float eps,
-    uint8_t* __restrict__ q, float* __restrict__ qscale) {
+    const uint16_t* hidden, const uint16_t* residual, uint16_t* hidden_out, uint16_t* residual_out,
+    const uint16_t* __restrict__ weight, int H, float eps, uint8_t* __restrict__ q, float* __restrict__ qscale) {
   __shared__ float sh[4];
   const int row = blockIdx.x;
-  uint16_t* hr = hidden + (size_t)row * H;
-  uint16_t* rr = residual + (size_t)row * H;
+  const uint16_t* hr = hidden + (size_t)row * H;
+  const uint16_t* rr = residual + (size_t)row * H;
+  uint16_t* ho = hidden_out + (size_t)row * H;
+  uint16_t* ro = residual_out + (size_t)row * H;
   float ss = 0.f;
   for (int i = threadIdx.x; i < H; i += NORM_THREADS) {
     float a = T::to_f32(hr[i]) + T::to_f32(rr[i]);
     ss = fmaf(a, a, ss);
-    rr[i] = T::from_f32(a);  // re-read below by this same thread only
+    ro[i] = T::from_f32(a);  // re-read below by this same thread only
   }
   ss = block_sum(ss, sh);
   const float inv = rsqrtf(ss / (float)H + eps);
   float amax = 0.f;
   for (int i = threadIdx.x; i < H; i += NORM_THREADS) {
-    uint16_t b = T::from_f32(f32_round(T::to_f32(rr[i]) * inv * T::to_f32(weight[i])));
+    uint16_t b = T::from_f32(f32_round(T::to_f32(ro[i]) * inv * T::to_f32(weight[i])));
     if (QUANT) amax = fmaxf(amax, fabsf(T::to_f32(b)));
-    else hr[i] = b;
+    else ho[i] = b;
   }
   if (!QUANT) return;
   amax = block_max(amax, sh);
@@ -145,7 +147,7 @@ __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_generic_kernel(
   const QuantDiv qd = quant_div(s);
   if (threadIdx.x == 0) qscale[row] = s;
   for (int i = threadIdx.x; i < H; i += NORM_THREADS) {
-    uint16_t b = T::from_f32(f32_round(T::to_f32(rr[i]) * inv * T::to_f32(weight[i])));
+    uint16_t b = T::from_f32(f32_round(T::to_f32(ro[i]) * inv * T::to_f32(weight[i])));
     q[(size_t)row * H + i] = (uint8_t)f32_to_e4m3(quant_clamp(T::to_f32(b), qd));
   }
 }
@@ -257,20 +259,22 @@ static void launch_quant_t(const uint16_t* x, int64_t rows, int H, uint8_t* q, f
 }
 
 template <typename T, bool QUANT>
-static int launch_norm_t(void* hidden, void* residual, const void* weight, int rows, int H, float eps,
-                         uint8_t* q, float* qs, hipStream_t st) {
-  uint16_t* h = static_cast<uint16_t*>(hidden);
-  uint16_t* r = static_cast<uint16_t*>(residual);
+static int launch_norm_t(const void* hidden, const void* residual, void* hidden_out, void* residual_out,
+                         const void* weight, int rows, int H, float eps, uint8_t* q, float* qs, hipStream_t st) {
+  const uint16_t* h = static_cast<const uint16_t*>(hidden);
+  const uint16_t* r = static_cast<const uint16_t*>(residual);
+  uint16_t* ho = static_cast<uint16_t*>(hidden_out);
+  uint16_t* ro = static_cast<uint16_t*>(residual_out);
   const uint16_t* w = static_cast<const uint16_t*>(weight);
   const int units = H / 8;
   const bool vec = H % 8 == 0 && aligned(hidden, 16) && aligned(residual, 16) && aligned(weight, 16) &&
-                   (!QUANT || aligned(q, 8));
+                   aligned(residual_out, 16) && (QUANT ? aligned(q, 8) : aligned(hidden_out, 16));
   const int upt = (units + NORM_THREADS - 1) / NORM_THREADS;
   dim3 grid(rows);
 #define CEK_NORM(UPT)                                                                                          \
   do {                                                                                                         \
-    if (QUANT || rows <= 1024) add_rmsnorm_kernel<T, UPT, QUANT, true><<<grid, NORM_THREADS, 0, st>>>(h, r, w, H, eps, q, qs); \
-    else add_rmsnorm_kernel<T, UPT, QUANT, false><<<grid, NORM_THREADS, 0, st>>>(h, r, w, H, eps, q, qs);      \
+    if (QUANT || rows <= 1024) add_rmsnorm_kernel<T, UPT, QUANT, true><<<grid, NORM_THREADS, 0, st>>>(h, r, ho, ro, w, H, eps, q, qs); \
+    else add_rmsnorm_kernel<T, UPT, QUANT, false><<<grid, NORM_THREADS, 0, st>>>(h, r, ho, ro, w, H, eps, q, qs);      \
   } while (0)
   if (vec && upt <= 1) CEK_NORM(1);
   else if (vec && upt <= 2) CEK_NORM(2);
@@ -278,7 +282,7 @@ static int launch_norm_t(void* hidden, void* residual, const void* weight, int r
   else if (vec && upt <= 4) CEK_NORM(4);
   else if (vec && upt <= 8) CEK_NORM(8);
 #undef CEK_NORM
-  else add_rmsnorm_generic_kernel<T, QUANT><<<grid, NORM_THREADS, 0, st>>>(h, r, w, H, eps, q, qs);
+  else add_rmsnorm_generic_kernel<T, QUANT><<<grid, NORM_THREADS, 0, st>>>(h, r, ho, ro, w, H, eps, q, qs);
   return check_launch();
 }
 
@@ -292,30 +296,41 @@ static int norm_args_ok(const void* h, const void* r, const void* w, int64_t row
   return CEK_OK;
 }
 
-extern "C" int cek_fused_add_rms_norm(void* hidden, void* residual, const void* weight,
-                                      int64_t rows, int64_t H, float eps, int io_dtype, void* stream) {
+extern "C" int cek_add_rms_norm_out(const void* hidden, const void* residual, const void* weight, void* residual_out,
+                                    void* hidden_out, int64_t rows, int64_t H, float eps, int io_dtype, uint8_t* q,
+                                    float* scale, void* stream) {
   int rc = norm_args_ok(hidden, residual, weight, rows, H);
   if (rc) return rc;
   if (rows == 0) return CEK_OK;
+  if (!residual_out || (q ? !scale : !hidden_out)) return CEK_ERR_INVALID;
   hipStream_t st = (hipStream_t)stream;
-  if (io_dtype == CEK_F16) return launch_norm_t<F16, false>(hidden, residual, weight, rows, H, eps, nullptr, nullptr, st);
-  if (io_dtype == CEK_BF16) return launch_norm_t<BF16, false>(hidden, residual, weight, rows, H, eps, nullptr, nullptr, st);
+  const int r = (int)rows, h = (int)H;
+  void* ho = q ? residual_out : hidden_out;  // (never stored by the quantising form)
+  if (io_dtype == CEK_F16) {
+    if (q) return launch_norm_t<F16, true>(hidden, residual, ho, residual_out, weight, r, h, eps, q, scale, st);
+    return launch_norm_t<F16, false>(hidden, residual, ho, residual_out, weight, r, h, eps, nullptr, nullptr, st);
+  }
+  if (io_dtype == CEK_BF16) {
+    if (q) return launch_norm_t<BF16, true>(hidden, residual, ho, residual_out, weight, r, h, eps, q, scale, st);
+    return launch_norm_t<BF16, false>(hidden, residual, ho, residual_out, weight, r, h, eps, nullptr, nullptr, st);
+  }
   return CEK_ERR_INVALID;
+}
+
+extern "C" int cek_fused_add_rms_norm(void* hidden, void* residual, const void* weight,
+                                      int64_t rows, int64_t H, float eps, int io_dtype, void* stream) {
+  return cek_add_rms_norm_out(hidden, residual, weight, residual, hidden, rows, H, eps, io_dtype, nullptr, nullptr,
+                              stream);
 }
 
 extern "C" int cek_fused_add_rms_norm_quant_fp8(const void* hidden, void* residual, const void* weight,
                                                 int64_t rows, int64_t H, float eps, int io_dtype,
                                                 uint8_t* q, float* scale, void* stream) {
-  int rc = norm_args_ok(hidden, residual, weight, rows, H);
-  if (rc) return rc;
-  if (rows == 0) return CEK_OK;
-  if (!q || !scale) return CEK_ERR_INVALID;
-  hipStream_t st = (hipStream_t)stream;
-  // hidden is read-only in the quantising variant (the kernel never stores it).
-  void* h = const_cast<void*>(hidden);
-  if (io_dtype == CEK_F16) return launch_norm_t<F16, true>(h, residual, weight, rows, H, eps, q, scale, st);
-  if (io_dtype == CEK_BF16) return launch_norm_t<BF16, true>(h, residual, weight, rows, H, eps, q, scale, st);
-  return CEK_ERR_INVALID;
+  if (!q || !scale) {  // (no rows: nothing to write them to)
+    const int rc = norm_args_ok(hidden, residual, weight, rows, H);
+    return rc ? rc : (rows == 0 ? CEK_OK : CEK_ERR_INVALID);
+  }
+  return cek_add_rms_norm_out(hidden, residual, weight, residual, nullptr, rows, H, eps, io_dtype, q, scale, stream);
 }
 
 extern "C" int cek_per_token_quant_fp8(const void* x, int64_t rows, int64_t H, int io_dtype,

@@ -61,12 +61,15 @@ static void run_gemv(const at::Tensor& input, const at::Tensor& weight, const at
   const int io = io_code(input.scalar_type());
   const int fmt = fp8_code(weight);
   // Up to 16 rows the decode GEMV kernels; more rows the w8a16 GEMM, which
-  // streams the weights once for all of them.
-  const int rc = per_tensor ? cek_gemv_fp8_pert(input.data_ptr(), weight.data_ptr(),
-                                                static_cast<const float*>(scale.data_ptr()), output.data_ptr(), M, N,
-                                                K, io, fmt, st)
-                            : cek_gemv_fp8_pern(input.data_ptr(), weight.data_ptr(), scale.data_ptr(),
-                                                output.data_ptr(), M, N, K, io, fmt, scale_code, st);
+  // streams the weights once for all of them, split in K where its plan says so.
+  at::Tensor ws;
+  const int64_t need = M > 64 ? split_workspace(ws, cek_gemm_fp8_pert_workspace_size(M, N, K), input) : 0;
+  void* wp = need > 0 ? ws.data_ptr() : nullptr;
+  const int rc = per_tensor ? cek_gemm_fp8_pert_ws(input.data_ptr(), weight.data_ptr(),
+                                                   static_cast<const float*>(scale.data_ptr()), output.data_ptr(), M,
+                                                   N, K, io, fmt, wp, need, st)
+                            : cek_gemv_fp8_pern_ws(input.data_ptr(), weight.data_ptr(), scale.data_ptr(),
+                                                   output.data_ptr(), M, N, K, io, fmt, scale_code, wp, need, st);
   check_rc(rc, op);
 }
 
@@ -286,8 +289,10 @@ void esimd_gemv_fp8_gelu_and_mul(at::Tensor input, at::Tensor weight, at::Tensor
   if (M > 16) {
     // the GEMV over all rows at once (weights streamed once), then gelu_and_mul
     at::Tensor gu = at::empty({M, 2 * d}, input.options());
-    check_rc(cek_gemv_fp8_pern(input.data_ptr(), weight.data_ptr(), weight_scale.data_ptr(), gu.data_ptr(), M, 2 * d,
-                               K, io, fmt, scale_code, st),
+    at::Tensor ws;
+    const int64_t need = split_workspace(ws, cek_gemm_fp8_pert_workspace_size(M, 2 * d, K), input);
+    check_rc(cek_gemv_fp8_pern_ws(input.data_ptr(), weight.data_ptr(), weight_scale.data_ptr(), gu.data_ptr(), M,
+                                  2 * d, K, io, fmt, scale_code, need > 0 ? ws.data_ptr() : nullptr, need, st),
              op);
     check_rc(cek_gelu_and_mul(output.data_ptr(), gu.data_ptr(), M, d, 2 * d, d, io, st), op);
     return;
@@ -359,13 +364,15 @@ void esimd_qk_norm_rope(at::Tensor q, at::Tensor k, at::Tensor q_weight, at::Ten
 // ---- add+RMSNorm (+ quant) fused into the GEMV that consumes it ----
 // residual_out = hidden + residual; the normed rows (or their e4m3 codes and
 // scales) feed the GEMV (or the gate/up GEMV with gelu_and_mul).  Decode
-// batches of up to four rows run as one launch; other shapes, and a
-// residual_out that aliases the inputs, run the norm op on a copy and then
-// the GEMV op (the same values).
-// The norm kernels update their residual argument in place: residual_out
-// takes residual's values first (nothing to copy when it is residual).
-static void seed_residual_out(at::Tensor& residual_out, const at::Tensor& residual) {
-  if (at::get_overlap_status(residual_out, residual) != at::MemOverlapStatus::Full) residual_out.copy_(residual);
+// batches of up to four rows run as one launch; other shapes run the norm and
+// then the GEMV op (the same values), the norm on copies if residual_out
+// aliases its inputs.
+// Whether the norm may write residual_out while it reads hidden and residual:
+// it is residual, or shares no memory with either.
+static bool norm_writes_out(const at::Tensor& residual_out, const at::Tensor& hidden, const at::Tensor& residual) {
+  const auto with_r = at::get_overlap_status(residual_out, residual);
+  return (with_r == at::MemOverlapStatus::Full || with_r == at::MemOverlapStatus::No) &&
+         at::get_overlap_status(residual_out, hidden) == at::MemOverlapStatus::No;
 }
 
 static void check_norm_gemv_common(const at::Tensor& h, const at::Tensor& r, const at::Tensor& nw,
@@ -416,10 +423,13 @@ void esimd_fused_add_rms_norm_gemv_fp8(at::Tensor hidden_states, at::Tensor resi
     check_rc(rc, op);
     return;
   }
-  // two launches: the norm in place on copies, then the GEMV
-  at::Tensor x = hidden_states.clone();
-  seed_residual_out(residual_out, residual);
-  check_rc(cek_fused_add_rms_norm(x.data_ptr(), residual_out.data_ptr(), weight.data_ptr(), M, K, (float)eps, io, st),
+  // two launches: the norm, then the GEMV
+  at::Tensor x = at::empty_like(hidden_states);
+  const bool direct = norm_writes_out(residual_out, hidden_states, residual);
+  const at::Tensor h = direct ? hidden_states : hidden_states.clone();
+  const at::Tensor r = direct ? residual : residual.clone();
+  check_rc(cek_add_rms_norm_out(h.data_ptr(), r.data_ptr(), weight.data_ptr(), residual_out.data_ptr(), x.data_ptr(),
+                                M, K, (float)eps, io, nullptr, nullptr, st),
            op);
   if (gelu_and_mul) esimd_gemv_fp8_gelu_and_mul(x.view({M, K}), w, w_scale, output.view({M, N / 2}));
   else run_gemv(x, w, w_scale, output, N, K, false, op);
@@ -448,27 +458,31 @@ void esimd_fused_add_rms_norm_quant_gemv_fp8(at::Tensor hidden_states, at::Tenso
     check_rc(rc, op);
     return;
   }
-  // two launches: norm + quant (hidden only read), then the a8w8 product.
-  // hidden is read after residual_out has been seeded with residual, so it
-  // is read from a copy when residual_out shares its memory.
-  const at::Tensor h = at::get_overlap_status(residual_out, hidden_states) == at::MemOverlapStatus::No
-                           ? hidden_states
-                           : hidden_states.clone();
-  seed_residual_out(residual_out, residual);
-  check_rc(cek_fused_add_rms_norm_quant_fp8(h.data_ptr(), residual_out.data_ptr(), weight.data_ptr(), M, K,
-                                            (float)eps, io, q, qs, st),
+  // two launches: norm + quant, then the a8w8 product
+  const bool direct = norm_writes_out(residual_out, hidden_states, residual);
+  const at::Tensor h = direct ? hidden_states : hidden_states.clone();
+  const at::Tensor r = direct ? residual : residual.clone();
+  check_rc(cek_add_rms_norm_out(h.data_ptr(), r.data_ptr(), weight.data_ptr(), residual_out.data_ptr(), nullptr, M, K,
+                                (float)eps, io, q, qs, st),
            op);
   const auto* bp = static_cast<const uint8_t*>(b.data_ptr());
   const auto* sb = static_cast<const float*>(b_scale.data_ptr());
+  // At 64 rows the weight-streaming kernel that a call without a workspace
+  // takes is faster up to K = 5120 (us, streaming / split K: K = 4096, N = 6144
+  // 10.9 / 13.2, N = 14336 18.2 / 20.7; K = 8192, N = 4096 14.3 / 13.5).
+  at::Tensor ws;
+  const bool split = M > 64 || (M == 64 && (K > 5120 || N > 16384));
+  const int64_t need = split ? split_workspace(ws, cek_gemm_fp8_a8w8_workspace_size(M, N, K), out_scale) : 0;
+  void* wp = need > 0 ? ws.data_ptr() : nullptr;
   if (!gelu_and_mul) {
-    check_rc(cek_gemm_fp8_a8w8(q, qs, bp, sb, output.data_ptr(), M, N, K, io, st), op);
+    check_rc(cek_gemm_fp8_a8w8_ws(q, qs, bp, sb, output.data_ptr(), M, N, K, io, wp, need, st), op);
     return;
   }
   rc = M <= 16 ? cek_gemv_fp8_gelu_and_mul(q, qs, bp, sb, output.data_ptr(), M, N / 2, K, io, CEK_E4M3, CEK_F32, st)
                : CEK_ERR_UNSUPPORTED;
   if (rc == CEK_ERR_UNSUPPORTED) {
     at::Tensor gu = at::empty({M, N}, output.options());
-    check_rc(cek_gemm_fp8_a8w8(q, qs, bp, sb, gu.data_ptr(), M, N, K, io, st), op);
+    check_rc(cek_gemm_fp8_a8w8_ws(q, qs, bp, sb, gu.data_ptr(), M, N, K, io, wp, need, st), op);
     rc = cek_gelu_and_mul(output.data_ptr(), gu.data_ptr(), M, N / 2, N, N / 2, io, st);
   }
   check_rc(rc, op);

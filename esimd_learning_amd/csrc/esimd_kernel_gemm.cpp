@@ -130,7 +130,11 @@ void esimd_gemm_fp8_a8w8_gelu_and_mul(at::Tensor a, at::Tensor a_scale, at::Tens
                    : CEK_ERR_UNSUPPORTED;
   if (rc == CEK_ERR_UNSUPPORTED && M > 0 && d > 0) {
     at::Tensor gu = at::empty({M, 2 * d}, output.options());
-    check_rc(cek_gemm_fp8_a8w8(ap, sa, bp, sb, gu.data_ptr(), M, 2 * d, K, io, st), op);
+    at::Tensor ws;
+    const int64_t need = split_workspace(ws, cek_gemm_fp8_a8w8_workspace_size(M, 2 * d, K), a_scale);
+    check_rc(cek_gemm_fp8_a8w8_ws(ap, sa, bp, sb, gu.data_ptr(), M, 2 * d, K, io, need > 0 ? ws.data_ptr() : nullptr,
+                                  need, st),
+             op);
     rc = cek_gelu_and_mul(output.data_ptr(), gu.data_ptr(), M, d, 2 * d, d, io, st);
   }
   check_rc(rc, op);

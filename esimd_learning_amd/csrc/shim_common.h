@@ -47,4 +47,11 @@ inline void check_rc(int rc, const char* op) {
               rc == CEK_ERR_HIP ? cek_last_hip_error() : "");
 }
 
+// The split-K workspace of `need` bytes (a *_workspace_size; 0: none) on like's
+// device, from the caching allocator (no kernel runs to allocate or clear it).
+inline int64_t split_workspace(at::Tensor& ws, int64_t need, const at::Tensor& like) {
+  if (need > 0) ws = at::empty({(need + 3) / 4}, like.options().dtype(at::kFloat));
+  return need;
+}
+
 }  // namespace cek_shim

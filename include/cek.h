@@ -70,6 +70,15 @@ int cek_gemv_fp8_pert(const void* x, const void* w, const float* scale, void* y,
                       int io_dtype, int fp8_fmt, void* stream);
 
 /*
+ * cek_gemv_fp8_pern with a workspace for the split-K forms that more than 64
+ * rows may take (the contract of cek_gemm_fp8_pert_ws, and its
+ * cek_gemm_fp8_pert_workspace_size for the same M, N, K).
+ */
+int cek_gemv_fp8_pern_ws(const void* x, const void* w, const void* scale, void* y,
+                         int64_t M, int64_t N, int64_t K, int io_dtype, int fp8_fmt, int scale_dtype,
+                         void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * Several fp8-weight GEMVs that share one activation matrix, in one launch
  * (e.g. Q, K and V, or gate and up projections).  Host arrays of `count`
  * (1..8) device pointers / row counts: w[i] [N[i], K], scale[i] (per-channel
@@ -139,6 +148,17 @@ int cek_fused_add_rms_norm(void* hidden, void* residual, const void* weight,
 int cek_fused_add_rms_norm_quant_fp8(const void* hidden, void* residual, const void* weight,
                                      int64_t rows, int64_t H, float eps, int io_dtype,
                                      uint8_t* q, float* scale, void* stream);
+
+/*
+ * NEW: the two above with their outputs apart from their inputs: hidden and
+ * residual are only read, the sum goes to residual_out and, with q == NULL, the
+ * normed rows to hidden_out; else the codes and scales to q and scale
+ * (hidden_out unused).  residual_out may be residual and hidden_out may be
+ * hidden; otherwise outputs must not overlap inputs.  Same values bit for bit.
+ */
+int cek_add_rms_norm_out(const void* hidden, const void* residual, const void* weight, void* residual_out,
+                         void* hidden_out, int64_t rows, int64_t H, float eps, int io_dtype,
+                         uint8_t* q, float* scale, void* stream);
 
 /* NEW: per-token e4m3 quantisation of x [rows, H] (same formula as above). */
 int cek_per_token_quant_fp8(const void* x, int64_t rows, int64_t H, int io_dtype,
