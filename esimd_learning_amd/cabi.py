@@ -39,6 +39,7 @@ SIGNATURES = {
     "cek_gemm_fp8_a8w8_workspace_size": (_i64, [_i64, _i64, _i64]),
     "cek_gemm_fp8_a8w8_ws": (_i, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i, _p, _i64, _p]),
     "cek_gemm_fp8_a8w8_noalloc": (_i, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i, _p]),
+    "cek_gemm_fp8_a8w8_gelu_and_mul": (_i, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i, _p]),
     "cek_gelu_and_mul": (_i, [_p, _p, _i64, _i64, _i64, _i64, _i, _p]),
     "cek_gemv_fp8_gelu_and_mul": (_i, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i, _i, _i, _p]),
     "cek_add_rms_norm_gemv_fp8": (_i, [_p, _p, _p, _f, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i, _i, _i, _i,

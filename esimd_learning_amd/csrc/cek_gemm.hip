@@ -226,6 +226,55 @@ __device__ inline void store_tile(const f4 (&acc)[BM / WM / 16][BN / WN / 16], u
   }
 }
 
+// The GLU form's epilogue: a wave's first FN / 2 block columns are gate, the
+// others the up values of the same outputs (glu_row); both rounded to T as the
+// plain GEMM stores them, then gelu_tanh(gate) up, staged and written as in
+// store_tile, BN / 2 output columns per tile.  rs, cs: LDS copies of the scales.
+template <typename T, int BM, int BN, int WM, int WN, int NT>
+__device__ inline void store_tile_glu(const f4 (&acc)[BM / WM / 16][BN / WN / 16], uint8_t* smem, int wm, int wn,
+                                      int lane, int m0, int n0, int M, int d, const float* rs, const float* cs,
+                                      uint16_t* Y, int mlo, int nlo) {
+  constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 16, FN = TN / 16, BO = BN / 2;
+  constexpr int CPR = BO / 8, RS = BO * 2;
+  static_assert(CPR % 8 == 0, "chunk swizzle inside aligned groups of 8");
+  auto cpos = [](int r, int k) { return k ^ (2 * ((r >> 2) & 3)); };
+  const int r16 = lane & 15, g = lane >> 4;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    const f4 rv = *reinterpret_cast<const f4*>(rs + wm * TM + i * 16 + 4 * g);
+#pragma unroll
+    for (int j = 0; j < FN / 2; ++j) {
+      const int c = wn * (TN / 2) + j * 16 + r16;
+      const float cg = cs[wn * TN + j * 16 + r16], cu = cs[wn * TN + TN / 2 + j * 16 + r16];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int r = wm * TM + i * 16 + 4 * g + v;
+        const float gate = T::to_f32(T::from_f32(acc[i][j][v] * rv[v] * cg));
+        const float up = T::to_f32(T::from_f32(acc[i][j + FN / 2][v] * rv[v] * cu));
+        *reinterpret_cast<uint16_t*>(smem + r * RS + cpos(r, c >> 3) * 16 + (c & 7) * 2) =
+            T::from_f32(f32_round(gelu_tanh(gate) * up));
+      }
+    }
+  }
+  __syncthreads();
+  const bool vec = (d & 7) == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;
+  for (int q = threadIdx.x; q < BM * CPR; q += NT) {
+    const int r = q / CPR, k = q % CPR;
+    const int m = m0 + r, n = n0 + 8 * k;
+    if (m < mlo) continue;  // (the tile lies inside the matrix)
+    const uint8_t* src = smem + r * RS + cpos(r, k) * 16;
+    uint16_t* dst = Y + (size_t)m * d + n;
+    if (vec && n >= nlo) {
+      __builtin_nontemporal_store(*reinterpret_cast<const u4*>(src), reinterpret_cast<u4*>(dst));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (n + e >= nlo) dst[e] = reinterpret_cast<const uint16_t*>(src)[e];
+    }
+  }
+}
+
 template <typename T, int BM, int BN, int WM, int WN, int LAYOUT, int OCC>
 __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_a8w8_lds_kernel(
     const uint8_t* __restrict__ A, const float* __restrict__ sa,
@@ -377,15 +426,26 @@ __device__ inline __amdgpu_buffer_rsrc_t buf_rsrc(const void* p, uint32_t n) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)n, 0x00020000);
 }
 
+// GLU form: a tile's BN columns are BN / 2 gate rows of B and the BN / 2 up
+// rows d further; wave wn's TN columns hold its TN / 2 gate rows, then their up
+// rows, so that a lane's accumulators hold both factors of its outputs.  Row
+// of B (from the tile's first gate row) behind tile column r.
+template <int TN>
+__device__ inline uint32_t glu_row(int r, int d) {
+  return (uint32_t)((r % TN >= TN / 2 ? d : 0) + (r / TN) * (TN / 2) + r % (TN / 2));
+}
+
 // Direct-to-LDS loads of chunk ch (of NCH) of one K step (128 bytes of each
 // row) by loader w: its BL B loads, then its AL A loads, cut into NCH runs of
 // ceil((AL + BL) / NCH).  Load i of a kind moves rows 8 j .. 8 j + 7, j = w +
 // LW i, into 1 KB piece j of the slot; the lane's byte offset (ga / gb, one
 // VGPR) plus kb addresses chunk 0's row and i * LW * 8 * K (a uniform
 // SGPR offset, unsigned 32-bit like the whole offset) the row of load i.
-template <int AL, int BL, int LW, int NCH>
+// With GTN (> 0: the GLU form, columns per wave) the B rows of load i are
+// those of glu_row: their offset is computed per load (uniform, scalar).
+template <int AL, int BL, int LW, int NCH, int GTN = 0>
 __device__ __forceinline__ void a8w8_issue_chunk(int ch, uint8_t* sB, uint8_t* sA, int kb, int w, __amdgpu_buffer_rsrc_t rA,
-                                                 __amdgpu_buffer_rsrc_t rB, int K, uint32_t ga, uint32_t gb) {
+                                                 __amdgpu_buffer_rsrc_t rB, int K, uint32_t ga, uint32_t gb, int d = 0) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int T = AL + BL, CS = (T + NCH - 1) / NCH;
 #pragma unroll
@@ -393,7 +453,10 @@ __device__ __forceinline__ void a8w8_issue_chunk(int ch, uint8_t* sB, uint8_t* s
     if (i < ch * CS || i >= ch * CS + CS) continue;
     if (i < BL)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, (lds_ptr_t)(sB + (w + LW * i) * 1024), 16, gb + (uint32_t)kb,
-                                               (int)((uint32_t)(i * LW * 8) * (uint32_t)K), 0, 0);
+                                               (int)((GTN > 0 ? glu_row<(GTN > 0 ? GTN : 2)>(8 * (w + LW * i), d)
+                                                              : (uint32_t)(i * LW * 8)) *
+                                                     (uint32_t)K),
+                                               0, 0);
     else
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, (lds_ptr_t)(sA + (w + LW * (i - BL)) * 1024), 16, ga + (uint32_t)kb,
                                                (int)((uint32_t)((i - BL) * LW * 8) * (uint32_t)K), 0, 0);
@@ -408,9 +471,9 @@ __device__ __forceinline__ void a8w8_issue_chunk(int ch, uint8_t* sB, uint8_t* s
 // the compiler drain every load before using them.  Waves 0 .. BM / 64 - 1
 // load row scales, the rest column scales.  Each wave issues at most one
 // load, before any of its operand loads.
-template <int BM, int BN, int NW>
+template <int BM, int BN, int NW, int GTN = 0>
 __device__ __forceinline__ void stage_tile_scales(float* sc, const float* sa, const float* sb, int M, int N, int m0,
-                                                  int n0, int wave, int lane) {
+                                                  int n0, int wave, int lane, int d = 0) {
   static_assert(BM % 64 == 0, "a wave's scales come from one of sa, sb");
   static_assert(BM + BN <= 64 * NW, "one scale per thread");
   if (64 * wave < BM + BN) {
@@ -419,7 +482,11 @@ __device__ __forceinline__ void stage_tile_scales(float* sc, const float* sa, co
 #if defined(__HIP_DEVICE_COMPILE__)
     __builtin_amdgcn_raw_ptr_buffer_load_lds(buf_rsrc(rows ? sa : sb, (uint32_t)(rows ? M : N) * 4u),
                                              (lds_ptr_t)(sc + 64 * wave), 4,
-                                             (uint32_t)(rows ? m0 + t : n0 + t - BM) * 4u, 0, 0, 0);
+                                             (rows ? (uint32_t)(m0 + t)
+                                                   : (uint32_t)n0 + (GTN > 0 ? glu_row<(GTN > 0 ? GTN : 2)>(t - BM, d)
+                                                                             : (uint32_t)(t - BM))) *
+                                                 4u,
+                                             0, 0, 0);
 #endif
   }
 }
@@ -431,13 +498,13 @@ __device__ __forceinline__ void stage_tile_scales(float* sc, const float* sa, co
 // kt + RING - 1 (whose chunk 0 went out after the previous step's barrier)
 // go out in groups 0 .. NCH - 2.  Steps 0 .. RING - 1 are loaded whole by the
 // prologue, hence kt >= 1 for the chunks.
-template <int BM, int BN, int WM, int WN, int LW, int RING, int NCH>
+template <int BM, int BN, int WM, int WN, int LW, int RING, int NCH, bool GLU = false>
 __device__ __forceinline__ void a8w8_pipe_step(int kt, int KT, int c, int cn, uint8_t* sAr, uint8_t* sBr, bool loader, int wave,
                                                int wm, int wn, int r16, int p0, int p1, __amdgpu_buffer_rsrc_t rA,
                                                __amdgpu_buffer_rsrc_t rB, int K, uint32_t ga, uint32_t gb,
                                                f4 (&acc)[PipeCfg<BM, BN, WM, WN>::FM][PipeCfg<BM, BN, WM, WN>::FN],
                                                i8 (&a)[2], const i8 (&bc)[PipeCfg<BM, BN, WM, WN>::FN],
-                                               i8 (&bn)[PipeCfg<BM, BN, WM, WN>::FN]) {
+                                               i8 (&bn)[PipeCfg<BM, BN, WM, WN>::FN], int d = 0) {
   using C = PipeCfg<BM, BN, WM, WN>;
   using L = LoadSplit<BM, BN, LW>;
   constexpr int BK = C::BK, TM = C::TM, TN = C::TN, FM = C::FM, FN = C::FN;
@@ -449,14 +516,14 @@ __device__ __forceinline__ void a8w8_pipe_step(int kt, int KT, int c, int cn, ui
       a[(i + 1) & 1] = lds_frag(sA + (i + 1) * 16 * BK, p0, p1);
       if (i < NCH - 1 && loader && kt >= 1 && kt + RING - 1 < KT) {
         const int cl = c == 0 ? RING - 1 : c - 1;  // slot of step kt + RING - 1
-        a8w8_issue_chunk<L::AL, L::BL, LW, NCH>(i + 1, sBr + cl * C::BSLOT, sAr + cl * C::ASLOT, (kt + RING - 1) * BK,
-                                                wave, rA, rB, K, ga, gb);
+        a8w8_issue_chunk<L::AL, L::BL, LW, NCH, GLU ? TN : 0>(i + 1, sBr + cl * C::BSLOT, sAr + cl * C::ASLOT,
+                                                              (kt + RING - 1) * BK, wave, rA, rB, K, ga, gb, d);
       }
     } else if (kt + 1 < KT) {
       barrier_upto<RING - 2, L::AL + L::BL>(KT - 2 - kt);
       if (loader && kt + RING < KT)
-        a8w8_issue_chunk<L::AL, L::BL, LW, NCH>(0, sBr + c * C::BSLOT, sAr + c * C::ASLOT, (kt + RING) * BK, wave, rA, rB,
-                                                K, ga, gb);
+        a8w8_issue_chunk<L::AL, L::BL, LW, NCH, GLU ? TN : 0>(0, sBr + c * C::BSLOT, sAr + c * C::ASLOT,
+                                                              (kt + RING) * BK, wave, rA, rB, K, ga, gb, d);
       const uint8_t* nA = sAr + cn * C::ASLOT + (wm * TM + r16) * BK;
       const uint8_t* nB = sBr + cn * C::BSLOT + (wn * TN + r16) * BK;
 #pragma unroll
@@ -477,7 +544,8 @@ __device__ __forceinline__ void a8w8_pipe_step(int kt, int KT, int c, int cn, ui
 // adds the parts in order, scales and converts.
 // RING: slots of the A and B rings (loads run RING - 1 steps ahead).  NCH:
 // chunks a loader's loads of a step are issued in (a8w8_pipe_step).
-template <typename T, int BM, int BN, int WM, int WN, int OCC, int LW, int SPLIT = 1, int RING = 2, int NCH = 1>
+template <typename T, int BM, int BN, int WM, int WN, int OCC, int LW, int SPLIT = 1, int RING = 2, int NCH = 1,
+          bool GLU = false>
 __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_a8w8_pipe_kernel(
     const uint8_t* __restrict__ A, const float* __restrict__ sa,
     const uint8_t* __restrict__ B, const float* __restrict__ sb,
@@ -497,7 +565,11 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_a8w8_pipe_kernel(
   uint8_t* sBr = smem + RING * C::ASLOT;
   float* sc = reinterpret_cast<float*>(smem + SMEM);
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = GLU ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : (int)threadIdx.x >> 6;
+  constexpr int BO = GLU ? BN / 2 : BN;  // output columns of a tile (GLU: N is d, B and sb have 2 d rows)
+  static_assert(!GLU || (SPLIT == 1 && FN % 2 == 0 && (TN / 2) % 8 == 0), "GLU tiles");
+  const int NB = GLU ? 2 * N : N;
   const int wm = wave / WN, wn = wave % WN;
   const bool loader = wave < LW;
   const int part = SPLIT > 1 ? (int)blockIdx.x % SPLIT : 0;
@@ -507,11 +579,11 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_a8w8_pipe_kernel(
   // N >= BN): every row it loads exists, so no load needs a clamp, and it
   // stores only from its own first row (column) mlo (nlo) on -- the rows
   // before are the previous tile's, which computes the same values.
-  const int mlo = tm * BM, nlo = tn * BN;
-  const int m0 = min(mlo, M - BM), n0 = min(nlo, N - BN);
+  const int mlo = tm * BM, nlo = tn * BO;
+  const int m0 = min(mlo, M - BM), n0 = min(nlo, N - BO);
   const __amdgpu_buffer_rsrc_t rA = buf_rsrc(A, (uint32_t)((size_t)M * K));
-  const __amdgpu_buffer_rsrc_t rB = buf_rsrc(B, (uint32_t)((size_t)N * K));
-  stage_tile_scales<BM, BN, NW>(sc, sa, sb, M, N, m0, n0, wave, lane);
+  const __amdgpu_buffer_rsrc_t rB = buf_rsrc(B, (uint32_t)((size_t)NB * K));
+  stage_tile_scales<BM, BN, NW, GLU ? TN : 0>(sc, sa, sb, M, NB, m0, n0, wave, lane, N);
 
   // loader chunk j = wave + LW i: lane l fills row 8 j + (l >> 3), position
   // l & 7, i.e. logical chunk (l & 7) ^ s(row) (s(row) = row & 7 = (l >> 3)
@@ -520,7 +592,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_a8w8_pipe_kernel(
   const uint32_t cofs = (uint32_t)(((lane & 7) ^ swz<1>(lane >> 3)) * 16);
   const uint32_t kpart = (uint32_t)(part * (K / SPLIT));  // first K value of this part
   const uint32_t ga = (uint32_t)(m0 + wave * 8 + (lane >> 3)) * (uint32_t)K + cofs + kpart;
-  const uint32_t gb = (uint32_t)(n0 + wave * 8 + (lane >> 3)) * (uint32_t)K + cofs + kpart;
+  const uint32_t gb = (uint32_t)(n0 + (GLU ? 0 : wave * 8) + (lane >> 3)) * (uint32_t)K + cofs + kpart;
   const int r16 = lane & 15, g = lane >> 4;
   const int p0 = g ^ swz<1>(r16), p1 = (g + 4) ^ swz<1>(r16);
 
@@ -538,7 +610,8 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_a8w8_pipe_kernel(
 #pragma unroll
     for (int s = 0; s < RING; ++s)
       if (s == 0 || s < KT) {
-        a8w8_issue_chunk<AL, BL, LW, 1>(0, sBr + s * C::BSLOT, sAr + s * C::ASLOT, s * BK, wave, rA, rB, K, ga, gb);
+        a8w8_issue_chunk<AL, BL, LW, 1, GLU ? TN : 0>(0, sBr + s * C::BSLOT, sAr + s * C::ASLOT, s * BK, wave, rA, rB, K,
+                                                      ga, gb, N);
       }
   }
   barrier_upto<RING - 1, AL + BL>(KT - 1);
@@ -554,15 +627,15 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_a8w8_pipe_kernel(
   auto nxt = [](int v) { return v + 1 == RING ? 0 : v + 1; };
   for (; kt + 1 < KT; kt += 2) {
     const int c1 = RING == 2 ? 1 : nxt(c), c2 = RING == 2 ? 0 : nxt(c1);
-    a8w8_pipe_step<BM, BN, WM, WN, LW, RING, NCH>(kt, KT, RING == 2 ? 0 : c, c1, sAr, sBr, loader, wave, wm, wn, r16,
-                                                  p0, p1, rA, rB, K, ga, gb, acc, a, b0, b1);
-    a8w8_pipe_step<BM, BN, WM, WN, LW, RING, NCH>(kt + 1, KT, c1, c2, sAr, sBr, loader, wave, wm, wn, r16, p0, p1, rA,
-                                                  rB, K, ga, gb, acc, a, b1, b0);
+    a8w8_pipe_step<BM, BN, WM, WN, LW, RING, NCH, GLU>(kt, KT, RING == 2 ? 0 : c, c1, sAr, sBr, loader, wave, wm, wn, r16,
+                                                  p0, p1, rA, rB, K, ga, gb, acc, a, b0, b1, N);
+    a8w8_pipe_step<BM, BN, WM, WN, LW, RING, NCH, GLU>(kt + 1, KT, c1, c2, sAr, sBr, loader, wave, wm, wn, r16, p0, p1, rA,
+                                                  rB, K, ga, gb, acc, a, b1, b0, N);
     c = c2;
   }
   if (kt < KT)
-    a8w8_pipe_step<BM, BN, WM, WN, LW, RING, NCH>(kt, KT, RING == 2 ? 0 : c, RING == 2 ? 1 : nxt(c), sAr, sBr, loader,
-                                                  wave, wm, wn, r16, p0, p1, rA, rB, K, ga, gb, acc, a, b0, b1);
+    a8w8_pipe_step<BM, BN, WM, WN, LW, RING, NCH, GLU>(kt, KT, RING == 2 ? 0 : c, RING == 2 ? 1 : nxt(c), sAr, sBr, loader,
+                                                  wave, wm, wn, r16, p0, p1, rA, rB, K, ga, gb, acc, a, b0, b1, N);
   // every wave's loads (a non-loader's scale load included) are complete
   // here: step KT - 2's barrier (the last) waited for vmcnt(0), and with
   // KT == 1 the prologue's did
@@ -584,6 +657,8 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_a8w8_pipe_kernel(
           if (m >= mlo && n >= nlo) Pp[(size_t)m * N + n] = acc[i][j][v];
         }
       }
+  } else if constexpr (GLU) {
+    store_tile_glu<T, BM, BN, WM, WN, 64 * NW>(acc, smem, wm, wn, lane, m0, n0, M, N, sc, sc + BM, Y, mlo, nlo);
   } else {
     store_tile<T, BM, BN, WM, WN, 64 * NW, true>(acc, smem, wm, wn, lane, m0, n0, M, N, sc, sc + BM, 1.f, Y, mlo, nlo);
   }
@@ -1809,7 +1884,8 @@ static double a8w8_round_us(const A8w8Opt& o, int64_t M, int64_t N, int64_t K, i
 // the measured fastest on all nine, with cache-resident operands too; on
 // twelve other shapes (M = 128 .. 3000, K = 2048 .. 14336, ragged N) within
 // 6% of the fastest of thirteen measured forms.
-static A8w8Plan plan_a8w8_rounds(int64_t M, int64_t N, int64_t K, bool allow_split) {
+// t_us, if given, takes the model's time.
+static A8w8Plan plan_a8w8_rounds(int64_t M, int64_t N, int64_t K, bool allow_split, double* t_us = nullptr) {
   A8w8Plan best{1, 1};
   double tbest = -1.0;
   for (int c = 0; c < kA8w8Cfgs; ++c) {
@@ -1824,6 +1900,7 @@ static A8w8Plan plan_a8w8_rounds(int64_t M, int64_t N, int64_t K, bool allow_spl
       }
     }
   }
+  if (t_us) *t_us = tbest;
   return best;
 }
 
@@ -1888,10 +1965,70 @@ static int64_t a8w8_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 static int launch_a8w8(const uint8_t* a, const float* sa, const uint8_t* b, const float* sb, void* y, int64_t M,
                        int64_t N, int64_t K, int out_dtype, float* ws, int64_t ws_bytes, hipStream_t st);
 
+// a8w8 gate/up product with gelu_and_mul in the epilogue (prefill):
+// y[m, i] = gelu_tanh(g) u, g and u the rounded outputs of B rows i and d + i.
+// Saves the [M, 2d] product's way to memory and back (6 M d bytes of the two
+// launches' traffic) and a launch.  Tiles whose waves can hold gate and up of
+// the same outputs (an even count of block columns): 128 x 128 (two per CU), 256
+// x 256, 128 x 256 and 256 x 128, by the round model.  CEK_ERR_UNSUPPORTED where
+// the model has the separate launches faster (64-row tiles, 256 x 192 or split K
+// fit the shape better by more than the second pass costs), below one tile, above
+// 4 GB and for K % 128.  Bound by the matrix cores from ~1000 rows on.  GEMM +
+// gelu_and_mul -> here (us, MI355X, weights from HBM, M x d x K): 2048 x 14336 x
+// 4096 228.7 -> 197.0 (2.44 PFLOP/s), 2048 x 24576 x 5120 470 -> 390, 4096 x
+// 14336 x 4096 425 -> 362, 1024 x 24576 x 3072 159 -> 129, 256 x 14336 x 4096
+// 45.1 -> 38.4, 333 x 6912 x 2560 30.1 -> 26.9, 1000 x 3072 x 1024 18.4 -> 11.9.
+static int launch_a8w8_glu(const uint8_t* a, const float* sa, const uint8_t* b, const float* sb, void* y, int64_t M,
+                           int64_t d, int64_t K, int out_dtype, hipStream_t st) {
+  if (M < 0 || d < 0 || K <= 0 || K % 16 != 0) return CEK_ERR_INVALID;
+  if (M > 65535 * 64 || d > INT32_MAX / 2 || K > INT32_MAX) return CEK_ERR_INVALID;
+  if (M == 0 || d == 0) return CEK_OK;
+  if (!a || !sa || !b || !sb || !y || !aligned(a, 16) || !aligned(b, 16)) return CEK_ERR_INVALID;
+  if (out_dtype != CEK_F16 && out_dtype != CEK_BF16) return CEK_ERR_INVALID;
+  if (M < 128 || d < 128 || K % 128 != 0 || !a8w8_off32(M, 2 * d, K)) return CEK_ERR_UNSUPPORTED;
+  int cfg = -1;
+  double t_glu = 0, t_gemm = 0;
+  for (int c : {1, 3, 5, 6}) {
+    const A8w8Opt& o = kA8w8Opts[c];
+    if (M < o.bm || d < o.bn / 2) continue;
+    const double t = a8w8_round_us(o, M, (d + o.bn / 2 - 1) / (o.bn / 2) * o.bn, K, 1);
+    if (cfg < 0 || t < t_glu) {
+      t_glu = t;
+      cfg = c;
+    }
+  }
+  plan_a8w8_rounds(M, 2 * d, K, true, &t_gemm);
+  if (t_glu > t_gemm + (double)M * (double)d * 6.0 / 5.0e6 + 1.5) return CEK_ERR_UNSUPPORTED;
+  uint16_t* yp = static_cast<uint16_t*>(y);
+#define CEK_GLU8(TY, BM, BN, WM, WN, OCC, RING, NCH)                                                          \
+  do {                                                                                                        \
+    const int tm = (int)((M + BM - 1) / BM), tn = (int)((d + BN / 2 - 1) / (BN / 2));                         \
+    gemm_a8w8_pipe_kernel<TY, BM, BN, WM, WN, OCC, 4, 1, RING, NCH, true>                                     \
+        <<<dim3((unsigned)(tm * tn)), 64 * WM * WN, 0, st>>>(a, sa, b, sb, yp, nullptr, (int)M, (int)d, (int)K, tm, tn); \
+  } while (0)
+#define CEK_GLU8_ALL(TY)                                     \
+  do {                                                       \
+    if (cfg == 3) CEK_GLU8(TY, 256, 256, 2, 4, 1, 2, 3);     \
+    else if (cfg == 5) CEK_GLU8(TY, 128, 256, 2, 4, 1, 3, 3); \
+    else if (cfg == 6) CEK_GLU8(TY, 256, 128, 2, 4, 1, 3, 3); \
+    else CEK_GLU8(TY, 128, 128, 2, 2, 2, 2, 1);              \
+  } while (0)
+  if (out_dtype == CEK_F16) CEK_GLU8_ALL(F16);
+  else CEK_GLU8_ALL(BF16);
+#undef CEK_GLU8
+#undef CEK_GLU8_ALL
+  return check_launch();
+}
+
 }  // namespace cek
 
 extern "C" int64_t cek_gemm_fp8_a8w8_workspace_size(int64_t M, int64_t N, int64_t K) {
   return cek::a8w8_workspace_bytes(M, N, K);
+}
+
+extern "C" int cek_gemm_fp8_a8w8_gelu_and_mul(const uint8_t* a, const float* sa, const uint8_t* b, const float* sb, void* y,
+                                              int64_t M, int64_t d, int64_t K, int out_dtype, void* stream) {
+  return cek::launch_a8w8_glu(a, sa, b, sb, y, M, d, K, out_dtype, (hipStream_t)stream);
 }
 
 extern "C" int cek_gemm_fp8_a8w8_ws(const uint8_t* a, const float* sa, const uint8_t* b, const float* sb, void* y,

@@ -370,9 +370,8 @@ void esimd_qk_norm_rope(at::Tensor q, at::Tensor k, at::Tensor q_weight, at::Ten
 // Whether the norm may write residual_out while it reads hidden and residual:
 // it is residual, or shares no memory with either.
 static bool norm_writes_out(const at::Tensor& residual_out, const at::Tensor& hidden, const at::Tensor& residual) {
-  const auto with_r = at::get_overlap_status(residual_out, residual);
-  return (with_r == at::MemOverlapStatus::Full || with_r == at::MemOverlapStatus::No) &&
-         at::get_overlap_status(residual_out, hidden) == at::MemOverlapStatus::No;
+  return !overlaps(residual_out, hidden) &&
+         (residual_out.data_ptr() == residual.data_ptr() || !overlaps(residual_out, residual));
 }
 
 static void check_norm_gemv_common(const at::Tensor& h, const at::Tensor& r, const at::Tensor& nw,
@@ -459,7 +458,8 @@ void esimd_fused_add_rms_norm_quant_gemv_fp8(at::Tensor hidden_states, at::Tenso
     return;
   }
   // two launches: norm + quant, then the a8w8 product
-  const bool direct = norm_writes_out(residual_out, hidden_states, residual);
+  const bool direct = norm_writes_out(residual_out, hidden_states, residual) && !overlaps(out_q, residual) &&
+                      !overlaps(out_scale, residual);
   const at::Tensor h = direct ? hidden_states : hidden_states.clone();
   const at::Tensor r = direct ? residual : residual.clone();
   check_rc(cek_add_rms_norm_out(h.data_ptr(), r.data_ptr(), weight.data_ptr(), residual_out.data_ptr(), nullptr, M, K,
@@ -478,8 +478,12 @@ void esimd_fused_add_rms_norm_quant_gemv_fp8(at::Tensor hidden_states, at::Tenso
     check_rc(cek_gemm_fp8_a8w8_ws(q, qs, bp, sb, output.data_ptr(), M, N, K, io, wp, need, st), op);
     return;
   }
-  rc = M <= 16 ? cek_gemv_fp8_gelu_and_mul(q, qs, bp, sb, output.data_ptr(), M, N / 2, K, io, CEK_E4M3, CEK_F32, st)
-               : CEK_ERR_UNSUPPORTED;
+  // as esimd_gemm_fp8_a8w8_gelu_and_mul
+  rc = CEK_ERR_UNSUPPORTED;
+  if (M <= 16)
+    rc = cek_gemv_fp8_gelu_and_mul(q, qs, bp, sb, output.data_ptr(), M, N / 2, K, io, CEK_E4M3, CEK_F32, st);
+  else if (!overlaps(output, out_q) && !overlaps(output, b) && !overlaps(output, out_scale) && !overlaps(output, b_scale))
+    rc = cek_gemm_fp8_a8w8_gelu_and_mul(q, qs, bp, sb, output.data_ptr(), M, N / 2, K, io, st);
   if (rc == CEK_ERR_UNSUPPORTED) {
     at::Tensor gu = at::empty({M, N}, output.options());
     check_rc(cek_gemm_fp8_a8w8_ws(q, qs, bp, sb, gu.data_ptr(), M, N, K, io, wp, need, st), op);

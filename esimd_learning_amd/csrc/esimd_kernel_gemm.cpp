@@ -95,8 +95,8 @@ at::Tensor esimd_gemm_fp8_a8w8(at::Tensor a, at::Tensor a_scale, at::Tensor b, a
 
 // a8w8 gate/up GEMM over a merged [2d, K] e4m3 weight with gelu_and_mul fused
 // into the epilogue: output[m, i] = gelu_tanh(g[m, i]) * u[m, i], g and u the
-// rounded outputs of weight rows i and d + i.  Decode batches (M <= 16) take
-// the fused kernel; other shapes run esimd_gemm_fp8_a8w8's kernels into a
+// rounded outputs of weight rows i and d + i.  Decode batches (M <= 16) and
+// prefill (M >= 128) take the fused kernels; other shapes run esimd_gemm_fp8_a8w8's kernels into a
 // workspace and then gelu_and_mul (the same values).
 void esimd_gemm_fp8_a8w8_gelu_and_mul(at::Tensor a, at::Tensor a_scale, at::Tensor b, at::Tensor b_scale,
                                       at::Tensor output) {
@@ -126,8 +126,12 @@ void esimd_gemm_fp8_a8w8_gelu_and_mul(at::Tensor a, at::Tensor a_scale, at::Tens
   const auto* sa = static_cast<const float*>(a_scale.data_ptr());
   const auto* bp = static_cast<const uint8_t*>(b.data_ptr());
   const auto* sb = static_cast<const float*>(b_scale.data_ptr());
-  int rc = M <= 16 ? cek_gemv_fp8_gelu_and_mul(ap, sa, bp, sb, output.data_ptr(), M, d, K, io, CEK_E4M3, CEK_F32, st)
-                   : CEK_ERR_UNSUPPORTED;
+  // the prefill kernel writes outputs while it reads operands: separate memory only
+  int rc = CEK_ERR_UNSUPPORTED;
+  if (M <= 16)
+    rc = cek_gemv_fp8_gelu_and_mul(ap, sa, bp, sb, output.data_ptr(), M, d, K, io, CEK_E4M3, CEK_F32, st);
+  else if (!overlaps(output, a) && !overlaps(output, b) && !overlaps(output, a_scale) && !overlaps(output, b_scale))
+    rc = cek_gemm_fp8_a8w8_gelu_and_mul(ap, sa, bp, sb, output.data_ptr(), M, d, K, io, st);
   if (rc == CEK_ERR_UNSUPPORTED && M > 0 && d > 0) {
     at::Tensor gu = at::empty({M, 2 * d}, output.options());
     at::Tensor ws;

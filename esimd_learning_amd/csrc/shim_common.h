@@ -47,6 +47,13 @@ inline void check_rc(int rc, const char* op) {
               rc == CEK_ERR_HIP ? cek_last_hip_error() : "");
 }
 
+// Whether two contiguous tensors share bytes, by address (also when their
+// storages are different objects over one allocation).
+inline bool overlaps(const at::Tensor& a, const at::Tensor& b) {
+  const auto pa = reinterpret_cast<uintptr_t>(a.data_ptr()), pb = reinterpret_cast<uintptr_t>(b.data_ptr());
+  return a.nbytes() > 0 && b.nbytes() > 0 && pa < pb + b.nbytes() && pb < pa + a.nbytes();
+}
+
 // The split-K workspace of `need` bytes (a *_workspace_size; 0: none) on like's
 // device, from the caching allocator (no kernel runs to allocate or clear it).
 inline int64_t split_workspace(at::Tensor& ws, int64_t need, const at::Tensor& like) {

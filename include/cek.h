@@ -209,6 +209,18 @@ int cek_gemm_fp8_a8w8_noalloc(const uint8_t* a, const float* sa, const uint8_t* 
                               void* y, int64_t M, int64_t N, int64_t K, int out_dtype, void* stream);
 
 /*
+ * NEW: a8w8 gate/up GEMM with gelu_and_mul in its epilogue (no counterpart in
+ * the reference: cek_gemm_fp8_a8w8 over a merged [2d, K] weight followed by
+ * cek_gelu_and_mul, in one launch):
+ *   y[m, i] = Out(gelu_tanh(g) * u),  g, u = Out(a8w8 sums of B rows i, d + i)
+ * y [M, d] shares no memory with the operands.  CEK_ERR_UNSUPPORTED (nothing
+ * launched) below 128 rows or columns, for K % 128 != 0, matrices above 4 GB,
+ * and where the two launches are faster: run those instead.
+ */
+int cek_gemm_fp8_a8w8_gelu_and_mul(const uint8_t* a, const float* sa, const uint8_t* b, const float* sb, void* y,
+                                   int64_t M, int64_t d, int64_t K, int out_dtype, void* stream);
+
+/*
  * NEW: out[t, i] = gelu_tanh(x[t, i]) * x[t, d + i], fp32 math.
  * x rows have stride x_stride elements (>= 2d), out rows out_stride (>= d).
  */
