@@ -43,6 +43,21 @@ def test_gelu_and_mul_many_rows(ops, dev, d):
     assert_close_fp(out.cpu(), torch.from_numpy(oact.gelu_and_mul(x.float().numpy())), f"gelu T={T} d={d}")
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_gelu_every_gate(ops, dev, dtype):
+    """Every finite gate of the type, bit for bit the fp32 formula's value
+    0.5 u (1 + tanh(k0 (u + k1 u u u))) taken one rounded operation at a time."""
+    _say(f"gelu every gate {dtype}")
+    g = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dtype)
+    g = g[torch.isfinite(g.float())].to(dev)
+    out = torch.empty(1, g.numel(), dtype=dtype, device=dev)
+    ops.esimd_gelu_and_mul(out, torch.cat([g, torch.ones_like(g)])[None])
+    u = g.float()
+    k0, k1 = (torch.tensor(v, dtype=torch.float32, device=dev) for v in (0.7978845608028654, 0.044715))
+    want = ((0.5 * u) * (1.0 + torch.tanh(k0 * (u + ((k1 * u) * u) * u)))).to(dtype)
+    assert torch.equal(out[0].view(torch.int16), want.view(torch.int16))
+
+
 def test_gelu_and_mul_strided_rows(ops, dev):
     # input rows are a view into a wider buffer (e.g. a fused gate/up output)
     T, d = 4, 512
