@@ -26,6 +26,7 @@
 // fill and epilogue); a deeper weight ring beside a shallow activation ring
 // (within 2%); run-time loads per stage (M = 48 12.4 -> 17.7 us: the waits
 // become a branch tree).
+#include <algorithm>
 #include <type_traits>
 
 #include "cek_segs.h"
@@ -255,22 +256,31 @@ void stream_kernel(const uint8_t* __restrict__ x, GemvSegs sg, int skind, int M,
 constexpr int kStreamRows[] = {8, 12, 16, 24, 32, 40, 48, 56, 64};
 
 // Weight rows per workgroup: the count with the least work for the busiest
-// CU, whose workgroups each cost their weight rows and, at about a third of
-// a weight row each (90 against 30 bytes per ns and CU measured), the
-// activation rows; a CU that holds one workgroup at a time also fills and
-// drains the rings between two of them (about 45 KB worth).  Measured on
-// MI355X, us: M = 4, K = 10240, N = 2560 8 / 12 / 16 rows 10.9 / 8.5 / 9.0; M =
-// 16, K = 4096, N = 14336 32 / 56 rows 15.0 / 13.6; M = 8, K = 2560, N = 20480 40
-// / 48 rows 12.4 / 12.9; M = 5, K = 1024, N = 32768 32 / 48 / 64 rows 9.9 / 9.7 /
-// 11.0; M = 48, K = 4096, N = 6144 24 / 32 rows 12.3 / 12.9.
+// CU.  Its workgroups each cost their weight rows and the activation rows (at
+// 0.3-0.4 of a weight row each: 90 against 30 bytes per ns and CU measured),
+// and every one after the first something by itself: 0.3 us where a CU holds two
+// at a time, and where it holds one the filling and draining of the rings
+// between two of them (2.7 us, or with e4m3 activations as long as the weight
+// rows take if that is less; 1.5 us above 16 rows).  Without the first of these,
+// up to 16 rows took workgroups of 8-16 weight rows for wide matrices (us,
+// before -> now: M = 3, K = 5376, N = 26240 47.5 -> 27.7; M = 5, K = 1024, N =
+// 28672 12.4 -> 9.1; e4m3 activations, M = 5, K = 1024, N = 26240 18.2 -> 9.9).  Over
+// 2800 shapes of 3-16 rows the pick is 1% (geometric mean) above the fastest
+// count.  Measured on MI355X, us: M = 4, K = 10240, N = 2560 8 / 12 / 16 rows
+// 10.9 / 8.5 / 9.0; M = 16, K = 4096, N = 14336 32 / 56 rows 15.0 / 13.6; M = 8, K
+// = 2560, N = 20480 40 / 48 rows 12.4 / 12.9; M = 5, K = 1024, N = 32768 32 / 48 /
+// 64 rows 9.9 / 9.7 / 11.0; M = 48, K = 4096, N = 6144 24 / 32 rows 12.3 / 12.9.
 static int stream_rows(int M, int64_t N, int K, bool xf8, int max_rows) {
   int best = 8;
   int64_t cost = INT64_MAX;
+  const int64_t act = (M > 16 ? 3 : 4) * (xf8 ? (M + 1) / 2 : M);
   for (int r : kStreamRows) {
     if (r > max_rows) break;
     const int64_t per_cu = ((N + r - 1) / r + kCUs - 1) / kCUs;
     const bool pair = M <= 16 && r <= (xf8 ? 24 : 48);  // two workgroups per CU
-    const int64_t c = per_cu * (10 * r + 3 * (xf8 ? (M + 1) / 2 : M)) * K + (pair ? 0 : (per_cu - 1) * 450000);
+    int64_t next = pair ? 100000 : (M > 16 ? 450000 : 800000);
+    if (!pair && xf8 && M <= 16) next = std::min(next, (int64_t)8 * r * K);
+    const int64_t c = per_cu * (10 * r + act) * K + (per_cu - 1) * next;
     if (c <= cost) {
       cost = c;
       best = r;

@@ -73,6 +73,39 @@ def test_stream_a8w8(ops, dev, M, K, N):
            f"M={M} K={K} N={N}")
 
 
+# Columns at which a workgroup has 8, 12, 16, 24, 32, 40, 48, 56 and 64 weight rows
+FORM_N = [1001, 2500, 3500, 5000, 6201, 8201, 11000, 12700, 16001]
+
+
+@pytest.mark.parametrize("act,out,fmt", [("fp16", torch.float16, torch.float8_e4m3fn),
+                                         ("bf16", torch.bfloat16, torch.float8_e5m2),
+                                         ("e4m3", torch.float16, torch.float8_e4m3fn),
+                                         ("e4m3", torch.bfloat16, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("M", [3, 6, 13, 20, 30, 40, 60])
+def test_stream_every_form(ops, dev, M, act, out, fmt):
+    """Every activation block (4 .. 64 rows) with every count of weight rows, K of a
+    whole stage and a part."""
+    K = 320
+    Wall, sall = synthetic.weight_fp8(max(FORM_N), K, seed=31, fmt=fmt)
+    x = synthetic.activations(M, K, seed=M, dtype=torch.float16 if act == "e4m3" else out)
+    if act == "e4m3":
+        x, sa = synthetic.quantize_rows(x.float())
+    for N in FORM_N:
+        print(f"stream form M={M} N={N} {act} {out} {fmt}", flush=True)
+        W8, s = Wall[:N], sall[:N]
+        y = torch.full((M, N), float("nan"), dtype=out, device=dev)
+        if act == "e4m3":
+            ops.esimd_gemm_fp8_a8w8(x.to(dev), sa.to(dev), W8.to(dev), s.to(dev), y)
+            _check(y, x.float().double() * sa.double()[:, None], W8.float().double(), s.double(), K + 2, f"N={N}")
+        elif M <= 16:
+            ops.esimd_gemv_fp8_pern(x.to(dev), W8.to(dev), s.to(dev), y, N, K)
+            _check(y, x.double(), W8.float().double(), s.double(), K, f"N={N}")
+        else:
+            s = s[:1].contiguous()
+            ops.esimd_gemm_fp8_pert(x.to(dev), W8.to(dev), s.to(dev), y)
+            _check(y, x.double(), W8.float().double(), s.double(), K, f"N={N}")
+
+
 @pytest.mark.parametrize("M,K,Ns", [(4, 2560, (4096, 512, 512)), (8, 2112, (9000, 1000, 8200)),
                                     (16, 4096, (14336, 4096, 9000)), (3, 6144, (1000, 3000))])
 def test_stream_fused_equals_single(ops, dev, M, K, Ns):
