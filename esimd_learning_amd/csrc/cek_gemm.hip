@@ -1648,12 +1648,17 @@ int launch_w8a16(const void* x, const void* w, const void* scale, int skind, voi
 #undef CEK_TINYN
     return check_launch();
   }
-  // M <= 64: the weight-streaming kernel, but for very wide matrices of short
-  // K, whose many workgroups each read the activations again (M = 64, K =
-  // 1024, N = 49152: tiles 20.6 us, streaming 23.1; K = 2048 34.3 / 35.2).  M =
-  // 48, K = 4096, N = 6144 47.7 -> 12.5 us; M = 64, K = 14336, N = 4096 157 -> 34;
-  // M = 32, K = 4096, N = 14336 (staged GEMV before) 36.7 -> 15.2.
-  if (M <= kStreamM && (N <= 32768 || K >= 4096) && aligned(x, 16) && aligned(w, 16) && N * K <= ((int64_t)1 << 40)) {
+  // M <= 64: the weight-streaming kernel, but for wide matrices of short K,
+  // whose workgroups each read the activations again and fill and drain their
+  // rings for a few stages: above 32768 rows below K = 4096 (M = 64, K = 1024, N =
+  // 49152: tiles 20.6 us, streaming 23.1; K = 2048 34.3 / 35.2), and above 16384
+  // (two workgroups or more per CU) up to K = 128 + 7 M (us, tiles / streaming, N
+  // = 24576: M = 17, K = 128 5.6 / 6.1, K = 256 7.2 / 6.9; M = 64, K = 448 10.1 /
+  // 10.7, K = 576 11.7 / 11.8, with N = 28672 11.8 / 13.4).  M = 48, K = 4096, N = 6144 47.7 -> 12.5 us; M = 64, K =
+  // 14336, N = 4096 157 -> 34; M = 32, K = 4096, N = 14336 (staged GEMV before)
+  // 36.7 -> 15.2.
+  const bool stream = N <= 16384 || (K > 128 + 7 * M && (N <= 32768 || K >= 4096));
+  if (M <= kStreamM && stream && aligned(x, 16) && aligned(w, 16) && N * K <= ((int64_t)1 << 40)) {
     GemvSegs sg{};
     sg.count = 1;
     sg.w[0] = static_cast<const uint8_t*>(w);

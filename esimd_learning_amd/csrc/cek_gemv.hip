@@ -1712,13 +1712,20 @@ int launch_gemv_a8w8(const uint8_t* x, const float* xs, const uint8_t* w, const 
   }
   if (M > 16) {
     // The weight-streaming kernel reads the activations once per workgroup
-    // of up to 64 weight rows: with several of those per CU and short K the
-    // tiled GEMM is faster (MI355X, weights from HBM, us, tiles / streaming:
-    // M = 64, K = 2048, N = 16384 16.3 / 12.4, N = 24576 17.6 / 19.6; K = 4096, N
-    // = 24576 33.9 / 31.4, N = 32768 37.0 / 37.7; M = 48, K = 2048, N = 24576 18.5
-    // / 16.5, N = 32768 19.6 / 20.2; K = 1024, N = 20480 10.9 / 11.4).
-    const bool wide = M <= 48 ? K >= 2048 && (N <= 24576 || K >= 4096) : K >= 4096 && N <= 24576;
-    if (N > 16384 && M > 32 && !wide) return CEK_ERR_UNSUPPORTED;
+    // of up to 64 weight rows and fills and drains its rings for each: with
+    // several of those per CU and short K the tiled GEMM is faster (MI355X,
+    // weights from HBM, us, tiles / streaming).  Above 16384 rows: M = 32, K = 512,
+    // N = 20480 7.1 / 8.4, K = 768 8.7 / 9.0, K = 960 13.0 / 9.9, K = 1024, N = 40960
+    // 13.2 / 16.3; M = 64, K = 2048, N = 16384 16.3 / 12.4, N = 24576 17.6 / 19.6; K =
+    // 4096, N = 24576 33.9 / 31.4, N = 32768 37.0 / 37.7; M = 48, K = 2048, N = 24576
+    // 18.5 / 16.5, N = 32768 19.6 / 20.2; K = 5376, N = 40960 50.6 / 49.7, N = 49152
+    // 53.9 / 64.6.  Above 32 rows also from 10240 up to K = 4 M: M = 64, K = 256, N =
+    // 14336 4.4 / 5.5; M = 48, K = 128, N = 12288 4.2 / 4.5, K = 256 4.7 / 4.6.
+    const bool wide = M <= 32   ? K > 768 && (K >= 2048 || N <= 32768)
+                      : M <= 48 ? K >= 2048 && (N <= 24576 || (K >= 4096 && N <= 40960))
+                                : K >= 4096 && N <= 24576;
+    if (N > 16384 && !wide) return CEK_ERR_UNSUPPORTED;
+    if (N >= 10240 && M > 32 && K <= 4 * M && K % 128 == 0) return CEK_ERR_UNSUPPORTED;
     return launch_stream(x, sg, SK_F32, M, K, out_dtype, CEK_E4M3, st);
   }
   if (out_dtype == CEK_F16) return launch_gemv_t<F16, F16, CEK_E4M3, true>(x, sg, SK_F32, (int)M, (int)K, true, st);

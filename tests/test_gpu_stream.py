@@ -17,6 +17,7 @@ value (2^-25 below fp16's normal range), plus the fp32 sum's (K + 16) 2^-24 sum
 import pytest
 import torch
 
+from conftest import assert_close_fp
 from esimd_learning_amd import synthetic
 
 pytestmark = pytest.mark.gpu
@@ -71,6 +72,28 @@ def test_stream_a8w8(ops, dev, M, K, N):
     # the two scales are multiplied in fp32 (2^-24), one more rounding of the product
     _check(y, a8.float().double() * sa.double()[:, None], W8.float().double(), s.double(), K + 2,
            f"M={M} K={K} N={N}")
+
+
+@pytest.mark.parametrize("act,M,K,N", [("fp16", 17, 192, 16385), ("fp16", 17, 256, 16385), ("fp16", 64, 576, 16390),
+                                       ("fp16", 64, 640, 16390), ("fp16", 33, 64, 32769), ("e4m3", 20, 768, 16400),
+                                       ("e4m3", 20, 832, 16400), ("e4m3", 32, 1024, 32800), ("e4m3", 40, 128, 10240),
+                                       ("e4m3", 40, 192, 10241), ("e4m3", 64, 256, 10250), ("e4m3", 64, 320, 10250)])
+def test_stream_or_tiles(ops, dev, act, M, K, N):
+    """Wide matrices of short K on both sides of the line to the tiled GEMMs
+    (whose fp8 MFMA sums 128 products in one step, hence the op pack's
+    tolerance for e4m3 activations)."""
+    print(f"stream or tiles {act} M={M} K={K} N={N}", flush=True)
+    W8, s = synthetic.weight_fp8(N, K, seed=K)
+    x = synthetic.activations(M, K, seed=M)
+    y = torch.full((M, N), float("nan"), dtype=torch.float16, device=dev)
+    if act == "e4m3":
+        x, sa = synthetic.quantize_rows(x.float())
+        ops.esimd_gemm_fp8_a8w8(x.to(dev), sa.to(dev), W8.to(dev), s.to(dev), y)
+        ref = (x.float().double() * sa.double()[:, None]) @ (W8.float().double() * s.double()[:, None]).t()
+        assert_close_fp(y.cpu(), ref, f"a8w8 M={M} K={K} N={N}")
+    else:
+        ops.esimd_gemv_fp8_pern(x.to(dev), W8.to(dev), s.to(dev), y, N, K)
+        _check(y, x.double(), W8.float().double(), s.double(), K, "w8a16")
 
 
 # Columns at which a workgroup has 8, 12, 16, 24, 32, 40, 48, 56 and 64 weight rows
