@@ -1556,19 +1556,26 @@ int launch_norm_gemv(const NormArgs& na, const void* w, const void* scale, int s
 // long-K matrix, whose few workgroups each pay the stages' barriers (N = 1000,
 // K = 6144 5.3 against 5.9; N = 2048 6.6 -> 6.2; e4m3 activations N = 2048, K =
 // 8192 6.6 against 7.0).
-// K that it has (16-bit activations): 9 .. 16 rows of a wide matrix (M = 16,
-// K = 4096, N = 8208 12.3 -> 9.6, N = 14336 15.5 -> 13.2, N = 28672 26.5 -> 25.2;
-// K = 14336, N = 16384 66.7 -> 43.4; M = 9, N = 9000 12.0 -> 9.6, but K = 3072, N =
-// 49152 28.2 against 30.2), K = 2048 above 4096 rows (M = 16, N = 6144 7.4 ->
-// 5.7; N = 4096 4.9 against 5.1) and K = 24576 from 12 rows on (M = 16, N = 3072
-// 29.4 -> 23.9).  The wide bound is above every merged gate/up width at which
-// the fused gate/up launch is held to the plain one bit for bit.
+// K that it has (16-bit activations), 9 .. 16 rows:
+//  * 3072, 4096 and 5120, matrices above 8192 rows (M = 16, K = 4096, N = 8208
+//    12.3 -> 9.6, N = 14336 15.5 -> 13.2, N = 28672 26.5 -> 25.2; M = 9, N = 9000
+//    12.0 -> 9.6).  Not at 8192, where the smaller matrices of a multi-matrix
+//    call would take a second launch (8192 + 1024 + 1024 rows, M = 9, K = 4096 11.6
+//    against 14.4 us) for little (K = 3072 8.2 / 7.6, K = 5120 11.6 / 11.0), nor
+//    above 32768 (K = 5120 24576 below 12 rows) except at K = 4096 from 12 rows on
+//    (N = 49152, M = 12: K = 4096 41.8 -> 36.3, K = 3072 29.0 against 29.6, K =
+//    5120 46.8 against 47.8);
+//  * 2048, above 4096 rows (M = 16, N = 6144 7.4 -> 5.7; N = 4096 4.9 against 5.1);
+//  * 14336, from 8192 rows (M = 16, N = 16384 66.7 -> 43.4);
+//  * 24576, from 12 activation rows on (M = 16, N = 3072 29.4 -> 23.9).
 static bool stream_matrix(bool xf8, int64_t M, int64_t K, int64_t n) {
   if (M < 3 || M > 16 || K % 64 != 0 || K > kStreamMaxK) return false;
-  if (!lds_k(K)) return !(M <= 4 && n <= (xf8 ? 2048 : 1024) && K > 4096);
+  if (!lds_k(K)) return !(M <= 4 && K > 4096 && n <= (xf8 ? 2048 : 1024));
   if (xf8 || M < 9) return false;
-  if (n >= 8192) return M >= 12 || n <= 24576 || (n <= 32768 && K <= 4096);
-  return (K == 2048 && n > 4096) || (K == 24576 && M >= 12 && n >= 2048);
+  if (K == 2048) return n > 4096 && (M >= 12 || n <= 32768);
+  if (K == 14336) return n >= 8192 && (M >= 12 || n <= 24576);
+  if (K == 24576) return M >= 12 ? n >= 2048 : n >= 8192 && n <= 24576;
+  return n > 8192 && (n <= (K == 5120 && M < 12 ? 24576 : 32768) || (K == 4096 && M >= 12));
 }
 
 template <typename T, typename TO, int FMT, bool XF8>
@@ -1576,30 +1583,17 @@ static int launch_gemv_t(const void* x, GemvSegs sg, int skind, int M, int K, bo
   const uint16_t* xp = static_cast<const uint16_t*>(x);
   int N = 0;  // launch shape is chosen from the total row count
   for (int i = 0; i < sg.count; ++i) N += sg.n[i];
-  // The LDS-staged MFMA kernel from three rows on (measured faster than the
-  // v_dot2 kernel there, and than the direct MFMA kernel throughout); from one
-  // row on for K >= 14336, whose v_dot2 workgroups re-read long activation
-  // rows (M = 1, K = 14336, N = 4096: 11.54 -> 11.06 us).  The choice depends
-  // on M and K only, so a multi-matrix launch runs the kernel family that
-  // each matrix alone would (the LDS forms it may pick between agree bit for
-  // bit).
-  const int m_lds = K >= 14336 ? 1 : 3;
   // Matrices that the weight-streaming kernel serves go to it, the rest on
   // through the kernels below (its sum order differs from theirs, so the
   // choice is per matrix: a multi-matrix launch gives each matrix what it
   // gets alone).
-  if (vec16) {
-    GemvSegs ss{}, so{};
-    ss.xs = so.xs = sg.xs;
-    for (int i = 0; i < sg.count; ++i) {
-      GemvSegs& d = stream_matrix(XF8, M, K, sg.n[i]) ? ss : so;
-      d.w[d.count] = sg.w[i];
-      d.s[d.count] = sg.s[i];
-      d.y[d.count] = sg.y[i];
-      d.n[d.count] = sg.n[i];
-      ++d.count;
-    }
-    if (ss.count > 0) {
+  if (vec16 && M >= 3) {
+    bool streams[MAX_SEGS], any = false;
+    for (int i = 0; i < sg.count; ++i) any |= streams[i] = stream_matrix(XF8, M, K, sg.n[i]);
+    if (any) {
+      GemvSegs ss{}, so{};
+      ss.xs = so.xs = sg.xs;
+      for (int i = 0; i < sg.count; ++i) seg_push(streams[i] ? ss : so, sg, i);
       const int rc = launch_stream(x, ss, skind, M, K, TO::code, FMT, st);
       if (rc != CEK_OK || so.count == 0) return rc;
       sg = so;
@@ -1607,6 +1601,14 @@ static int launch_gemv_t(const void* x, GemvSegs sg, int skind, int M, int K, bo
       for (int i = 0; i < sg.count; ++i) N += sg.n[i];
     }
   }
+  // The LDS-staged MFMA kernel from three rows on (measured faster than the
+  // v_dot2 kernel there, and than the direct MFMA kernel throughout); from one
+  // row on for K >= 14336, whose v_dot2 workgroups re-read long activation
+  // rows (M = 1, K = 14336, N = 4096: 11.54 -> 11.06 us).  Among the matrices
+  // left here the choice depends on M and K only, so a multi-matrix launch runs
+  // the kernel family that each matrix alone would (the LDS forms it may pick
+  // between agree bit for bit).
+  const int m_lds = K >= 14336 ? 1 : 3;
   if (vec16 && M >= m_lds && launch_lds<T, TO, FMT, XF8>(x, sg, skind, M, K, N, st)) return check_launch();
   if (vec16 && M <= 4) {
     // Rows per workgroup (measured on MI355X, one pass over > 2 GB of

@@ -36,6 +36,15 @@ __device__ inline SegRef find_seg(const GemvSegs& sg, int b) {
   return SegRef{sg.w[i], sg.s[i], sg.y[i], sg.n[i], b - sg.gstart[i]};
 }
 
+// Append matrix i of `from` to `to`.
+inline void seg_push(GemvSegs& to, const GemvSegs& from, int i) {
+  to.w[to.count] = from.w[i];
+  to.s[to.count] = from.s[i];
+  to.y[to.count] = from.y[i];
+  to.n[to.count] = from.n[i];
+  ++to.count;
+}
+
 // Fill gstart for `rows_per_wg` output rows per workgroup; returns the grid.
 inline int seg_grid(GemvSegs& sg, int rows_per_wg) {
   int g = 0;

@@ -35,6 +35,8 @@ namespace cek {
 
 constexpr int kStreamConsumers = 8;  // waves that multiply
 constexpr int kStreamMaxRows = 64;   // weight rows of a workgroup
+constexpr int kStreamNarrowRows = 24;    // the same, for the narrow form (launch_stream)
+constexpr int kStreamRotateRows = 8192;  // rows from which on a matrix has its K stages rotated
 constexpr int kStreamScaleBytes = kStreamMaxRows * 4 + 64 * 4;
 
 // One configuration: AR activation rows held in LDS, RW weight rows per
@@ -124,7 +126,7 @@ __device__ __forceinline__ void stream_load(uint8_t* slots, int rmax, uint32_t r
 
 template <typename T, int FMT, bool XF8, int AR, int RW, int KW>
 __global__ __launch_bounds__((StreamCfg<XF8, AR, RW, KW>::THREADS), (StreamCfg<XF8, AR, RW, KW>::LDSB > 81920 ? 3 : 6))
-void stream_kernel(const uint8_t* __restrict__ x, GemvSegs sg, int skind, int M, int K, int bf16_out, int rotate) {
+void stream_kernel(const uint8_t* __restrict__ x, GemvSegs sg, int skind, int M, int K, int bf16_out) {
   using C = StreamCfg<XF8, AR, RW, KW>;
   constexpr int KS = C::KS, ARB = C::ARB, MB = C::MB, NT = C::NT, R = C::R;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[C::LDSB];
@@ -136,7 +138,7 @@ void stream_kernel(const uint8_t* __restrict__ x, GemvSegs sg, int skind, int M,
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int r16 = lane & 15, g = lane >> 4;
   const int S = (K + KS - 1) / KS;
-  const int k_first = rotate ? (int)((unsigned)(sr.group >> 3) % (unsigned)S) : 0;
+  const int k_first = N >= kStreamRotateRows ? (int)((unsigned)(sr.group >> 3) % (unsigned)S) : 0;
 
   f4 acc[MB][NT];
 #pragma unroll
@@ -276,6 +278,7 @@ static int stream_rows(int M, int64_t N, int K, bool xf8, int max_rows) {
   const int64_t act = (M > 16 ? 3 : 4) * (xf8 ? (M + 1) / 2 : M);
   for (int r : kStreamRows) {
     if (r > max_rows) break;
+    if (r == 8 && N >= kStreamRotateRows) continue;  // (never the fastest there)
     const int64_t per_cu = ((N + r - 1) / r + kCUs - 1) / kCUs;
     const bool pair = M <= 16 && r <= (xf8 ? 24 : 48);  // two workgroups per CU
     int64_t next = pair ? 100000 : (M > 16 ? 450000 : 800000);
@@ -290,13 +293,13 @@ static int stream_rows(int M, int64_t N, int K, bool xf8, int max_rows) {
 }
 
 template <typename T, int FMT, bool XF8>
-static int launch_stream_t(const uint8_t* x, GemvSegs& sg, int skind, int M, int K, bool bf16_out, int rw, bool narrow, bool rotate,
+static int launch_stream_t(const uint8_t* x, GemvSegs& sg, int skind, int M, int K, bool bf16_out, int rw, bool narrow,
                            hipStream_t st) {
   const dim3 grid((unsigned)seg_grid(sg, rw));
 #define CEK_ST(AR, RW, KW)                                                                        \
   do {                                                                                            \
     stream_kernel<T, FMT, XF8, AR, RW, KW><<<grid, StreamCfg<XF8, AR, RW, KW>::THREADS, 0, st>>>( \
-        x, sg, skind, M, K, bf16_out, rotate);                                                    \
+        x, sg, skind, M, K, bf16_out);                                                    \
     return check_launch();                                                                        \
   } while (0)
 #define CEK_ST_ROWS(AR)                             \
@@ -308,12 +311,15 @@ static int launch_stream_t(const uint8_t* x, GemvSegs& sg, int skind, int M, int
           case 8: CEK_ST(AR, 8, 64);                \
           case 12: CEK_ST(AR, 12, 64);              \
           case 16: CEK_ST(AR, 16, 64);              \
+          case 24: CEK_ST(AR, 24, 64);              \
           default: return CEK_ERR_UNSUPPORTED;      \
         }                                           \
       }                                             \
     }                                               \
+    if constexpr (XF8 || (AR) > 8) {                \
+      if (rw == 8) CEK_ST(AR, 8, kw);               \
+    }                                               \
     switch (rw) {                                   \
-      case 8: CEK_ST(AR, 8, kw);                    \
       case 12: CEK_ST(AR, 12, kw);                  \
       case 16: CEK_ST(AR, 16, kw);                  \
       case 24: CEK_ST(AR, 24, kw);                  \
@@ -339,55 +345,61 @@ static int launch_stream_t(const uint8_t* x, GemvSegs& sg, int skind, int M, int
 // x: fp16 / bf16 [M, K] (io_dtype), or e4m3 codes with sg.xs set (io_dtype:
 // the output type); x and the weights 16-byte aligned.  M <= 64, K % 64 == 0;
 // CEK_ERR_UNSUPPORTED otherwise.  An output's sum order must not depend on
-// which matrices share the launch, so what it depends on is set per matrix,
-// and matrices that differ in it get launches of their own:
+// which matrices share the launch, so what it depends on is set per matrix:
 //  * 8192 rows or more: workgroup g starts at K stage (g / 8) mod S (g / 8: its
 //    place on its XCD), so that workgroups streaming at the same time read
 //    different columns of their rows and HBM's channels share the load (M =
-//    16, K = 4096, N = 16384: 17.3 -> 14.6 us); the matrix is launched alone;
-//  * up to 8 rows of 16-bit activations and 4096 weight rows (`narrow`, at
-//    most 16 rows per workgroup): 64 K values per wave and stage instead of
-//    32, half the barriers (M = 4, K = 10240, N = 2560 9.2 -> 8.5 us).
+//    16, K = 4096, N = 16384: 17.3 -> 14.6 us).  g counts workgroups of the rows
+//    that stream_rows gives the matrix alone: matrices that agree in it share a
+//    launch, and the other ones of their K per stage join it, whatever its rows;
+//  * up to 8 rows of 16-bit activations and fewer than 8192 weight rows (narrow,
+//    at most 24 rows per workgroup): 64 K values per wave and stage instead of
+//    32, half the barriers (M = 4, K = 10240, N = 2560 9.2 -> 8.5 us, N = 512 9.4
+//    -> 7.1; N = 6144 within 3%): a launch of their own.
+// Three matrices of 9000 rows, M = 4, K = 2560 27.9 us in a launch each -> 15.8;
+// 5120 + 1024 + 1024 rows, M = 5 10.1 us in two launches -> 6.4.
 int launch_stream(const void* x, const GemvSegs& sg, int skind, int64_t M, int64_t K, int io_dtype, int fp8_fmt,
                   hipStream_t st) {
   if (M < 1 || M > 64 || K < 64 || K > kStreamMaxK || K % 64 != 0) return CEK_ERR_UNSUPPORTED;
   const uint8_t* xp = static_cast<const uint8_t*>(x);
   const int m = (int)M, k = (int)K;
-  const bool bf = io_dtype == CEK_BF16;
-  auto launch = [&](GemvSegs& part, bool narrow, bool rotate) {
-    int64_t N = 0;
-    for (int i = 0; i < part.count; ++i) N += part.n[i];
-    const int rw = stream_rows(m, N, k, sg.xs != nullptr, narrow ? 16 : kStreamMaxRows);
-    if (sg.xs) return launch_stream_t<F16, CEK_E4M3, true>(xp, part, skind, m, k, bf, rw, narrow, rotate, st);
+  const bool bf = io_dtype == CEK_BF16, xf8 = sg.xs != nullptr;
+  auto launch = [&](GemvSegs& part, bool narrow, int rw) {
+    if (part.count == 0) return (int)CEK_OK;
+    if (rw == 0) {
+      int64_t N = 0;
+      for (int i = 0; i < part.count; ++i) N += part.n[i];
+      rw = stream_rows(m, N, k, xf8, narrow ? kStreamNarrowRows : kStreamMaxRows);
+    }
+    if (xf8) return launch_stream_t<F16, CEK_E4M3, true>(xp, part, skind, m, k, bf, rw, narrow, st);
     if (!bf) {
-      if (fp8_fmt == CEK_E4M3) return launch_stream_t<F16, CEK_E4M3, false>(xp, part, skind, m, k, bf, rw, narrow, rotate, st);
-      return launch_stream_t<F16, CEK_E5M2, false>(xp, part, skind, m, k, bf, rw, narrow, rotate, st);
+      if (fp8_fmt == CEK_E4M3) return launch_stream_t<F16, CEK_E4M3, false>(xp, part, skind, m, k, bf, rw, narrow, st);
+      return launch_stream_t<F16, CEK_E5M2, false>(xp, part, skind, m, k, bf, rw, narrow, st);
     }
-    if (fp8_fmt == CEK_E4M3) return launch_stream_t<BF16, CEK_E4M3, false>(xp, part, skind, m, k, bf, rw, narrow, rotate, st);
-    return launch_stream_t<BF16, CEK_E5M2, false>(xp, part, skind, m, k, bf, rw, narrow, rotate, st);
+    if (fp8_fmt == CEK_E4M3) return launch_stream_t<BF16, CEK_E4M3, false>(xp, part, skind, m, k, bf, rw, narrow, st);
+    return launch_stream_t<BF16, CEK_E5M2, false>(xp, part, skind, m, k, bf, rw, narrow, st);
   };
-  GemvSegs part[2]{};  // the others: wide, narrow
-  part[0].xs = part[1].xs = sg.xs;
+  GemvSegs narrow{}, wide{};  // wide: with the first group of rotated matrices
+  narrow.xs = wide.xs = sg.xs;
+  int rows[MAX_SEGS];  // of a rotated matrix not yet launched, else 0
   for (int i = 0; i < sg.count; ++i) {
-    GemvSegs one{};
-    one.xs = sg.xs;
-    GemvSegs& d = sg.n[i] >= 8192 ? one : part[!sg.xs && M <= 8 && sg.n[i] <= 4096];
-    d.w[d.count] = sg.w[i];
-    d.s[d.count] = sg.s[i];
-    d.y[d.count] = sg.y[i];
-    d.n[d.count] = sg.n[i];
-    ++d.count;
-    if (one.count) {
-      const int rc = launch(one, false, true);
-      if (rc != CEK_OK) return rc;
-    }
+    rows[i] = sg.n[i] >= kStreamRotateRows ? stream_rows(m, sg.n[i], k, xf8, kStreamMaxRows) : 0;
+    if (!rows[i]) seg_push(!xf8 && M <= 8 ? narrow : wide, sg, i);
   }
-  for (int narrow = 0; narrow < 2; ++narrow) {
-    if (part[narrow].count == 0) continue;
-    const int rc = launch(part[narrow], narrow != 0, false);
+  for (int i = 0; i < sg.count; ++i) {
+    const int rw = rows[i];
+    if (!rw) continue;
+    for (int j = i; j < sg.count; ++j)
+      if (rows[j] == rw) {
+        seg_push(wide, sg, j);
+        rows[j] = 0;
+      }
+    const int rc = launch(wide, false, rw);
     if (rc != CEK_OK) return rc;
+    wide.count = 0;
   }
-  return CEK_OK;
+  const int rc = launch(wide, false, 0);
+  return rc != CEK_OK ? rc : launch(narrow, true, 0);
 }
 
 }  // namespace cek

@@ -14,6 +14,8 @@ value (2^-25 below fp16's normal range), plus the fp32 sum's (K + 16) 2^-24 sum
 |x w| s.
 """
 
+import ctypes
+
 import pytest
 import torch
 
@@ -148,3 +150,35 @@ def test_stream_fused_equals_single(ops, dev, M, K, Ns):
         one = torch.empty(M, n, dtype=torch.float16, device=dev)
         ops.esimd_gemv_fp8_pern(x, w, s, one, n, K)
         assert torch.equal(one, y), f"N={n}"
+
+
+def _launches(fn):
+    """Kernels that fn launches: the nodes of a graph captured from it."""
+    with open("/proc/self/maps") as f:  # the HIP runtime that this process runs on
+        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64.so" in line))
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        fn()
+    n = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("M,K,Ns,launches", [
+    (4, 2560, (9000, 9000, 9000), 1), (5, 2560, (5120, 1024, 1024), 1), (8, 1088, (8191, 17), 1),
+    (9, 4096, (8192, 1024, 1024), 1), (12, 6144, (8192, 1024, 1024), 1), (16, 2560, (1000, 9000, 14336, 9001), 2),
+    (3, 1088, (9000, 1000, 8200), 2), (12, 4096, (14336, 4096), 2)])
+def test_stream_fused_launches(ops, dev, M, K, Ns, launches):
+    """Matrices of a multi-matrix call share a launch unless their sums differ in
+    order (narrow ones and ones that start at rotated K stages, or whose rotation
+    differs; the streaming and the staged kernel), and get what they get alone."""
+    print(f"stream launches M={M} K={K} N={Ns}", flush=True)
+    x = synthetic.activations(M, K, seed=5).to(dev)
+    ws, ss = zip(*[[t.to(dev) for t in synthetic.weight_fp8(n, K, seed=20 + i)] for i, n in enumerate(Ns)])
+    ys = [torch.full((M, n), float("nan"), dtype=torch.float16, device=dev) for n in Ns]
+    ops.esimd_gemv_fp8_pern_fused(x, ws, ss, ys)
+    for n, w, s, y in zip(Ns, ws, ss, ys):
+        one = torch.empty(M, n, dtype=torch.float16, device=dev)
+        ops.esimd_gemv_fp8_pern(x, w, s, one, n, K)
+        assert torch.equal(one, y), f"N={n}"
+    assert _launches(lambda: ops.esimd_gemv_fp8_pern_fused(x, ws, ss, ys)) == launches
