@@ -36,7 +36,8 @@ def _check(y, x64, w64, s64, K, what):
 
 @pytest.mark.parametrize("io,fmt,per_channel", [(torch.float16, torch.float8_e4m3fn, True),
                                                 (torch.bfloat16, torch.float8_e5m2, False)])
-@pytest.mark.parametrize("K,N", [(64, 7), (320, 250), (2112, 1025), (2560, 8200), (10240, 1), (6144, 136)])
+@pytest.mark.parametrize("K,N", [(64, 7), (320, 250), (2112, 1025), (2560, 8200), (10240, 1), (6144, 136), (8192, 2048),
+                                 (8192, 2049)])
 @pytest.mark.parametrize("M", [3, 4, 5, 8, 9, 16])
 def test_stream_gemv(ops, dev, M, K, N, io, fmt, per_channel):
     print(f"stream gemv M={M} K={K} N={N} {io} {fmt}", flush=True)
