@@ -1914,13 +1914,11 @@ static A8w8Plan plan_a8w8_rounds(int64_t M, int64_t N, int64_t K, bool allow_spl
 // rounds of workgroups at its full-occupancy rate (a partial round costs a
 // full one), the 64 x 128 tile also split in 2, 4 or 8 parts plus the fp32
 // partials' traffic and the finalize launch; split only when allowed, on the
-// pipelined path, and 10% faster than the best unsplit plan.  At M = 64
-// (config 3's prefill-sized decode) the split plans measured 1.2-1.8x faster
-// than the weight-streaming kernels, and 8 parts of 512 K values slower than
-// 4 (M = 64, K = 4096: 13.8 against 11.2 us).  The split 64 x 128 launches
-// run a 3-slot ring (72 KB per workgroup, two per CU): M = 64, N = 6144,
-// weights from HBM, K = 4096 15.3 -> 13.2 us, K = 5120 16.0 -> 13.2 us; M = 96
-// 17.4 -> 16.4 us.
+// pipelined path, and 10% faster than the best unsplit plan (and at M = 64
+// only where a8w8_streams64 leaves the shape to them).  8 parts of 512 K values
+// are slower than 4 (M = 64, K = 4096: 13.8 against 11.2 us).  The split 64 x 128
+// launches run a 3-slot ring (72 KB per workgroup, two per CU): M = 96, K = 4096,
+// N = 6144, weights from HBM 17.4 -> 16.4 us.
 static A8w8Plan plan_a8w8(int64_t M, int64_t N, int64_t K, bool pipe_ok, bool allow_split) {
   if (pipe_ok && M >= 128 && N >= 128) return plan_a8w8_rounds(M, N, K, allow_split);
   A8w8Plan best{0, 1};
@@ -1960,9 +1958,17 @@ static bool a8w8_off32(int64_t M, int64_t N, int64_t K) {
   return (uint64_t)M * (uint64_t)K < (1ull << 32) && (uint64_t)N * (uint64_t)K < (1ull << 32);
 }
 
+// M = 64 on the weight-streaming kernel (launch_gemv_a8w8) rather than on split
+// 64 x 128 tiles: K up to 5120 and N up to 16384 (us, split / streaming: K = 2048,
+// N = 4096 9.5 / 6.2; K = 4096, N = 6144 12.9 / 10.8, N = 14336 19.9 / 17.3; K =
+// 5376, N = 14336 20.7 / 22.5; K = 8192, N = 4096 13.4 / 14.1; K = 4096, N = 26240
+// 28.9 / 33.0).
+static bool a8w8_streams64(int64_t N, int64_t K) { return K <= 5120 && N <= 16384; }
+
 // Bytes of fp32 partials the split-K plan for this shape needs (0: unsplit).
 static int64_t a8w8_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M < 64 || K % 128 != 0 || M > 65535 * 64 || N > INT32_MAX || K > INT32_MAX || M <= 0 || N <= 0) return 0;
+  if (M == 64 && a8w8_streams64(N, K)) return 0;
   const A8w8Plan p = plan_a8w8(M, N, K, a8w8_off32(M, N, K), true);
   return p.split > 1 ? (int64_t)p.split * M * N * 4 : 0;
 }
@@ -2123,9 +2129,8 @@ static int launch_a8w8(const uint8_t* a, const float* sa, const uint8_t* b, cons
   if (out_dtype != CEK_F16 && out_dtype != CEK_BF16) return CEK_ERR_INVALID;
   // Skinny A: stream the weights once with the GEMV kernels rather than tile
   // a mostly empty GEMM (they decline the shapes the tiles serve better).
-  // At M = 64 (the 64-row tile's smallest M), given the workspace the
-  // split-K plan asks for, the tiled GEMM in K parts is 1.2-1.8x faster
-  // (measured on MI355X, K = 4096..14336, N = 4096..28672).
+  // At M = 64 (the 64-row tile's smallest M), given the workspace that a
+  // split-K plan asks for (a8w8_workspace_bytes), the tiled GEMM in K parts.
   if (M <= 64) {
     const int64_t need64 = M == 64 ? a8w8_workspace_bytes(M, N, K) : 0;
     if (!(need64 > 0 && ws && ws_bytes >= need64)) {

@@ -467,12 +467,8 @@ void esimd_fused_add_rms_norm_quant_gemv_fp8(at::Tensor hidden_states, at::Tenso
            op);
   const auto* bp = static_cast<const uint8_t*>(b.data_ptr());
   const auto* sb = static_cast<const float*>(b_scale.data_ptr());
-  // At 64 rows the weight-streaming kernel that a call without a workspace
-  // takes is faster up to K = 5120 (us, streaming / split K: K = 4096, N = 6144
-  // 10.9 / 13.2, N = 14336 18.2 / 20.7; K = 8192, N = 4096 14.3 / 13.5).
   at::Tensor ws;
-  const bool split = M > 64 || (M == 64 && (K > 5120 || N > 16384));
-  const int64_t need = split ? split_workspace(ws, cek_gemm_fp8_a8w8_workspace_size(M, N, K), out_scale) : 0;
+  const int64_t need = split_workspace(ws, cek_gemm_fp8_a8w8_workspace_size(M, N, K), out_scale);
   void* wp = need > 0 ? ws.data_ptr() : nullptr;
   if (!gelu_and_mul) {
     check_rc(cek_gemm_fp8_a8w8_ws(q, qs, bp, sb, output.data_ptr(), M, N, K, io, wp, need, st), op);

@@ -54,9 +54,10 @@ The intermediate buffers and counters are allocated once in the
 constructor, so at decode sizes a step enqueues only kernels: it can be
 captured in a HIP graph (``capture``) and replayed, which removes host launch
 overhead from the latency-bound small kernels between the GEMVs.  (One
-exception: with ``act_fp8`` at M = 64 the a8w8 op splits K and takes its
-fp32 workspace from PyTorch's caching allocator on every call -- inside a
-captured graph, from the graph's memory pool.)
+exception: with ``act_fp8`` at M = 64 the a8w8 op splits K where K exceeds
+5120 or N 16384 (a wide gate/up matrix) and takes its fp32 workspace from
+PyTorch's caching allocator on every call -- inside a captured graph, from the
+graph's memory pool.)
 """
 
 import torch

@@ -205,12 +205,12 @@ def test_a8w8_large_tiles(ops, dev, M, K, N):
 @pytest.mark.parametrize("M,K,N", [(65, 4096, 200), (100, 2048, 512), (300, 8192, 4096), (300, 14336, 4096),
                                    (512, 14336, 4096), (200, 8192, 2048), (150, 4096, 1000), (65, 4096, 203),
                                    (100, 2048, 1001),
-                                   (64, 4096, 6144), (64, 14336, 4096), (64, 4096, 300), (64, 4096, 28672)])
+                                   (64, 6144, 6144), (64, 14336, 4096), (64, 8192, 300), (64, 4096, 28672)])
 def test_a8w8_split_k(ops, dev, M, K, N):
     """Shapes with too few output tiles split K (the op allocates the
     workspace the plan asks for): 64 x 128 tiles in 8, 4 and 2 parts (M = 64
-    included, which without a workspace takes the weight-streaming kernels;
-    at N = 6144 on 64 x 96 tiles, 256 parts), 128 x 256 in 4 parts, 128 x 128
+    included where K or N is too large for the weight-streaming kernel, which
+    serves it without a workspace; at N = 6144 on 64 x 96 tiles, 256 parts), 128 x 256 in 4 parts, 128 x 128
     (four waves) in 8 and 4 parts.  Against the CPU oracle;
     the unsplit C-ABI call (no workspace) agrees within the same tolerance;
     two split calls agree bit for bit (the parts are added in order), and a

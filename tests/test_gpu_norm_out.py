@@ -54,3 +54,33 @@ def test_norm_gemv_beyond_four_rows(ops, dev, M, N, K, alias):
     y1 = torch.full_like(y, float("nan"))
     ops.esimd_fused_add_rms_norm_gemv_fp8(buf[:M], buf[M:2 * M], w, 1e-6, buf[out], W8, sw, y1)
     assert torch.equal(buf[out], rn) and torch.equal(y1, y)
+
+
+@pytest.mark.parametrize("K,N", [(4096, 6144), (5120, 16384), (5120, 16386), (6144, 512)])
+def test_quant_gemv_at_64_rows(ops, dev, K, N):
+    """64 rows, where the a8w8 product is a streaming launch or split in K by its
+    sizes: the fused op, its two ops and the entry point without a workspace of
+    the caller's make the same choice, so they agree bit for bit."""
+    M = 64
+    print(f"norm quant gemv M={M} N={N} K={K}", flush=True)
+    lib = cabi.load()
+    W8, sw = synthetic.weight_fp8(N, K, seed=3)
+    W8, sw = W8.view(torch.uint8).to(dev), sw.to(dev)
+    h, r = (synthetic.activations(M, K, seed=s).to(dev) for s in (4, 5))
+    w = synthetic.norm_weight(K).to(dev)
+    q = torch.empty(M, K, dtype=torch.float8_e4m3fn, device=dev)
+    s, ro, rn = torch.empty(M, device=dev), torch.empty_like(r), r.clone()
+    ops.esimd_fused_add_rms_norm_quant_fp8(h, rn, w, 1e-6, q, s)
+    a = q.view(torch.uint8)
+    y, y1, y2, g, g1 = (torch.full((M, n), float("nan"), dtype=torch.float16, device=dev)
+                        for n in (N, N, N, N // 2, N // 2))
+    ops.esimd_gemm_fp8_a8w8(a, s, W8, sw, y)
+    ops.esimd_gemm_fp8_a8w8_gelu_and_mul(a, s, W8, sw, g)
+    cabi.check(lib.cek_gemm_fp8_a8w8_noalloc(cabi.ptr(a), cabi.ptr(s), cabi.ptr(W8), cabi.ptr(sw), cabi.ptr(y2), M, N,
+                                             K, 0, cabi.stream_ptr()))
+    assert torch.equal(y, y2)
+    q1, s1 = torch.empty_like(q), torch.empty_like(s)
+    ops.esimd_fused_add_rms_norm_quant_gemv_fp8(h, r, w, 1e-6, ro, q1, s1, W8, sw, y1)
+    assert torch.equal(y, y1)
+    ops.esimd_fused_add_rms_norm_quant_gemv_fp8(h, r, w, 1e-6, ro, q1, s1, W8, sw, g1, True)
+    assert torch.equal(g, g1)

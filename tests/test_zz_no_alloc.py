@@ -6,7 +6,7 @@ Against cek_gemm_fp8_a8w8_ws with a workspace of the plan's size (the same
 kernels and plan, so bit for bit) and against the CPU oracle to the op
 pack's tolerance, on calls in a row that share the static buffer: the
 largest split plan the buffer holds (M = 512, K = 14336, N = 4096: 4 parts,
-32 MiB), then a smaller one (M = 64, K = 4096, N = 6144: 4 parts, 6 MiB),
+32 MiB), then a smaller one (M = 64, K = 8192, N = 3072: 8 parts, 6 MiB),
 then the first again; a shape that runs unsplit uses no scratch; a plan
 larger than the buffer is refused with CEK_ERR_SCRATCH before any launch;
 an eager call allocates nothing, and the call captured in a HIP graph
@@ -64,7 +64,7 @@ def test_a8w8_noalloc_calls_in_a_row(dev):
     assert torch.cuda.is_available()
     lib = cabi.load()
     _run_pair(lib, dev, 512, 14336, 4096, seed=3, expect_split=True)
-    _run_pair(lib, dev, 64, 4096, 6144, seed=4, expect_split=True)
+    _run_pair(lib, dev, 64, 8192, 3072, seed=4, expect_split=True)
     _run_pair(lib, dev, 512, 14336, 4096, seed=5, expect_split=True)
     _run_pair(lib, dev, 2048, 4096, 6144, seed=6, expect_split=False)
 
