@@ -1553,24 +1553,25 @@ constexpr int64_t kStreamM = 64;
 //  3  128 x 256, 3 slots;   4  128 x 128, 3 slots (split K only);
 //  5  128 x 96 (4 x 2 waves, two loader waves), 3 slots, unsplit, only as one
 //     round of 192 .. 256 tiles with K <= 8192 (fitted at M = 512, N = 6144);
-//  6  128 x 128 in two K teams (gemm_w8a16_team_kernel), 3 slots, unsplit or
-//     split, only as one round of at most 256 workgroups, where it is 4-10%
-//     faster than 4 (two rounds are slower: a workgroup's fill is longer).
-//     Also for 64 < M < 128.  In that round a workgroup takes t0 + step per
-//     64-deep step, 0.9 of it with few others and 1.1 with all CUs busy.  (An
-//     unsplit launch of the others that does not fill its first round pays a
-//     whole t0, at least 4.3: 128 x 256, M = 256, K = 1024, N = 5120 16.4 us in
-//     40 workgroups, against 11.7 in 80 of 6.)
+//  6  128 x 128 in two K teams (gemm_w8a16_team_kernel), 3 slots, unsplit or in
+//     2 or 4 parts, only as one round of at most 256 workgroups (two rounds are
+//     slower: a workgroup's fill is longer).  Also for 64 < M < 128.  In that
+//     round a workgroup takes t0 + step per 64-deep step, 0.9 of it with few
+//     others and 1.1 with all CUs busy.  In 4 parts it is as fast as 4 up to K =
+//     8192 and 4% faster at 14336; the model, with no t0 for 4, takes it from
+//     about K = 27000 on (M = 65, N = 8192).
 //     Measured (us, weights from HBM, before -> now): M = 333, K = 2560, N =
 //     10752 32.0 (256 split parts of 128 x 256) -> 23.5; M = 512, K = 4096, N =
-//     6144 32.0 -> 30.2; M = 256, K = 14336, N = 4096 in 4 parts 37.7 -> 36.2;
-//     M = 100, K = 4096, N = 6144 47.9 (128 x 128, two per CU) -> 29.5, in 4
-//     parts of 4 18.5.
-// Unsplit: 0-3, 5 and 6; split in 2, 4 or 8 parts (K values per part >= 1024):
-// 0, 3 and 6, and 4 in 4 or 8 parts.  On the nine config-4 shapes (HBM and
-// cache-resident) and ten others (M = 128 .. 3000) the plan's pick measured
-// within 7% of the fastest of sixteen forms (M = 512, K = 14336: 171 -> 68 us
-// split in 4; M = 512, K = 4096, N = 6144: 52 -> 36 us).
+//     6144 32.0 -> 30.2; M = 100, K = 4096, N = 6144 47.9 (128 x 128, two per CU)
+//     -> 29.5, in 4 parts of 4 18.5.
+// A round of an unsplit launch takes at least 4.3 us beside its steps, whole in
+// the last one, whose steps are shared with fewer others (0.6 + 0.4 of its fill):
+// M = 256, K = 1024, N = 5120 16.4 us in 40 workgroups of 3, 11.7 in 80 of 6; M =
+// 1024, K = 512, N = 10752 21.9 us in 1.3 rounds of 0, 17.6 in 0.7 of 2.
+// Unsplit: 0-3, 5 and 6; split in 2, 4 or 8 parts (K values per part >= 1024): 0
+// and 3, 6 in 2 or 4, 4 in 4 or 8.  Over 1348 shapes of 128 .. 4096 rows the plan's
+// pick is 3% (geometric mean) above the fastest form, and slower than the plan
+// without 6 and these fixed parts at one of them by more than 3%.
 struct W8Opt { int bm, bn; double t0, step; };
 constexpr int kW8Cfgs = 7;
 constexpr W8Opt kW8Opts[kW8Cfgs] = {{256, 128, 0.49, 0.972}, {256, 192, 6.84, 1.166}, {256, 256, 0.0, 1.595},
@@ -1593,7 +1594,7 @@ static W8Plan plan_w8a16(int64_t M, int64_t N, int64_t K, bool allow_split) {
     // (128 rows at 64 < M < 128 for 4 and 6: every tiled kernel's loads clamp rows)
     if ((M < o.bm && c != 4 && c != 6) || N < o.bn) continue;
     for (int sp : {1, 2, 4, 8}) {
-      const bool ok = sp == 1 ? c != 4 : (allow_split && (c == 0 || c == 3 || c == 6 || (c == 4 && sp >= 4)));
+      const bool ok = sp == 1 ? c != 4 : (allow_split && (c == 0 || c == 3 || (c == 6 && sp <= 4) || (c == 4 && sp >= 4)));
       if (!ok || (K / 64) % sp || (sp > 1 && K / sp < 1024)) continue;
       const int64_t units = ((M + o.bm - 1) / o.bm) * ((N + o.bn - 1) / o.bn) * sp;
       // 128 x 96 only as one nearly full round of at most 8192 K values, where
@@ -1606,10 +1607,17 @@ static W8Plan plan_w8a16(int64_t M, int64_t N, int64_t K, bool allow_split) {
       const double steps = (double)(K / 64 / sp) * o.step;
       const double part = 0.6 + 0.4 * f;
       double t;
-      if (c == 6) t = (0.9 + 0.2 * (double)units / 256.0) * (o.t0 + steps);
-      else if (full == 0 && sp == 1) t = std::max(o.t0, 4.3) + steps * part;
-      else t = ((double)full + (f > 0.0 ? part : 0.0)) * (o.t0 + steps);
-      if (sp > 1) t += ((double)sp * M * N * 4.0 + (double)M * N * 2.0) / 5.0e6 + 1.5;
+      if (c == 6) {
+        t = (0.9 + 0.2 * (double)units / 256.0) * (o.t0 + steps);
+      } else if (sp == 1) {
+        const double fixed = std::max(o.t0, 4.3);
+        t = (double)full * (fixed + steps) + (f > 0.0 ? fixed + steps * part : 0.0);
+      } else {
+        t = ((double)full + (f > 0.0 ? part : 0.0)) * (o.t0 + steps);
+      }
+      // the parts read and the output written, and the second launch; 4% in
+      // favour of no split, about what the model errs by
+      if (sp > 1) t = (t + ((double)sp * M * N * 4.0 + (double)M * N * 2.0) / 5.0e6 + 3.5) * 1.04;
       if (tbest < 0 || t < tbest) {
         tbest = t;
         best = W8Plan{c, sp};
@@ -1715,8 +1723,7 @@ int launch_w8a16(const void* x, const void* w, const void* scale, int skind, voi
     if (plan.cfg == 6) {                                                   \
       if (plan.split == 1) CEK_W8T(TY, F, 1);                              \
       else if (plan.split == 2) CEK_W8T(TY, F, 2);                         \
-      else if (plan.split == 4) CEK_W8T(TY, F, 4);                         \
-      else CEK_W8T(TY, F, 8);                                              \
+      else CEK_W8T(TY, F, 4);                                              \
     } else if (plan.split > 1) {                                           \
       if (plan.cfg == 0) CEK_W8P_SPLITS(TY, F, 256, 128);                  \
       else if (plan.cfg == 3) CEK_W8P_SPLITS(TY, F, 128, 256);             \
@@ -1820,6 +1827,13 @@ extern "C" int cek_gemm_fp8_pert(const void* x, const void* w, const float* scal
                                  int io_dtype, int fp8_fmt, void* stream) {
   return cek::launch_w8a16(x, w, scale, cek::SK_F32_SCALAR, y, M, N, K, io_dtype, fp8_fmt, nullptr, 0,
                            (hipStream_t)stream);
+}
+
+extern "C" int cek_gemm_fp8_pert_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_bytes) {
+  if (M <= cek::kStreamM || N <= 16 || M > 65535 * 64 || N > INT32_MAX || K > INT32_MAX || K <= 0) return -1;
+  const int64_t need = cek::w8a16_workspace_bytes(M, N, K);
+  const cek::W8Plan p = cek::plan_w8a16(M, N, K, need > 0 && workspace_bytes >= need);
+  return p.cfg < 0 ? -1 : 16 * p.cfg + p.split;
 }
 
 extern "C" int64_t cek_gemm_fp8_pert_workspace_size(int64_t M, int64_t N, int64_t K) {

@@ -120,6 +120,12 @@ int cek_gemm_fp8_pert(const void* x, const void* w, const float* scale, void* y,
  * reference entry as cek_gemm_fp8_pert): the reference has no split K.
  */
 int64_t cek_gemm_fp8_pert_workspace_size(int64_t M, int64_t N, int64_t K);
+/*
+ * NEW, for tests and tuning: the tiled launch that a call of more than 64
+ * rows with that much workspace takes, 16 * tile + parts of K (tile: the index
+ * into the library's list of w8a16 tiles); -1 where other kernels serve it.
+ */
+int cek_gemm_fp8_pert_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_bytes);
 int cek_gemm_fp8_pert_ws(const void* x, const void* w, const float* scale, void* y,
                          int64_t M, int64_t N, int64_t K, int io_dtype, int fp8_fmt,
                          void* workspace, int64_t workspace_bytes, void* stream);

@@ -61,34 +61,46 @@ def test_gemm_pert_prefill(ops, dev, M, K, N):
     assert_close_fp(y.cpu(), ogemv.gemm_fp8_pert(x, W8, sv), f"prefill M={M}")
 
 
-@pytest.mark.parametrize("M,K,N,parts,io,fmt", [
-    (276, 2048, 130, 2, torch.float16, torch.float8_e4m3fn),     # 256 x 128, 2 parts
-    (1736, 16384, 847, 4, torch.bfloat16, torch.float8_e4m3fn),  # 256 x 128, 4 parts
-    (2977, 2048, 1325, 0, torch.float16, torch.float8_e5m2),     # 256 x 128
-    (1444, 2048, 5388, 0, torch.float16, torch.float8_e4m3fn),   # 256 x 192
-    (1298, 2048, 8256, 0, torch.bfloat16, torch.float8_e5m2),    # 256 x 256
-    (787, 128, 8256, 0, torch.float16, torch.float8_e4m3fn),     # 256 x 256, one K step
-    (641, 2048, 5388, 0, torch.float16, torch.float8_e4m3fn),    # 128 x 256
-    (130, 128, 369, 0, torch.bfloat16, torch.float8_e4m3fn),     # 128 x 256, one K step
-    (130, 2048, 369, 2, torch.float16, torch.float8_e4m3fn),     # 128 x 256, 2 parts
-    (130, 8192, 6344, 4, torch.float16, torch.float8_e5m2),      # 128 x 256, 4 parts
-    (1000, 8192, 1000, 4, torch.float16, torch.float8_e4m3fn),   # 128 x 128, 4 parts
-    (130, 130, 4096, 0, torch.float16, torch.float8_e4m3fn),     # K = 130: not a multiple of 64
-    (130, 4096, 130, 4, torch.float16, torch.float8_e4m3fn),     # 128 x 128, 4 parts
-    (130, 8192, 130, 8, torch.bfloat16, torch.float8_e4m3fn),    # 128 x 128, 8 parts
-    (500, 2048, 6000, 0, torch.float16, torch.float8_e4m3fn),    # 128 x 96 (4 x 2 waves, padded epilogue rows)
-    (450, 4096, 5000, 0, torch.bfloat16, torch.float8_e5m2),     # 128 x 96
+# the list of w8a16 tiles (cek_gemm_fp8_pert_plan), 6: 128 x 128 in two K teams
+TILE = {"256 x 128": 0, "256 x 192": 1, "256 x 256": 2, "128 x 256": 3, "128 x 128": 4, "128 x 96": 5, "team": 6}
+
+
+@pytest.mark.parametrize("M,K,N,parts,tile,io,fmt", [
+    (276, 2048, 130, 2, "256 x 128", torch.float16, torch.float8_e4m3fn),
+    (1736, 16384, 847, 4, "256 x 128", torch.bfloat16, torch.float8_e4m3fn),
+    (3604, 2048, 2056, 0, "256 x 128", torch.float16, torch.float8_e5m2),
+    (390, 64, 142, 0, "256 x 128", torch.bfloat16, torch.float8_e4m3fn),   # one K step
+    (1444, 2048, 5388, 0, "256 x 192", torch.float16, torch.float8_e4m3fn),
+    (1298, 2048, 8256, 0, "256 x 256", torch.bfloat16, torch.float8_e5m2),
+    (1032, 128, 7171, 0, "256 x 256", torch.float16, torch.float8_e4m3fn),  # two K steps
+    (898, 64, 8201, 0, "256 x 256", torch.float16, torch.float8_e5m2),      # one K step
+    (2977, 2048, 1325, 0, "128 x 256", torch.float16, torch.float8_e5m2),
+    (641, 2048, 5388, 0, "128 x 256", torch.float16, torch.float8_e4m3fn),
+    (787, 128, 8256, 0, "128 x 256", torch.float16, torch.float8_e4m3fn),
+    (146, 64, 269, 0, "128 x 256", torch.bfloat16, torch.float8_e4m3fn),    # one K step
+    (130, 2048, 369, 2, "128 x 256", torch.float16, torch.float8_e4m3fn),
+    (130, 8192, 6344, 4, "128 x 256", torch.float16, torch.float8_e5m2),
+    (1000, 8192, 1000, 4, "128 x 128", torch.float16, torch.float8_e4m3fn),
+    (130, 130, 4096, 0, None, torch.float16, torch.float8_e4m3fn),          # K = 130: not a multiple of 64
+    (130, 128, 369, 0, "team", torch.bfloat16, torch.float8_e4m3fn),
+    (130, 4096, 130, 4, "128 x 128", torch.float16, torch.float8_e4m3fn),
+    (130, 8192, 130, 8, "128 x 128", torch.bfloat16, torch.float8_e4m3fn),
+    (500, 2048, 6000, 0, "128 x 96", torch.float16, torch.float8_e4m3fn),   # 4 x 2 waves, padded epilogue rows
+    (450, 4096, 5000, 0, "128 x 96", torch.bfloat16, torch.float8_e5m2),
+    (258, 128, 6049, 0, "128 x 96", torch.float16, torch.float8_e4m3fn),    # two K steps
 ])
-def test_gemm_pert_round_model(ops, dev, M, K, N, parts, io, fmt):
+def test_gemm_pert_round_model(ops, dev, M, K, N, parts, tile, io, fmt):
     """Ragged shapes (M and N not multiples of the tile) on which the w8a16
     round-model plan (M, N >= 128) picks each register-pipelined tile,
     unsplit or split in `parts` (0: unsplit; the op allocates the
-    workspace); the bare C-ABI call (no workspace) runs the unsplit plan.
+    workspace), short K included; the bare C-ABI call (no workspace) runs the unsplit plan.
     Both against the CPU oracle; two calls of the op agree bit for bit."""
     from esimd_learning_amd import cabi
     _say(f"gemm pert round model M={M} K={K} N={N} parts={parts} {io} {fmt}")
     lib = cabi.load()
-    assert lib.cek_gemm_fp8_pert_workspace_size(M, N, K) == (parts * M * N * 4 if parts else 0)
+    need = lib.cek_gemm_fp8_pert_workspace_size(M, N, K)
+    assert need == (parts * M * N * 4 if parts else 0)
+    assert lib.cek_gemm_fp8_pert_plan(M, N, K, need) == (-1 if tile is None else 16 * TILE[tile] + max(parts, 1))
     g = torch.Generator().manual_seed(M + K + N)
     W8 = (torch.randn(N, K, generator=g) * 0.05).to(fmt)
     x = (torch.randn(M, K, generator=g) * 0.5).to(io)
