@@ -1995,14 +1995,36 @@ static int launch_a8w8(const uint8_t* a, const float* sa, const uint8_t* b, cons
 // Saves the [M, 2d] product's way to memory and back (6 M d bytes of the two
 // launches' traffic) and a launch.  Tiles whose waves can hold gate and up of
 // the same outputs (an even count of block columns): 128 x 128 (two per CU), 256
-// x 256, 128 x 256 and 256 x 128, by the round model.  CEK_ERR_UNSUPPORTED where
-// the model has the separate launches faster (64-row tiles, 256 x 192 or split K
-// fit the shape better by more than the second pass costs), below one tile, above
-// 4 GB and for K % 128.  Bound by the matrix cores from ~1000 rows on.  GEMM +
-// gelu_and_mul -> here (us, MI355X, weights from HBM, M x d x K): 2048 x 14336 x
-// 4096 228.7 -> 197.0 (2.44 PFLOP/s), 2048 x 24576 x 5120 470 -> 390, 4096 x
-// 14336 x 4096 425 -> 362, 1024 x 24576 x 3072 159 -> 129, 256 x 14336 x 4096
-// 45.1 -> 38.4, 333 x 6912 x 2560 30.1 -> 26.9, 1000 x 3072 x 1024 18.4 -> 11.9.
+// x 256 and 128 x 256 (256 x 128 was never the best).  CEK_ERR_UNSUPPORTED where
+// the separate launches are faster (64-row tiles, 256 x 192 or split K fit the
+// shape better by more than the second pass costs), below one tile, above 4 GB
+// and for K % 128.  Bound by the matrix cores from ~1000 rows on.
+// The choice: a round of workgroups takes t0 + step per 128-deep K step, t0 whole
+// in the last round, whose steps are shared with fewer others (0.6 + 0.4 of its
+// fill); t0 and step of the GLU launches (kGluOpts: the epilogue's tanh is most
+// of t0) and of the plain ones (kA8w8Fixed, kA8w8Step) fitted to 1893 shapes of M
+// = 128 .. 4096, K = 512 .. 14336, d = 128 .. 24576 with weights from HBM (7-10% and
+// 8-15% rms); a split launch takes 1.25 of the plan's estimate, gelu_and_mul 2.9 us
+// and 9.5e-7 per output, and 0.8 us are in favour of the one launch, whose eager
+// call also saves the host's time for a second.  By the plan's own t0 and step
+// the two launches were overrated: 188 of the 1087 shapes taken were slower by over
+// 3%, up to a third (M = 640, K = 5120, d = 6912 72.6 against 55.8 us); now 57 of
+// 993, and the one launch takes 0.90 of the two's time (geometric mean).
+// GEMM + gelu_and_mul -> here (us, MI355X, weights from HBM, M x d x K): 2048 x
+// 8192 x 5120 154.9 -> 130.3 (2.6 PFLOP/s), 1024 x 24576 x 3072 156 -> 143, 512 x
+// 14336 x 4096 64.1 -> 60.6, 256 x 14336 x 4096 43.6 -> 39.4, 333 x 6912 x 2560
+// 30.8 -> 29.1, 1000 x 3072 x 1024 19.9 -> 14.5.
+struct GluOpt { int cfg; double t0, step; };
+constexpr GluOpt kGluOpts[] = {{1, 6.5, 1.28}, {3, 13.6, 1.46}, {5, 9.1, 0.95}};
+constexpr double kA8w8Fixed[kA8w8Cfgs] = {3.2, 3.2, 9.4, 9.5, 6.2, 7.1, 7.1, 4.7};
+constexpr double kA8w8Step[kA8w8Cfgs] = {0.95, 1.62, 1.02, 1.40, 0.61, 0.955, 0.955, 0.57};
+
+static double a8w8_launch_us(const A8w8Opt& o, int64_t M, int64_t N, int64_t K, double t0, double step) {
+  const int64_t units = ((M + o.bm - 1) / o.bm) * ((N + o.bn - 1) / o.bn), full = units / o.slots;
+  const double f = (double)(units - full * o.slots) / (double)o.slots, steps = (double)(K / 128) * step;
+  return (double)full * (t0 + steps) + (f > 0.0 ? t0 + steps * (0.6 + 0.4 * f) : 0.0);
+}
+
 static int launch_a8w8_glu(const uint8_t* a, const float* sa, const uint8_t* b, const float* sb, void* y, int64_t M,
                            int64_t d, int64_t K, int out_dtype, hipStream_t st) {
   if (M < 0 || d < 0 || K <= 0 || K % 16 != 0) return CEK_ERR_INVALID;
@@ -2012,18 +2034,20 @@ static int launch_a8w8_glu(const uint8_t* a, const float* sa, const uint8_t* b, 
   if (out_dtype != CEK_F16 && out_dtype != CEK_BF16) return CEK_ERR_INVALID;
   if (M < 128 || d < 128 || K % 128 != 0 || !a8w8_off32(M, 2 * d, K)) return CEK_ERR_UNSUPPORTED;
   int cfg = -1;
-  double t_glu = 0, t_gemm = 0;
-  for (int c : {1, 3, 5, 6}) {
-    const A8w8Opt& o = kA8w8Opts[c];
+  double t_glu = 0, t_plan = 0;
+  for (const GluOpt& g : kGluOpts) {
+    const A8w8Opt& o = kA8w8Opts[g.cfg];
     if (M < o.bm || d < o.bn / 2) continue;
-    const double t = a8w8_round_us(o, M, (d + o.bn / 2 - 1) / (o.bn / 2) * o.bn, K, 1);
+    const double t = a8w8_launch_us(o, M, (d + o.bn / 2 - 1) / (o.bn / 2) * o.bn, K, g.t0, g.step);
     if (cfg < 0 || t < t_glu) {
       t_glu = t;
-      cfg = c;
+      cfg = g.cfg;
     }
   }
-  plan_a8w8_rounds(M, 2 * d, K, true, &t_gemm);
-  if (t_glu > t_gemm + (double)M * (double)d * 6.0 / 5.0e6 + 1.5) return CEK_ERR_UNSUPPORTED;
+  const A8w8Plan p = plan_a8w8_rounds(M, 2 * d, K, true, &t_plan);
+  const double t_gemm = p.split > 1 ? 1.25 * t_plan
+                                    : a8w8_launch_us(kA8w8Opts[p.cfg], M, 2 * d, K, kA8w8Fixed[p.cfg], kA8w8Step[p.cfg]);
+  if (t_glu > t_gemm + (double)M * (double)d * 9.5e-7 + 2.9 + 0.8) return CEK_ERR_UNSUPPORTED;
   uint16_t* yp = static_cast<uint16_t*>(y);
 #define CEK_GLU8(TY, BM, BN, WM, WN, OCC, RING, NCH)                                                          \
   do {                                                                                                        \
@@ -2035,7 +2059,6 @@ static int launch_a8w8_glu(const uint8_t* a, const float* sa, const uint8_t* b, 
   do {                                                       \
     if (cfg == 3) CEK_GLU8(TY, 256, 256, 2, 4, 1, 2, 3);     \
     else if (cfg == 5) CEK_GLU8(TY, 128, 256, 2, 4, 1, 3, 3); \
-    else if (cfg == 6) CEK_GLU8(TY, 256, 128, 2, 4, 1, 3, 3); \
     else CEK_GLU8(TY, 128, 128, 2, 2, 2, 2, 1);              \
   } while (0)
   if (out_dtype == CEK_F16) CEK_GLU8_ALL(F16);

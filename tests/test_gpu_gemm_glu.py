@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("dtype,io", [(torch.float16, 0), (torch.bfloat16, 1)])
 @pytest.mark.parametrize("M,d,K", [
     (128, 128, 128), (129, 131, 128), (300, 1001, 256), (300, 2570, 384), (700, 4099, 640), (900, 8195, 384),
-    (2048, 6912, 512), (1500, 8195, 1152),
+    (2048, 6912, 512), (1500, 8195, 1152), (261, 6620, 1152),
 ])
 def test_glu_epilogue(ops, dev, M, d, K, dtype, io):
     print(f"a8w8 glu M={M} d={d} K={K} {dtype}", flush=True)
@@ -54,3 +54,34 @@ def test_glu_declines(dev):
     assert call(127, 128, 128) == unsupported and call(128, 127, 128) == unsupported and unsupported != 0
     assert call(128, 128, 128, a=None) == invalid and call(-1, 128, 128) == invalid and invalid not in (0, unsupported)
     assert call(0, 128, 128) == 0
+
+
+def test_glu_declines_faster_pair(ops, dev):
+    """Where the GEMM (256 x 192 tiles fit) and gelu_and_mul are faster, nothing is launched."""
+    lib = cabi.load()
+    M, d, K = 640, 6912, 5120
+    y = torch.full((M, d), float("nan"), dtype=torch.float16, device=dev)
+    z, s = torch.zeros(2 * d * K, dtype=torch.uint8, device=dev), torch.zeros(2 * d, device=dev)
+    rc = lib.cek_gemm_fp8_a8w8_gelu_and_mul(cabi.ptr(z), cabi.ptr(s), cabi.ptr(z), cabi.ptr(s), cabi.ptr(y), M, d, K, 0,
+                                            cabi.stream_ptr())
+    assert rc == cabi.CEK_ERR_UNSUPPORTED and y.isnan().all()
+
+
+@pytest.mark.parametrize("shared", ["a", "b", "a_scale"])
+def test_glu_output_over_operand(ops, dev, shared):
+    """An output that shares memory with an operand: the op keeps the two
+    launches, whose first has read the operands before the second writes."""
+    M, d, K = 700, 4099, 640
+    print(f"a8w8 glu output over {shared}", flush=True)
+    W8, sw = synthetic.weight_fp8(2 * d, K, seed=5)
+    a, sa = synthetic.quantize_rows(synthetic.activations(M, K, seed=6).float())
+    t = {"a": a.view(torch.uint8), "b": W8.view(torch.uint8), "a_scale": sa, "b_scale": sw.float()}
+    t = {k: v.to(dev) for k, v in t.items()}
+    want = torch.empty(M, d, dtype=torch.float16, device=dev)
+    ops.esimd_gemm_fp8_a8w8_gelu_and_mul(t["a"], t["a_scale"], t["b"], t["b_scale"], want)
+    nbytes = t[shared].numel() * t[shared].element_size()
+    buf = torch.empty(max(M * d * 2, nbytes), dtype=torch.uint8, device=dev)
+    t[shared] = buf[:nbytes].view(t[shared].dtype).view(t[shared].shape).copy_(t[shared])
+    got = buf[:M * d * 2].view(torch.float16).view(M, d)
+    ops.esimd_gemm_fp8_a8w8_gelu_and_mul(t["a"], t["a_scale"], t["b"], t["b_scale"], got)
+    assert torch.equal(got, want)
