@@ -46,19 +46,20 @@ __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_kernel(
   uint16_t* ho = hidden_out + (size_t)row * H;
   uint16_t* ro = residual_out + (size_t)row * H;
 
-  // EARLY (up to 1024 rows, where the chain of latencies is what a launch
-  // takes, and always when quantising): the norm weight's loads go out with the
-  // row's, not after the reduction (64 rows of 5120 3.9 -> 3.5 us, quantising
-  // 5.0 -> 4.3; 2048 rows of 4096 quantising 14.8 -> 13.5, but 2% slower
-  // without, which HBM bounds)
+  // EARLY (up to 512 rows of more than one unit a thread, where the chain of
+  // latencies is what a launch takes, and always when quantising): all loads, the
+  // norm weight's too, go out before the first sum (64 rows of 5120 3.35 -> 3.03
+  // us, quantising 4.46 -> 3.91; 2048 rows of 5120 quantising 17.7 -> 14.3).  Without
+  // quantising, more rows are up to 5% faster with a unit's loads beside its sum
+  // (1024 rows of 5120 6.45 against 6.78 us): other rows' waves cover them.
   u4 hv[UPT], rv[UPT], wv[UPT];
-#pragma unroll
-  for (int j = 0; j < UPT; ++j) {
-    const int u = min((int)threadIdx.x + j * NORM_THREADS, units - 1);
-    hv[j] = load_u4(hr + u * 8);
-    rv[j] = load_u4(rr + u * 8);
-  }
   if constexpr (EARLY) {
+#pragma unroll
+    for (int j = 0; j < UPT; ++j) {
+      const int u = min((int)threadIdx.x + j * NORM_THREADS, units - 1);
+      hv[j] = load_u4(hr + u * 8);
+      rv[j] = load_u4(rr + u * 8);
+    }
 #pragma unroll
     for (int j = 0; j < UPT; ++j) wv[j] = load_u4(weight + min((int)threadIdx.x + j * NORM_THREADS, units - 1) * 8);
   }
@@ -67,6 +68,10 @@ __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_kernel(
   for (int j = 0; j < UPT; ++j) {
     const int u = threadIdx.x + j * NORM_THREADS;
     if (u < units) {
+      if constexpr (!EARLY) {
+        hv[j] = load_u4(hr + u * 8);
+        rv[j] = load_u4(rr + u * 8);
+      }
       const u4 o = addnorm_pass1<T>(hv[j], rv[j], ss);
       rv[j] = o;
       *reinterpret_cast<u4*>(ro + u * 8) = o;
@@ -271,10 +276,12 @@ static int launch_norm_t(const void* hidden, const void* residual, void* hidden_
                    aligned(residual_out, 16) && (QUANT ? aligned(q, 8) : aligned(hidden_out, 16));
   const int upt = (units + NORM_THREADS - 1) / NORM_THREADS;
   dim3 grid(rows);
-#define CEK_NORM(UPT)                                                                                          \
-  do {                                                                                                         \
-    if (QUANT || rows <= 1024) add_rmsnorm_kernel<T, UPT, QUANT, true><<<grid, NORM_THREADS, 0, st>>>(h, r, ho, ro, w, H, eps, q, qs); \
-    else add_rmsnorm_kernel<T, UPT, QUANT, false><<<grid, NORM_THREADS, 0, st>>>(h, r, ho, ro, w, H, eps, q, qs);      \
+#define CEK_NORM_K(UPT, EARLY) \
+  add_rmsnorm_kernel<T, UPT, QUANT, EARLY><<<grid, NORM_THREADS, 0, st>>>(h, r, ho, ro, w, H, eps, q, qs)
+#define CEK_NORM(UPT)                                                                        \
+  do {                                                                                       \
+    if (QUANT || (UPT > 1 && rows <= 512)) CEK_NORM_K(UPT, (QUANT || UPT > 1));              \
+    else CEK_NORM_K(UPT, QUANT);                                                             \
   } while (0)
   if (vec && upt <= 1) CEK_NORM(1);
   else if (vec && upt <= 2) CEK_NORM(2);
@@ -282,6 +289,7 @@ static int launch_norm_t(const void* hidden, const void* residual, void* hidden_
   else if (vec && upt <= 4) CEK_NORM(4);
   else if (vec && upt <= 8) CEK_NORM(8);
 #undef CEK_NORM
+#undef CEK_NORM_K
   else add_rmsnorm_generic_kernel<T, QUANT><<<grid, NORM_THREADS, 0, st>>>(h, r, ho, ro, w, H, eps, q, qs);
   return check_launch();
 }

@@ -36,6 +36,18 @@ def test_norm_out_equals_in_place(ops, dev, T, H, dtype, io):
     assert torch.equal(ho, h) and torch.equal(ro, r)
 
 
+@pytest.mark.parametrize("H", [2048, 2056, 5120, 14336])
+def test_norm_few_rows_equal_many(ops, dev, H):
+    """512 rows and one more: the launches differ in when they load, not in values."""
+    print(f"norm rows H={H}", flush=True)
+    h, r = (synthetic.activations(513, H, seed=s).to(dev) for s in (1, 2))
+    w = synthetic.norm_weight(H).to(dev)
+    h1, r1 = h[:512].clone(), r[:512].clone()
+    ops.esimd_fused_add_rms_norm_batched(h, r, w, 1e-6)
+    ops.esimd_fused_add_rms_norm_batched(h1, r1, w, 1e-6)
+    assert torch.equal(h[:512], h1) and torch.equal(r[:512], r1)
+
+
 @pytest.mark.parametrize("alias", ["apart", "residual", "hidden", "half"])
 @pytest.mark.parametrize("M,N,K", [(6, 272, 1024), (100, 300, 2048), (200, 256, 4096)])
 def test_norm_gemv_beyond_four_rows(ops, dev, M, N, K, alias):
