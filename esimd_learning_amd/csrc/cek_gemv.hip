@@ -271,37 +271,33 @@ __global__ __launch_bounds__(256) void gemv_dot_kernel(const uint16_t* __restric
 // ---------------------------------------------------------------------------
 // Wave 0's output scales of the LDS-staged kernels: sc_n[t] (raw bits) for
 // column n0 + SH t + (lane & 15) (SH = 16 or 12 rows per MFMA tile; lanes past
-// SH repeat the tile's last row), sc_m[b][v] for row 16 b + 4 (lane >> 4) + v
+// SH repeat the tile's last row), sc_m[v] for row 4 (lane >> 4) + v
 // (xs: per-row activation scales, or null).  Loaded at the start of the
 // kernel so that their latency overlaps the weight loads'.
-template <int NT, int MB, int SH = 16>
-__device__ inline void lds_load_scales(uint32_t (&sc_n)[NT], float (&sc_m)[MB][4], int wave, int lane, int n0, int N,
+template <int NT, int SH = 16>
+__device__ inline void lds_load_scales(uint32_t (&sc_n)[NT], float (&sc_m)[4], int wave, int lane, int n0, int N,
                                        int M, const SegRef& sr, int skind, const float* xs) {
   const int n16 = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int t = 0; t < NT; ++t)
     sc_n[t] = wave == 0 ? load_scale_bits(sr.s, skind, min(n0 + t * SH + min(n16, SH - 1), N - 1)) : 0u;
 #pragma unroll
-  for (int b = 0; b < MB; ++b)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) sc_m[b][v] = (xs && wave == 0) ? xs[min(b * 16 + g * 4 + v, M - 1)] : 1.f;
+  for (int v = 0; v < 4; ++v) sc_m[v] = (xs && wave == 0) ? xs[min(g * 4 + v, M - 1)] : 1.f;
 }
 
 // COH: the outputs are stored at device scope (global_store ... sc1: written
 // through to the level every XCD sees), for a tail epilogue that another
 // workgroup runs on them.  SH: rows per MFMA tile (16, or 12 with operand
 // columns 12-15 repeating row 11, which are not stored).
-template <int NT, int MB, bool COH = false, int SH = 16>
-__device__ inline void lds_reduce_store(f4 (&acc)[NT][MB], uint8_t* smem, int wave, int lane, int n0, int N,
+template <int NT, bool COH = false, int SH = 16>
+__device__ inline void lds_reduce_store(f4 (&acc)[NT], uint8_t* smem, int wave, int lane, int n0, int N,
                                         int M, const SegRef& sr, int skind, const uint32_t (&sc_n)[NT],
-                                        const float (&sc_m)[MB][4], bool xscaled, bool bf16_out) {
-  f4* red = reinterpret_cast<f4*>(smem);  // [3][NT][MB][64]
+                                        const float (&sc_m)[4], bool xscaled, bool bf16_out) {
+  f4* red = reinterpret_cast<f4*>(smem);  // [3][NT][64]
   __syncthreads();                         // every wave is done with the stages
   if (wave > 0) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int b = 0; b < MB; ++b) red[(((wave - 1) * NT + t) * MB + b) * 64 + lane] = acc[t][b];
+    for (int t = 0; t < NT; ++t) red[((wave - 1) * NT + t) * 64 + lane] = acc[t];
   }
   __syncthreads();
   if (wave != 0) return;
@@ -311,20 +307,17 @@ __device__ inline void lds_reduce_store(f4 (&acc)[NT][MB], uint8_t* smem, int wa
     const int n = n0 + t * SH + n16;  // D column = lane & 15
     if (n >= N || n16 >= SH) continue;
     const float sc = scale_value(sc_n[t], skind);
+    f4 c = acc[t];
 #pragma unroll
-    for (int b = 0; b < MB; ++b) {
-      f4 c = acc[t][b];
+    for (int w = 0; w < 3; ++w) c += red[(w * NT + t) * 64 + lane];
 #pragma unroll
-      for (int w = 0; w < 3; ++w) c += red[((w * NT + t) * MB + b) * 64 + lane];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int m = b * 16 + g * 4 + v;  // D row = 4 * (lane >> 4) + v
-        if (m >= M) continue;
-        const float o = f32_round(c[v] * (xscaled ? sc * sc_m[b][v] : sc));
-        const uint16_t ob = bf16_out ? BF16::from_f32(o) : F16::from_f32(o);
-        if constexpr (COH) __hip_atomic_store(sr.y + (size_t)m * N + n, ob, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        else sr.y[(size_t)m * N + n] = ob;
-      }
+    for (int v = 0; v < 4; ++v) {
+      const int m = g * 4 + v;  // D row = 4 * (lane >> 4) + v
+      if (m >= M) continue;
+      const float o = f32_round(c[v] * (xscaled ? sc * sc_m[v] : sc));
+      const uint16_t ob = bf16_out ? BF16::from_f32(o) : F16::from_f32(o);
+      if constexpr (COH) __hip_atomic_store(sr.y + (size_t)m * N + n, ob, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      else sr.y[(size_t)m * N + n] = ob;
     }
   }
 }
@@ -381,50 +374,45 @@ __device__ inline void lds_reduce_addnorm(const f4& acc, uint8_t* smem, int wave
 }
 
 // The cross-wave sum of one tile of a multi-tile workgroup, in a reduction
-// area of its own (red, 3 x NT x MB x 64 f4), with LDS-only barriers so that
+// area of its own (red, 3 x NT x 64 f4), with LDS-only barriers so that
 // the next tile's loads stay in flight, and no early return.  The leading
 // barrier also orders this tile's reduction writes after wave 0's reads of
-// the previous tile's.  Wave 0 then calls emit(t, b, v, o) for every element
-// of its fragments: o = the scaled sum of D row 16 b + 4 (lane >> 4) + v,
+// the previous tile's.  Wave 0 then calls emit(t, v, o) for every element
+// of its fragments: o = the scaled sum of D row 4 (lane >> 4) + v,
 // column 16 t + (lane & 15) of the tile (rows and columns not yet bounded).
-template <int NT, int MB, typename Emit>
-__device__ inline void lds_reduce_tile(const f4 (&acc)[NT][MB], uint8_t* redp, int wave, int lane, int skind,
-                                       const uint32_t (&sc_n)[NT], const float (&sc_m)[MB][4], bool xscaled,
+template <int NT, typename Emit>
+__device__ inline void lds_reduce_tile(const f4 (&acc)[NT], uint8_t* redp, int wave, int lane, int skind,
+                                       const uint32_t (&sc_n)[NT], const float (&sc_m)[4], bool xscaled,
                                        Emit&& emit) {
-  f4* red = reinterpret_cast<f4*>(redp);  // [3][NT][MB][64]
+  f4* red = reinterpret_cast<f4*>(redp);  // [3][NT][64]
   lds_barrier();
   if (wave > 0) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int b = 0; b < MB; ++b) red[(((wave - 1) * NT + t) * MB + b) * 64 + lane] = acc[t][b];
+    for (int t = 0; t < NT; ++t) red[((wave - 1) * NT + t) * 64 + lane] = acc[t];
   }
   lds_barrier();
   if (wave == 0) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const float sc = scale_value(sc_n[t], skind);
+      f4 c = acc[t];
 #pragma unroll
-      for (int b = 0; b < MB; ++b) {
-        f4 c = acc[t][b];
+      for (int w = 0; w < 3; ++w) c += red[(w * NT + t) * 64 + lane];
 #pragma unroll
-        for (int w = 0; w < 3; ++w) c += red[((w * NT + t) * MB + b) * 64 + lane];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) emit(t, b, v, f32_round(c[v] * (xscaled ? sc * sc_m[b][v] : sc)));
-      }
+      for (int v = 0; v < 4; ++v) emit(t, v, f32_round(c[v] * (xscaled ? sc * sc_m[v] : sc)));
     }
   }
 }
 
 // lds_reduce_store for one tile of a multi-tile workgroup (n0 = the tile's
 // first row).
-template <int NT, int MB, int SH = 16>
-__device__ inline void lds_reduce_store_tile(const f4 (&acc)[NT][MB], uint8_t* redp, int wave, int lane, int n0, int N,
+template <int NT, int SH = 16>
+__device__ inline void lds_reduce_store_tile(const f4 (&acc)[NT], uint8_t* redp, int wave, int lane, int n0, int N,
                                              int M, const SegRef& sr, int skind, const uint32_t (&sc_n)[NT],
-                                             const float (&sc_m)[MB][4], bool xscaled, bool bf16_out) {
+                                             const float (&sc_m)[4], bool xscaled, bool bf16_out) {
   const int n16 = lane & 15, g = lane >> 4;
-  lds_reduce_tile<NT, MB>(acc, redp, wave, lane, skind, sc_n, sc_m, xscaled, [&](int t, int b, int v, float o) {
-    const int n = n0 + t * SH + n16, m = b * 16 + g * 4 + v;  // D column = lane & 15, row = 4 (lane >> 4) + v
+  lds_reduce_tile<NT>(acc, redp, wave, lane, skind, sc_n, sc_m, xscaled, [&](int t, int v, float o) {
+    const int n = n0 + t * SH + n16, m = g * 4 + v;  // D column = lane & 15, row = 4 (lane >> 4) + v
     if (n < N && n16 < SH && m < M) sr.y[(size_t)m * N + n] = bf16_out ? BF16::from_f32(o) : F16::from_f32(o);
   });
 }
@@ -582,25 +570,25 @@ __device__ void gemv_tail(const TailArgs& ta, uint16_t* y, int n0, int N, int M,
 // same rule: fp16 / bf16 activations and M <= 4 (launch_lds_steps).  The
 // runtime chunk offsets cost VALU address arithmetic, which made the
 // multi-tile and M > 4 forms 1-5% slower with it.
-template <typename T, typename TO, int FMT, bool XF8, int NT, int MB, int D, int STEPS, int MX = 0, int TPW = 1,
+template <typename T, typename TO, int FMT, bool XF8, int NT, int D, int STEPS, int MX = 0, int TPW = 1,
           bool GLU = false, bool NORM = false, int TAIL = TAIL_NONE, int TP = 0, bool ROT = false, int EPI = EPI_NONE,
           bool R12 = false>
 __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs sg, int skind, int M, NormArgs na) {
   constexpr bool PROD = EPI == EPI_ADDNORM || EPI == EPI_ADDNORM12;  // deferred-norm producer
-  static_assert(!PROD || (TPW == 1 && NT == 1 && MB == 1 && !GLU && !NORM && TAIL == TAIL_NONE && !XF8 &&
+  static_assert(!PROD || (TPW == 1 && NT == 1 && !GLU && !NORM && TAIL == TAIL_NONE && !XF8 &&
                                        std::is_same<T, TO>::value),
                 "deferred norm producer: one 16- or 12-row tile, fp16 / bf16");
-  static_assert(EPI != EPI_ROWSCALE || (MB == 1 && !NORM && !XF8), "deferred norm consumer: fp16 / bf16, M <= 16");
+  static_assert(EPI != EPI_ROWSCALE || (!NORM && !XF8), "deferred norm consumer: fp16 / bf16, M <= 16");
   static_assert(EPI != EPI_ROWSCALE || STEPS >= 2, "deferred norm consumer: row scales at stage 1, before tile 0 ends");
   constexpr int NS = STEPS * TPW;  // stages of the workgroup
   static_assert(D >= 1 && D <= NS, "prefetch depth");
-  static_assert(MX == 0 || (MB == 1 && MX <= 16), "activations go through LDS only for M <= 16");
+  static_assert(MX <= 16, "one block of activation rows");
   static_assert(!GLU || (TPW == 2 && NT == 1), "gate/up pairs are two 16-row tiles");
   static_assert(!NORM || (MX >= 1 && MX <= 4 && NT == 1), "fused norm: up to four rows");
-  static_assert(TAIL == TAIL_NONE || (TPW == 1 && NT == 1 && MB == 1 && !GLU && !NORM && !XF8 &&
+  static_assert(TAIL == TAIL_NONE || (TPW == 1 && NT == 1 && !GLU && !NORM && !XF8 &&
                                       std::is_same<T, TO>::value),
                 "tails: one 16-row tile per workgroup, fp16 / bf16 activations");
-  static_assert(!R12 || (NT <= 2 && MB == 1 && !GLU && !NORM && TAIL == TAIL_NONE && !ROT && EPI == EPI_NONE),
+  static_assert(!R12 || (NT <= 2 && !GLU && !NORM && TAIL == TAIL_NONE && !ROT && EPI == EPI_NONE),
                 "12-row plain tiles: one or two tiles wide, no K rotation (so each output's sum order is the 16-row "
                 "form's)");
   constexpr int K = STEPS * 1024;
@@ -621,7 +609,7 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs 
   // STEPS stages); (TPW > 1) the cross-wave reduction area; (NORM) the
   // norm's per-row partial sums and maxima
   constexpr int XAREA = NORM ? STEPS * XSTAGE : 2 * XSTAGE;
-  constexpr int RED = TPW > 1 ? 3 * NT * MB * 64 * 16 : 0;
+  constexpr int RED = TPW > 1 ? 3 * NT * 64 * 16 : 0;
   constexpr int NSH = NORM ? 2 * 4 * MX * 4 : 0;
   __shared__ __align__(16) uint8_t smem[2 * STAGE + XAREA + RED + NSH];
   const SegRef sr = find_seg(sg, blockIdx.x);
@@ -644,8 +632,8 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs 
     }
   };
   uint32_t sc_n[NT];
-  float sc_m[MB][4];
-  lds_load_scales<NT, MB, SH>(sc_n, sc_m, wave, lane, nw, N, M, sr, skind, XF8 && !NORM ? sg.xs : nullptr);
+  float sc_m[4];
+  lds_load_scales<NT, SH>(sc_n, sc_m, wave, lane, nw, N, M, sr, skind, XF8 && !NORM ? sg.xs : nullptr);
   // this wave loads rows wave + 4 j of every stage of tile t: row
   // tile_row(t) + wave + 4 j, clamped into the tile's matrix (clamped rows are
   // never stored)
@@ -654,10 +642,8 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs 
     const int row = GLU ? t * half + min(nw + r, half - 1) : min(nw + ROWS * t + r, N - 1);
     return sr.w + (size_t)row * K + 16 * (lane ^ (r & 15));
   };
-  const uint8_t* gx[MB];
-#pragma unroll
-  for (int b = 0; b < MB; ++b)  // rows >= M are never stored
-    gx[b] = static_cast<const uint8_t*>(xv) + (size_t)min(16 * b + n16, M - 1) * K * XB;
+  // (rows >= M are never stored)
+  const uint8_t* gx = static_cast<const uint8_t*>(xv) + (size_t)min(n16, M - 1) * K * XB;
   // MX > 0: thread t's units t + 256 j of the MX x XROW stage: row, 16-byte chunk
   const uint8_t* gxu[XU];
   int xdst[XU];
@@ -673,8 +659,8 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs 
   auto unit = [&](int q) { return XF8 ? 2 * (4 * (wave + 4 * q) + g) : 4 * (wave + 4 * q) + g; };
 
   u4 wr[S][LW];
-  u4 xr[S][MX > 0 ? XU : QN][MX > 0 ? 1 : MB][MX > 0 ? 1 : 2];
-  auto issue = [&](int i, u4 (&ws)[LW], u4 (&xs)[MX > 0 ? XU : QN][MX > 0 ? 1 : MB][MX > 0 ? 1 : 2]) {
+  u4 xr[S][MX > 0 ? XU : QN][MX > 0 ? 1 : 2];
+  auto issue = [&](int i, u4 (&ws)[LW], u4 (&xs)[MX > 0 ? XU : QN][MX > 0 ? 1 : 2]) {
     const int k0 = kchunk(i) << 10;
 #pragma unroll
     for (int j = 0; j < LW; ++j) ws[j] = load_u4_stream(wrow(i / STEPS, j) + k0);  // 1 KB of one row per instruction
@@ -683,26 +669,22 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs 
       (void)xs;  // activations are resident in LDS
     } else if constexpr (MX > 0) {
 #pragma unroll
-      for (int j = 0; j < XU; ++j) xs[j][0][0] = load_u4(gxu[j] + (size_t)k0 * XB);
+      for (int j = 0; j < XU; ++j) xs[j][0] = load_u4(gxu[j] + (size_t)k0 * XB);
     } else {
 #pragma unroll
-      for (int q = 0; q < QN; ++q)
-#pragma unroll
-        for (int b = 0; b < MB; ++b) {
-          const u4* p = reinterpret_cast<const u4*>(gx[b] + (size_t)(k0 + 16 * unit(q)) * XB);
-          xs[q][b][0] = p[0];
-          xs[q][b][1] = p[1];
-        }
+      for (int q = 0; q < QN; ++q) {
+        const u4* p = reinterpret_cast<const u4*>(gx + (size_t)(k0 + 16 * unit(q)) * XB);
+        xs[q][0] = p[0];
+        xs[q][1] = p[1];
+      }
     }
     asm volatile("" ::: "memory");
   };
 
-  f4 acc[NT][MB];
+  f4 acc[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int b = 0; b < MB; ++b) acc[t][b] = f4{0.f, 0.f, 0.f, 0.f};
-  [[maybe_unused]] float gate[MB][4];  // GLU: wave 0's rounded gate values (D layout)
+  for (int t = 0; t < NT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+  [[maybe_unused]] float gate[4];  // GLU: wave 0's rounded gate values (D layout)
 
   // NORM: thread t's 8-element units t + 256 j of every row (add_rmsnorm_kernel's
   // layout), rows >= M repeating row M - 1 and units past the row repeating
@@ -773,17 +755,17 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs 
     }
     asm volatile("" ::: "memory");  // before the weight prologue
   }
-  // EPI_ROWSCALE: wave 0's epilogue row scales, sc_m[0][v] = inv of row 4 (lane >> 4) + v
+  // EPI_ROWSCALE: wave 0's epilogue row scales, sc_m[v] = inv of row 4 (lane >> 4) + v
   auto pick_rs = [&]() {
     if constexpr (EPI == EPI_ROWSCALE) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int m = min(g * 4 + v, 3);
-        sc_m[0][v] = m == 0 ? rinv[0] : (m == 1 ? rinv[1] : (m == 2 ? rinv[2] : rinv[3]));
+        sc_m[v] = m == 0 ? rinv[0] : (m == 1 ? rinv[1] : (m == 2 ? rinv[2] : rinv[3]));
       }
     }
   };
-  // NORM + XF8: wave 0's epilogue row scales, sc_m[0][v] for row 4 (lane >> 4) + v
+  // NORM + XF8: wave 0's epilogue row scales, sc_m[v] for row 4 (lane >> 4) + v
   auto pick_row_scales = [&]() {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -791,7 +773,7 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs 
       float pick = rsc[0];
 #pragma unroll
       for (int mm = 1; mm < NR; ++mm) pick = m == mm ? rsc[mm] : pick;
-      sc_m[0][v] = pick;
+      sc_m[v] = pick;
     }
   };
 
@@ -968,7 +950,7 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs 
     for (int jj = 0; jj < LW; ++jj) *reinterpret_cast<u4*>(sw + (wave + 4 * jj) * 1024 + 16 * lane) = wr[i % S][jj];
     if constexpr (MX > 0 && !NORM) {
 #pragma unroll
-      for (int j = 0; j < XU; ++j) *reinterpret_cast<u4*>(sx + xdst[j]) = xr[i % S][j][0][0];
+      for (int j = 0; j < XU; ++j) *reinterpret_cast<u4*>(sx + xdst[j]) = xr[i % S][j][0];
     }
     lds_barrier();
     if (i + D < NS) issue(i + D, wr[(i + D) % S], xr[(i + D) % S]);
@@ -991,23 +973,17 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs 
         if constexpr (XF8) {
           const i8 bf = cat_i8(*reinterpret_cast<const u4*>(rw + 16 * (v ^ (rr & 15))),
                                *reinterpret_cast<const u4*>(rw + 16 * ((v + 1) ^ (rr & 15))));
-#pragma unroll
-          for (int b = 0; b < MB; ++b) {
-            if constexpr (MX > 0) acc[t][b] = mfma_fp8_16x16x128(cat_i8(xa0, xa1), bf, acc[t][b]);
-            else acc[t][b] = mfma_fp8_16x16x128(cat_i8(xr[i % S][q][b][0], xr[i % S][q][b][1]), bf, acc[t][b]);
-          }
+          if constexpr (MX > 0) acc[t] = mfma_fp8_16x16x128(cat_i8(xa0, xa1), bf, acc[t]);
+          else acc[t] = mfma_fp8_16x16x128(cat_i8(xr[i % S][q][0], xr[i % S][q][1]), bf, acc[t]);
         } else {
           u4 lo, hi;
           decode16<T, FMT>(*reinterpret_cast<const u4*>(rw + 16 * (v ^ (rr & 15))), lo, hi);
-#pragma unroll
-          for (int b = 0; b < MB; ++b) {
-            if constexpr (MX > 0) {
-              acc[t][b] = mfma16x16x32<T>(xa0, lo, acc[t][b]);
-              acc[t][b] = mfma16x16x32<T>(xa1, hi, acc[t][b]);
-            } else {
-              acc[t][b] = mfma16x16x32<T>(xr[i % S][q][b][0], lo, acc[t][b]);
-              acc[t][b] = mfma16x16x32<T>(xr[i % S][q][b][1], hi, acc[t][b]);
-            }
+          if constexpr (MX > 0) {
+            acc[t] = mfma16x16x32<T>(xa0, lo, acc[t]);
+            acc[t] = mfma16x16x32<T>(xa1, hi, acc[t]);
+          } else {
+            acc[t] = mfma16x16x32<T>(xr[i % S][q][0], lo, acc[t]);
+            acc[t] = mfma16x16x32<T>(xr[i % S][q][1], hi, acc[t]);
           }
         }
       }
@@ -1017,28 +993,26 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs 
         uint8_t* redp = smem + 2 * STAGE + XAREA;
         if constexpr (GLU) {
           if (i / STEPS == 0) {  // gate tile: keep the rounded values
-            lds_reduce_tile<NT, MB>(acc, redp, wave, lane, skind, sc_n, sc_m, XF8 || EPI == EPI_ROWSCALE,
-                                    [&](int, int b, int v, float o) { gate[b][v] = TO::to_f32(TO::from_f32(o)); });
+            lds_reduce_tile<NT>(acc, redp, wave, lane, skind, sc_n, sc_m, XF8 || EPI == EPI_ROWSCALE,
+                                [&](int, int v, float o) { gate[v] = TO::to_f32(TO::from_f32(o)); });
           } else {  // up tile: gelu_and_mul and the store
-            lds_reduce_tile<NT, MB>(acc, redp, wave, lane, skind, sc_n, sc_m, XF8 || EPI == EPI_ROWSCALE,
-                                    [&](int, int b, int v, float o) {
-              const int n = nw + n16, m = b * 16 + g * 4 + v;
+            lds_reduce_tile<NT>(acc, redp, wave, lane, skind, sc_n, sc_m, XF8 || EPI == EPI_ROWSCALE,
+                                [&](int, int v, float o) {
+              const int n = nw + n16, m = g * 4 + v;
               if (n < half && m < M)
                 sr.y[(size_t)m * half + n] =
-                    TO::from_f32(f32_round(gelu_tanh(gate[b][v]) * TO::to_f32(TO::from_f32(o))));
+                    TO::from_f32(f32_round(gelu_tanh(gate[v]) * TO::to_f32(TO::from_f32(o))));
             });
           }
         } else {
-          lds_reduce_store_tile<NT, MB, SH>(acc, redp, wave, lane, tile_row(i / STEPS), N, M, sr, skind, sc_n, sc_m,
-                                            XF8 || EPI == EPI_ROWSCALE, std::is_same<TO, BF16>::value);
+          lds_reduce_store_tile<NT, SH>(acc, redp, wave, lane, tile_row(i / STEPS), N, M, sr, skind, sc_n, sc_m,
+                                        XF8 || EPI == EPI_ROWSCALE, std::is_same<TO, BF16>::value);
         }
         if (i + 1 < NS) {
 #pragma unroll
-          for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int b = 0; b < MB; ++b) acc[t][b] = f4{0.f, 0.f, 0.f, 0.f};
-          lds_load_scales<NT, MB, SH>(sc_n, sc_m, wave, lane, tile_row(i / STEPS + 1), N, M, sr, skind,
-                                      XF8 && !NORM ? sg.xs : nullptr);
+          for (int t = 0; t < NT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+          lds_load_scales<NT, SH>(sc_n, sc_m, wave, lane, tile_row(i / STEPS + 1), N, M, sr, skind,
+                                  XF8 && !NORM ? sg.xs : nullptr);
           if constexpr (NORM && XF8) pick_row_scales();
           pick_rs();
         }
@@ -1046,10 +1020,10 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(const void* xv, GemvSegs 
     }
   }
   if constexpr (PROD)
-    lds_reduce_addnorm<T, ROWS>(acc[0][0], smem, wave, lane, nw, N, M, sr, skind, sc_n[0], na, pres, pnw);
+    lds_reduce_addnorm<T, ROWS>(acc[0], smem, wave, lane, nw, N, M, sr, skind, sc_n[0], na, pres, pnw);
   else if constexpr (TPW == 1)
-    lds_reduce_store<NT, MB, TAIL != TAIL_NONE, SH>(acc, smem, wave, lane, nw, N, M, sr, skind, sc_n, sc_m,
-                                                    XF8 || EPI == EPI_ROWSCALE, std::is_same<TO, BF16>::value);
+    lds_reduce_store<NT, TAIL != TAIL_NONE, SH>(acc, smem, wave, lane, nw, N, M, sr, skind, sc_n, sc_m,
+                                                XF8 || EPI == EPI_ROWSCALE, std::is_same<TO, BF16>::value);
   if constexpr (TAIL != TAIL_NONE) gemv_tail<T, TAIL, TP>(na.tail, sr.y, nw, N, M, smem, rcs, rsn);
 }
 
@@ -1221,18 +1195,18 @@ __global__ __launch_bounds__(256) void gemv_generic_kernel(const uint16_t* __res
 // kernel.  Requires 16-byte aligned x and weights.
 template <typename T, typename TO, int FMT, bool XF8, int S>
 static bool launch_lds_steps(const void* x, GemvSegs& sg, int skind, int M, int N, hipStream_t st) {
-#define CEK_LDS(NT, MB, D) \
-  gemv_lds_kernel<T, TO, FMT, XF8, NT, MB, D, S><<<dim3(seg_grid(sg, 16 * (NT))), 256, 0, st>>>(x, sg, skind, M, NormArgs{})
+#define CEK_LDS(NT, D) \
+  gemv_lds_kernel<T, TO, FMT, XF8, NT, D, S><<<dim3(seg_grid(sg, 16 * (NT))), 256, 0, st>>>(x, sg, skind, M, NormArgs{})
 #define CEK_LDS_T(NT, D, MX, TPW, ROT)                                                                         \
-  gemv_lds_kernel<T, TO, FMT, XF8, NT, 1, D, S, MX, TPW, false, false, TAIL_NONE, 0, ROT>                     \
+  gemv_lds_kernel<T, TO, FMT, XF8, NT, D, S, MX, TPW, false, false, TAIL_NONE, 0, ROT>                     \
       <<<dim3(seg_grid(sg, 16 * (NT) * (TPW))), 256, 0, st>>>(x, sg, skind, M, NormArgs{})
   constexpr bool SHORT = S >= 3 && S <= 5;
   constexpr bool MULTI = S == 4 || S == 5;  // multi-tile workgroups (K = 4096, 5120)
 #define CEK_LDS_T12(D, MX, TPW)                                                                          \
-  gemv_lds_kernel<T, TO, FMT, XF8, 1, 1, D, S, MX, TPW, false, false, TAIL_NONE, 0, false, EPI_NONE, true> \
+  gemv_lds_kernel<T, TO, FMT, XF8, 1, D, S, MX, TPW, false, false, TAIL_NONE, 0, false, EPI_NONE, true> \
       <<<dim3(seg_grid(sg, 12 * (TPW))), 256, 0, st>>>(x, sg, skind, M, NormArgs{})
 #define CEK_LDS_24(D)                                                                                   \
-  gemv_lds_kernel<T, TO, FMT, XF8, 2, 1, D, S, 0, 1, false, false, TAIL_NONE, 0, false, EPI_NONE, true> \
+  gemv_lds_kernel<T, TO, FMT, XF8, 2, D, S, 0, 1, false, false, TAIL_NONE, 0, false, EPI_NONE, true> \
       <<<dim3(seg_grid(sg, 24)), 256, 0, st>>>(x, sg, skind, M, NormArgs{})
 #define CEK_LDS_TPW(NT, D, MX, ROT)                                  \
   do {                                                               \
@@ -1355,17 +1329,17 @@ static bool launch_lds_steps(const void* x, GemvSegs& sg, int skind, int M, int 
       // (fp16 / bf16 M <= 4 took the staged form above)
       if ((N + 15) / 16 > kCUs && (XF8 ? M > 8 : M >= 8)) {
         if (n24) CEK_LDS_24(2);
-        else CEK_LDS(2, 1, 2);
+        else CEK_LDS(2, 2);
       } else {
         CEK_LDS_TPW(1, 3, 0, false);
       }
     } else if constexpr (XF8 && S >= 3) {
-      CEK_LDS(1, 1, 3);
+      CEK_LDS(1, 3);
     } else if constexpr (!XF8) {
       if (M <= 4) CEK_LDS_T(1, 2, 0, 1, true);  // fp16 / bf16 M <= 4 rotate in every form
-      else CEK_LDS(1, 1, 2);
+      else CEK_LDS(1, 2);
     } else {
-      CEK_LDS(1, 1, 2);
+      CEK_LDS(1, 2);
     }
     return true;
   }
@@ -1407,11 +1381,11 @@ static void launch_glu_steps(const void* x, GemvSegs& sg, int skind, int M, int 
   sg.gstart[0] = 0;
   for (int i = 1; i <= MAX_SEGS; ++i) sg.gstart[i] = grid;
 #define CEK_GLU(D, MX, ROT)                                                                   \
-  gemv_lds_kernel<T, TO, FMT, XF8, 1, 1, D, S, MX, 2, true, false, TAIL_NONE, 0, ROT><<<dim3(grid), 256, 0, st>>>( \
+  gemv_lds_kernel<T, TO, FMT, XF8, 1, D, S, MX, 2, true, false, TAIL_NONE, 0, ROT><<<dim3(grid), 256, 0, st>>>( \
       x, sg, skind, M, NormArgs{})
   if constexpr (!XF8 && FMT == CEK_E4M3) {
     if (rs) {  // deferred RMSNorm consumer (M <= 4, checked by the caller)
-      gemv_lds_kernel<T, TO, FMT, XF8, 1, 1, 3, S, 4, 2, true, false, TAIL_NONE, 0, true, EPI_ROWSCALE>
+      gemv_lds_kernel<T, TO, FMT, XF8, 1, 3, S, 4, 2, true, false, TAIL_NONE, 0, true, EPI_ROWSCALE>
           <<<dim3(grid), 256, 0, st>>>(x, sg, skind, M, *rs);
       return;
     }
@@ -1452,18 +1426,18 @@ static void launch_norm_steps(GemvSegs& sg, const NormArgs& na, int skind, int M
     const int grid = (N / 2 + 15) / 16;
     sg.gstart[0] = 0;
     for (int i = 1; i <= MAX_SEGS; ++i) sg.gstart[i] = grid;
-    gemv_lds_kernel<T, TO, CEK_E4M3, XF8, 1, 1, 3, S, MX, 2, true, true, TAIL_NONE, 0, !XF8>
+    gemv_lds_kernel<T, TO, CEK_E4M3, XF8, 1, 3, S, MX, 2, true, true, TAIL_NONE, 0, !XF8>
         <<<dim3(grid), 256, 0, st>>>(nullptr, sg, skind, M, na);
     return;
   }
   if constexpr (S == 4 || S == 5) {
     if ((N + 15) / 16 >= 384) {
-      gemv_lds_kernel<T, TO, CEK_E4M3, XF8, 1, 1, 3, S, MX, 2, false, true, TAIL_NONE, 0, !XF8>
+      gemv_lds_kernel<T, TO, CEK_E4M3, XF8, 1, 3, S, MX, 2, false, true, TAIL_NONE, 0, !XF8>
           <<<dim3(seg_grid(sg, 32)), 256, 0, st>>>(nullptr, sg, skind, M, na);
       return;
     }
   }
-  gemv_lds_kernel<T, TO, CEK_E4M3, XF8, 1, 1, 3, S, MX, 1, false, true, TAIL_NONE, 0, !XF8>
+  gemv_lds_kernel<T, TO, CEK_E4M3, XF8, 1, 3, S, MX, 1, false, true, TAIL_NONE, 0, !XF8>
       <<<dim3(seg_grid(sg, 16)), 256, 0, st>>>(nullptr, sg, skind, M, na);
 }
 
@@ -1820,7 +1794,7 @@ template <typename T, int TAIL, int TP, int EPI = EPI_NONE>
 static void launch_tail_t(const void* x, GemvSegs& sg, int skind, int M, int K, const NormArgs& na, hipStream_t st) {
   const dim3 grid((unsigned)seg_grid(sg, 16));
 #define CEK_TAIL(S)                                                                                       \
-  gemv_lds_kernel<T, T, CEK_E4M3, false, 1, 1, 3, S, 4, 1, false, false, TAIL, TP, true, EPI><<<grid, 256, 0, st>>>( \
+  gemv_lds_kernel<T, T, CEK_E4M3, false, 1, 3, S, 4, 1, false, false, TAIL, TP, true, EPI><<<grid, 256, 0, st>>>( \
       x, sg, skind, M, na)
   if (K == 3072) CEK_TAIL(3);
   else if (K == 4096) CEK_TAIL(4);
@@ -1885,7 +1859,7 @@ int launch_gemv_tail(const void* x, const void* w, const void* scale, int skind,
 // KiB values.
 template <typename T, int EPI, int S>
 static void launch_defer_t(const void* x, GemvSegs& sg, int skind, int M, const NormArgs& na, hipStream_t st) {
-  gemv_lds_kernel<T, T, CEK_E4M3, false, 1, 1, (S >= 3 ? 3 : 2), S, 4, 1, false, false, TAIL_NONE, 0, true, EPI>
+  gemv_lds_kernel<T, T, CEK_E4M3, false, 1, (S >= 3 ? 3 : 2), S, 4, 1, false, false, TAIL_NONE, 0, true, EPI>
       <<<dim3(seg_grid(sg, EPI == EPI_ADDNORM12 ? 12 : 16)), 256, 0, st>>>(x, sg, skind, M, na);
 }
 
