@@ -13,7 +13,12 @@
 // Eight consumer waves each take an eighth of a stage's K values over all MB x
 // NT 16 x 16 blocks (every LDS byte is read once) and meet in LDS at the end;
 // their only memory operations in the loop are LDS reads.  One barrier per
-// stage.  What a launch takes is about 4.8 us (the launch, the first bytes,
+// stage.  e4m3 activations: up to 16 rows decoded to fp16 like the weights
+// (both exactly) and multiplied there, since the fp8 MFMA's sums are not
+// rounded as fp32 ones are: 1.5e-5 of the result (2-norm; 6.7% of the fp16
+// outputs differ from the correctly rounded product) against 1e-7 (0.1%); above
+// 16 rows by the fp8 MFMA, as in every other kernel for them.  What a launch
+// takes is about 4.8 us (the launch, the first bytes,
 // the stages' barriers, the epilogue) plus a CU's bytes at 90 per ns for the
 // activations and 25-30 for the weights.  Measured on MI355X, weights from
 // HBM, against the kernels that served these shapes before (us): M = 48, K =
@@ -191,9 +196,16 @@ void stream_kernel(const uint8_t* __restrict__ x, GemvSegs sg, int skind, int M,
         for (int b = 0; b < MB; ++b)
 #pragma unroll
           for (int u = 0; u < NU; ++u) af[b][u] = *reinterpret_cast<const u4*>(pa + ao[b][u]);
+        [[maybe_unused]] u4 alo, ahi;
+        if constexpr (XF8 && AR <= 16) decode16<F16, CEK_E4M3>(af[0][0], alo, ahi);
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-          if constexpr (XF8) {
+          if constexpr (XF8 && AR <= 16) {
+            u4 lo, hi;
+            decode16<F16, CEK_E4M3>(*reinterpret_cast<const u4*>(pw + wo[t]), lo, hi);
+            acc[0][t] = mfma16x16x32<F16>(alo, lo, acc[0][t]);
+            acc[0][t] = mfma16x16x32<F16>(ahi, hi, acc[0][t]);
+          } else if constexpr (XF8) {
             typedef long l2 __attribute__((ext_vector_type(2)));
             const l2 wv = *reinterpret_cast<const l2*>(pw + wo[t]);
 #pragma unroll

@@ -99,6 +99,22 @@ def test_stream_or_tiles(ops, dev, act, M, K, N):
         _check(y, x.double(), W8.float().double(), s.double(), K, "w8a16")
 
 
+@pytest.mark.parametrize("M", [3, 5, 16])
+@pytest.mark.parametrize("K", [320, 2560, 10240])
+def test_stream_a8w8_fp32_sums(ops, dev, M, K):
+    """Up to 16 rows of e4m3 activations are summed in fp32: an error of about
+    1e-7 of the result moves some 2 1e-7 / 2^-11 = 0.05% of the fp16 outputs to the
+    other side of a rounding boundary (the fp8 MFMA's sums move 6.7%)."""
+    N = 2050
+    print(f"stream a8w8 sums M={M} K={K}", flush=True)
+    W8, s = synthetic.weight_fp8(N, K, seed=K)
+    a8, sa = synthetic.quantize_rows(synthetic.activations(M, K, seed=M).float())
+    y = torch.empty(M, N, dtype=torch.float16, device=dev)
+    ops.esimd_gemm_fp8_a8w8(a8.to(dev), sa.to(dev), W8.to(dev), s.to(dev), y)
+    ref = (a8.float().double() @ W8.float().double().t()) * (sa[:, None] * s[None]).double()
+    assert float((y.cpu() != ref.half()).double().mean()) < 5e-3
+
+
 # Columns at which a workgroup has 8, 12, 16, 24, 32, 40, 48, 56 and 64 weight rows
 FORM_N = [1001, 2500, 3500, 5000, 6201, 8201, 11000, 12700, 16001]
 
