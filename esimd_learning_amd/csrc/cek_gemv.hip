@@ -1529,8 +1529,8 @@ int launch_norm_gemv(const NormArgs& na, const void* w, const void* scale, int s
 // 16, K = 8192, N = 8192 33.0 -> 14.8 -- but for up to four rows of a short and
 // long-K matrix, whose few workgroups each pay the stages' barriers (N = 1000,
 // K = 6144 5.3 against 5.9; N = 2048 6.6 -> 6.2, but at M = 3 K = 8192 7.0 against
-// 7.5, K = 16384 10.3 against 10.8; e4m3 activations N = 2048, K = 8192 6.6 against
-// 7.0).
+// 7.5, K = 16384 10.3 against 10.8, N = 4096 16.6 against 17.8; e4m3 activations N =
+// 2048, K = 8192 6.6 against 7.0, N = 4096, K = 16384 15.2 against 17.8).
 // K that it has (16-bit activations), 9 .. 16 rows:
 //  * 3072, 4096 and 5120, matrices above 8192 rows (M = 16, K = 4096, N = 8208
 //    12.3 -> 9.6, N = 14336 15.5 -> 13.2, N = 28672 26.5 -> 25.2; M = 9, N = 9000
@@ -1545,7 +1545,11 @@ int launch_norm_gemv(const NormArgs& na, const void* w, const void* scale, int s
 //  * 24576, from 12 activation rows on (M = 16, N = 3072 29.4 -> 23.9).
 static bool stream_matrix(bool xf8, int64_t M, int64_t K, int64_t n) {
   if (M < 3 || M > 16 || K % 64 != 0 || K > kStreamMaxK) return false;
-  if (!lds_k(K)) return !(M <= 4 && K > 4096 && n <= (xf8 || (M == 3 && K >= 8192) ? 2048 : 1024));
+  if (!lds_k(K)) {
+    int64_t dot = 1024;  // rows that up to four activation rows leave to v_dot2
+    if (xf8 || M == 3) dot = K >= 16384 ? 4096 : (xf8 || K >= 8192 ? 2048 : 1024);
+    return M > 4 || K <= 4096 || n > dot;
+  }
   if (xf8 || M < 9) return false;
   if (K == 2048) return n > 4096 && (M >= 12 || n <= 32768);
   if (K == 14336) return n >= 8192 && (M >= 12 || n <= 24576);
