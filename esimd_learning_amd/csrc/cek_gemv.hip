@@ -1529,8 +1529,11 @@ int launch_norm_gemv(const NormArgs& na, const void* w, const void* scale, int s
 // 16, K = 8192, N = 8192 33.0 -> 14.8 -- but for up to four rows of a short and
 // long-K matrix, whose few workgroups each pay the stages' barriers (N = 1000,
 // K = 6144 5.3 against 5.9; N = 2048 6.6 -> 6.2, but at M = 3 K = 8192 7.0 against
-// 7.5, K = 16384 10.3 against 10.8, N = 4096 16.6 against 17.8; e4m3 activations N =
-// 2048, K = 8192 6.6 against 7.0, N = 4096, K = 16384 15.2 against 17.8).
+// 7.5; e4m3 activations N = 2048, K = 8192 6.6 against 7.0).  K = 16384, N = 4096
+// 16.6 against 17.8 at M = 3, 17.5 / 18.0 at M = 4, e4m3 15.2 / 17.8; N = 2048 10.7 /
+// 10.9 at M = 4 alone, and a decode step of four layers with that down projection
+// 195.5 / 201.5: v_dot2's non-temporal weight loads leave the caches to the
+// step's other matrices.
 // K that it has (16-bit activations), 9 .. 16 rows:
 //  * 3072, 4096 and 5120, matrices above 8192 rows (M = 16, K = 4096, N = 8208
 //    12.3 -> 9.6, N = 14336 15.5 -> 13.2, N = 28672 26.5 -> 25.2; M = 9, N = 9000
@@ -1546,8 +1549,8 @@ int launch_norm_gemv(const NormArgs& na, const void* w, const void* scale, int s
 static bool stream_matrix(bool xf8, int64_t M, int64_t K, int64_t n) {
   if (M < 3 || M > 16 || K % 64 != 0 || K > kStreamMaxK) return false;
   if (!lds_k(K)) {
-    int64_t dot = 1024;  // rows that up to four activation rows leave to v_dot2
-    if (xf8 || M == 3) dot = K >= 16384 ? 4096 : (xf8 || K >= 8192 ? 2048 : 1024);
+    // (weight rows that up to four activation rows leave to v_dot2)
+    const int64_t dot = K >= 16384 ? 4096 : (xf8 || (M == 3 && K >= 8192) ? 2048 : 1024);
     return M > 4 || K <= 4096 || n > dot;
   }
   if (xf8 || M < 9) return false;

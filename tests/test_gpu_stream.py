@@ -81,7 +81,7 @@ def test_stream_a8w8(ops, dev, M, K, N):
                                        ("fp16", 64, 640, 16390), ("fp16", 33, 64, 32769), ("e4m3", 20, 768, 16400),
                                        ("e4m3", 20, 832, 16400), ("e4m3", 32, 1024, 32800), ("e4m3", 40, 128, 10240),
                                        ("e4m3", 40, 192, 10241), ("e4m3", 64, 256, 10250), ("e4m3", 64, 320, 10250),
-                                       ("e4m3", 4, 16384, 4096), ("e4m3", 4, 16384, 4097), ("fp16", 3, 16384, 4097)])
+                                       ("e4m3", 4, 16384, 4096), ("e4m3", 4, 16384, 4097), ("fp16", 4, 16384, 4097)])
 def test_stream_or_tiles(ops, dev, act, M, K, N):
     """Wide matrices of short K on both sides of the line to the tiled GEMMs
     (whose fp8 MFMA sums 128 products in one step, hence the op pack's
