@@ -180,7 +180,8 @@ __device__ inline float quant_scale(float amax) { return fmaxf(amax / E4M3_MAX, 
 // correction q0 + r (v - q0 s) in two fma, which is the correctly rounded
 // quotient when r is the correctly rounded reciprocal (Markstein, "Computation
 // of elementary functions on the IBM RISC System/6000 processor", 1990) -- four
-// VALU operations where the compiler's divide takes about twelve.  The sign
+// VALU operations where the compiler's divide takes about twelve.  (Quotients
+// below 2^-90, whose correction can underflow, round to code 0 either way.)  The sign
 // of a zero quotient is v's.  s = inf (a row that holds one): s = 1, r = 0 give
 // the quotients v / inf = 0 and inf / inf = NaN.
 struct QuantDiv { float s, r; };

@@ -263,11 +263,11 @@ __global__ __launch_bounds__(256) void gemv_dot_kernel(const uint16_t* __restric
 // them leaves those in flight.  Each wave takes a quarter of a stage's K
 // units; the four partial sums meet in LDS at the end.
 //
-//  * gemv_lds_kernel: fp16/bf16 activations; a lane's 16-byte weight unit
-//    (16 K values) is decoded to two 8-value operands of
+//  * fp16/bf16 activations (XF8 = false): a lane's 16-byte weight unit (16 K
+//    values) is decoded to two 8-value operands of
 //    v_mfma_f32_16x16x32_{f16,bf16}.
-//  * gemv_lds_a8w8_kernel: e4m3 activation codes with per-row scales; two
-//    units per lane feed one v_mfma_f32_16x16x128_f8f6f4 (no decode).
+//  * e4m3 activation codes with per-row scales (XF8): two units per lane feed
+//    one v_mfma_f32_16x16x128_f8f6f4 (no decode).
 // ---------------------------------------------------------------------------
 // Wave 0's output scales of the LDS-staged kernels: sc_n[t] (raw bits) for
 // column n0 + SH t + (lane & 15) (SH = 16 or 12 rows per MFMA tile; lanes past

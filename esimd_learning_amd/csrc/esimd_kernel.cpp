@@ -86,7 +86,8 @@ at::Tensor esimd_gemv_fp8_pert(at::Tensor input, at::Tensor weight, at::Tensor w
   return output;
 }
 
-// Fused GEMVs sharing `input`: one launch per group of up to 8 matrices.
+// Fused GEMVs sharing `input`, up to 8 matrices a call: one launch for each kernel
+// that they take alone (mostly one).
 static void run_gemv_fused(const at::Tensor& input, const std::vector<at::Tensor>& weights,
                            const std::vector<at::Tensor>& scales, const std::vector<at::Tensor>& outputs,
                            bool per_tensor, const char* op) {

@@ -14,7 +14,10 @@
 The gate/up projection and gelu_and_mul run as one launch (Wgu = [Wg; Wu],
 the GEMV's epilogue applies gelu_tanh(gate) * up to the rounded outputs);
 ``fuse_glu=False`` runs them as esimd_gemv_fp8_pern into [M, 2d] followed by
-esimd_gelu_and_mul, which gives the same values.  With ``fuse_norm`` (up to
+esimd_gelu_and_mul, which gives the same values -- but for 9 to 16 rows with
+16-bit hand-offs and 2d > 8192 (up to 32768; any above 8192 at hidden 4096 from
+12 rows on), where the plain GEMV runs the weight-streaming kernel, whose sums
+are in another order: the same within the op's rounding.  With ``fuse_norm`` (up to
 four rows) each add+RMSNorm runs in the prologue of the GEMV it feeds; r1 is
 then kept in a buffer of the layer, hidden is only read, and residual
 receives r2 as before.  It is off by default: every workgroup of the GEMV

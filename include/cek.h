@@ -80,7 +80,9 @@ int cek_gemv_fp8_pern_ws(const void* x, const void* w, const void* scale, void* 
 
 /*
  * Several fp8-weight GEMVs that share one activation matrix, in one launch
- * (e.g. Q, K and V, or gate and up projections).  Host arrays of `count`
+ * per kernel that the matrices take alone (mostly one: wide and narrow ones may
+ * take different kernels from three rows on); e.g. Q, K and V, or gate and up
+ * projections.  Host arrays of `count`
  * (1..8) device pointers / row counts: w[i] [N[i], K], scale[i] (per-channel
  * of scale_dtype for _pern, fp32 device scalar for _pert), y[i] [M, N[i]].
  * Each y[i] equals what cek_gemv_fp8_pern/pert computes for matrix i.

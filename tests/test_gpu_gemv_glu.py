@@ -16,7 +16,8 @@ Two references:
   bf16 activations at M <= 4 (where each 16-row tile reads its K chunks in a
   rotated order), for d not a multiple of 16: the fused kernel's up tiles
   then straddle two of the unfused GEMV's tiles, whose K sums run in
-  different orders.
+  different orders -- and, at 9 to 16 rows, for 2d above 8192, where the
+  unfused GEMV runs the weight-streaming kernel (to the op pack's tolerance).
 
 The shapes reach every fused configuration (M <= 4, <= 8, <= 16; K = 3, 4
 and 5 KiB values), d a multiple of 16 and not, M > 16 (the w8a16 GEMM, then
@@ -155,3 +156,20 @@ def test_glu_a8w8_bf16_out(ops, dev):
     torch.cuda.synchronize()
     ref = _ref_glu(ogemm.gemm_a8w8(q, qs, W8.view(torch.uint8), s.float()), torch.bfloat16)
     assert_close_fp(out.cpu(), ref, "glu a8w8 bf16")
+
+
+@pytest.mark.parametrize("M,K,d,same", [(16, 4096, 4096, True), (16, 4096, 4104, False), (9, 5120, 4104, False),
+                                        (12, 4096, 16400, False), (16, 3072, 16400, True)])
+def test_glu_wide_against_unfused(ops, dev, M, K, d, same):
+    """9 to 16 rows on both sides of the 2d at which the unfused GEMV streams
+    (above 8192; at K = 3072 up to 32768): equal bits, else within tolerance."""
+    _say(f"glu wide M={M} K={K} d={d}")
+    W8, s = synthetic.weight_fp8(2 * d, K, seed=d)
+    x, W8, s = synthetic.activations(M, K, seed=M).to(dev), W8.to(dev), s.to(dev)
+    y = torch.full((M, d), float("nan"), dtype=torch.float16, device=dev)
+    ops.esimd_gemv_fp8_gelu_and_mul(x, W8, s, y)
+    two = _unfused(ops, x, W8, s, torch.float16, dev)
+    if same:
+        assert torch.equal(y, two)
+    else:
+        assert_close_fp(y.cpu(), two.cpu(), f"glu wide M={M} K={K} d={d}")

@@ -1,13 +1,12 @@
-"""The wide batched GEMV: 9 <= M <= 16, K of 2, 3 or 4 KiB values and
-512 < N / 16 <= 2048 row tiles per weight matrix run gemv_xres_kernel
-(activations resident in LDS, weights streamed into MFMA operands, each
-tile's K in two halves).  Checked against the CPU oracle (tolerance as in
-the other GEMV tests) over 3 to 8 tiles per workgroup slot, ragged N, both
-fp8 formats, both activation types and every scale kind; and, since its sum
-order differs from the other GEMV kernels', the multi-matrix op must still
-give each matrix, bit for bit, what the single op gives it -- with matrices
-on either side of the kernel choice in one call, and with more slots than
-workgroups (grid-stride slots).
+"""The wide batched GEMV: 9 <= M <= 16, K of 2, 3 or 4 KiB values and more
+than 8192 rows per weight matrix run the weight-streaming kernel, where
+narrower ones run the staged one.  Checked against the CPU oracle (tolerance
+as in the other GEMV tests) over several counts of weight rows per workgroup,
+ragged N, both fp8 formats, both activation types and every scale kind; and,
+since its sum order differs from the staged kernel's, the multi-matrix op must
+still give each matrix, bit for bit, what the single op gives it -- with
+matrices on either side of the kernel choice in one call.  Then the a8w8 GEMV
+of 17 to 32 rows.
 """
 
 import sys
@@ -35,8 +34,7 @@ def _pern(ops, xd, Wd, sd, io):
     return y
 
 
-# (K, N): tiles per slot ceil(tiles / 256): 563 tiles (3 per slot, ragged N),
-# 768 (3), 896 (4), 1025 (5, ragged), 1536 (6), 1792 (7), 2048 (8)
+# (K, N): up to 128 rows per CU, in one to four workgroups, ragged N
 SHAPES = [(4096, 9000), (3072, 12288), (4096, 14336), (4096, 16400), (4096, 24576), (2048, 28672), (2048, 32768)]
 
 
@@ -81,8 +79,8 @@ def test_xres_per_tensor_scale(ops, dev):
     assert_close_fp(y.cpu(), ogemv.gemv_fp8_pert(x, W8, s), "xres pert")
 
 
-@pytest.mark.parametrize("Ns,K", [((14336, 4096, 1024, 9000), 4096),  # xres and LDS-kernel matrices in one call
-                                  ((32768, 32768), 2048),              # 4096 tiles: two slots per workgroup
+@pytest.mark.parametrize("Ns,K", [((14336, 4096, 1024, 9000), 4096),  # streamed and staged matrices in one call
+                                  ((32768, 32768), 2048),              # several workgroups per CU
                                   ((12288, 6144), 3072)])
 @pytest.mark.parametrize("M", [9, 16])
 def test_xres_multi_matrix_equals_single(ops, dev, M, Ns, K):
@@ -101,15 +99,9 @@ def test_xres_multi_matrix_equals_single(ops, dev, M, Ns, K):
         assert_close_fp(ys[i].cpu(), ogemv.gemv_fp8_pern(x, Ws[i], Ss[i]), f"matrix {i}")
 
 
-# The e4m3-activation form (gemv_xres8_kernel): the a8w8 GEMM op sends M <= 64
-# (without a split-K workspace) to the GEMV kernels; 17 <= M <= 32 with at
-# least 384 row tiles and K of 2, 3 or 4 KiB values takes this one (up to 512
-# tiles from 24 rows on).  N = 28672 gives 896 slots of 2 tiles: 3-4 slots per
-# workgroup.  K = 5120 (the 32 activation rows fill all of LDS; the K parts'
-# sums reuse it) up to 512 tiles; N = 14336 at K = 5120 and M = 17 at up to
-# 512 tiles stay on the other kernel.  N ~ 6144 runs 12-row tiles (256 slots),
-# N = 6140 and 6130 with a ragged last one; 12-row tiles also take N from 384
-# of them (4608) up, from 24 rows (N = 4608, 5000, 5120).
+# The a8w8 GEMM op sends 17 <= M <= 32 to the weight-streaming kernel, above
+# 16384 rows of K = 2, 3 or 4 KiB to gemv_xres8_kernel (activations resident in
+# LDS, slots of two 16-row tiles, 3-4 of them per workgroup at N = 28672).
 @pytest.mark.parametrize("M", [17, 24, 32])
 @pytest.mark.parametrize("K,N", [(4096, 6144), (4096, 6140), (3072, 12288), (2048, 8200), (4096, 28672), (5120, 6144),
                                  (5120, 6130), (5120, 8190), (5120, 14336), (4096, 4608), (4096, 5000), (5120, 5120)])
